@@ -409,16 +409,16 @@ int finish_reduction(gfc_ctx *c, unsigned blocks, double out[3]) {
     return GFC_OK;
 }
 
-// e2, theta, F of the factored state; fp32 selects the FP32 G (MIXED phase 1),
-// evaluated against the FP64 u0.
+// e2, theta, F of the factored state; fp32 selects the FP32 G (MIXED phase 1)
+// and the FP64 u0 in the configuration's own frame.
 int obs_factored(gfc_job *j, bool fp32, double out[3]) {
     gfc_ctx *c = j->ctx;
     const unsigned b = nblocks(2 * (int64_t)j->Vh);
     if (fp32)
-        hipLaunchKernelGGL((gfc::k_obs_factored<double, float>), dim3(b), dim3(kBlock), 0,
+        hipLaunchKernelGGL((gfc::k_obs_factored<float>), dim3(b), dim3(kBlock), 0,
                            c->stream, j->u0, j->gf, j->geom.ns, j->Vh, c->part);
     else
-        hipLaunchKernelGGL((gfc::k_obs_factored<double, double>), dim3(b), dim3(kBlock), 0,
+        hipLaunchKernelGGL((gfc::k_obs_factored<double>), dim3(b), dim3(kBlock), 0,
                            c->stream, j->u0, j->g, j->geom.ns, j->Vh, c->part);
     LAUNCH_CHECK();
     double s[3];
@@ -447,38 +447,49 @@ int obs_aos(gfc_job *j, double out[3]) {
     return GFC_OK;
 }
 
-int build_u0(gfc_job *j) { return build_u0(j, j->ctx->stream); }
-
-int build_u0(gfc_job *j, hipStream_t s) {
-    const unsigned b = nblocks(2 * (int64_t)j->Vh);
-    hipLaunchKernelGGL(gfc::k_build_u0<double>, dim3(b), dim3(kBlock), 0, s, j->cfg, j->u0,
-                       j->geom.ns, j->Vh);
+// u0 and G = 1 in the axial frame of cfg.
+int begin_frame(gfc_job *j, hipStream_t s) {
+    const int ns = j->geom.ns, ncol = ns * ns * j->geom.nt;
+    hipLaunchKernelGGL(gfc::k_frame_begin, dim3((ncol + 63) / 64), dim3(64), 0, s, j->cfg, j->u0,
+                       j->g, ns, j->Vh, ncol);
     LAUNCH_CHECK();
-    if (j->u0f) {
-        hipLaunchKernelGGL(gfc::k_build_u0<float>, dim3(b), dim3(kBlock), 0, s, j->cfg, j->u0f,
-                           j->geom.ns, j->Vh);
-        LAUNCH_CHECK();
-    }
+    hipLaunchKernelGGL(gfc::k_axial_u0, dim3(nblocks(2 * (int64_t)j->Vh)), dim3(kBlock), 0, s,
+                       j->cfg, j->g, j->u0, ns, j->Vh);
+    LAUNCH_CHECK();
     return GFC_OK;
 }
 
-// u0 from cfg and G <- 1 at the start of a fix; the FP32 copies only for a
-// mixed-precision fix.
-int prepare_fix(gfc_job *j, bool mixed) {
-    hipStream_t s = j->ctx->stream;
+// State at the start of a fix: G = 1 and u0, for FP64 sweeps in the axial
+// frame, for the FP32 phase of a mixed fix in the configuration's own.
+int begin_fix(gfc_job *j, hipStream_t s, bool mixed) {
+    if (!mixed) return begin_frame(j, s);
     const unsigned b = nblocks(2 * (int64_t)j->Vh);
-    hipLaunchKernelGGL(gfc::k_build_u0<double>, dim3(b), dim3(kBlock), 0, s, j->cfg, j->u0,
+    hipLaunchKernelGGL(gfc::k_build_u0, dim3(b), dim3(kBlock), 0, s, j->cfg, j->u0, j->u0f,
                        j->geom.ns, j->Vh);
     LAUNCH_CHECK();
-    hipLaunchKernelGGL(gfc::k_g_identity<double>, dim3(b), dim3(kBlock), 0, s, j->g, j->Vh);
+    hipLaunchKernelGGL(gfc::k_g_identity<float>, dim3(b), dim3(kBlock), 0, s, j->gf, j->Vh);
     LAUNCH_CHECK();
-    if (mixed) {
-        hipLaunchKernelGGL(gfc::k_build_u0<float>, dim3(b), dim3(kBlock), 0, s, j->cfg, j->u0f,
-                           j->geom.ns, j->Vh);
-        LAUNCH_CHECK();
-        hipLaunchKernelGGL(gfc::k_g_identity<float>, dim3(b), dim3(kBlock), 0, s, j->gf, j->Vh);
-        LAUNCH_CHECK();
-    }
+    return GFC_OK;
+}
+
+// FP32 -> FP64 hand-off: u0 and G go into the axial frame.
+int promote_g(gfc_job *j, hipStream_t s) {
+    RC_TRY(begin_frame(j, s));
+    hipLaunchKernelGGL(gfc::k_g_promote, dim3(nblocks(2 * (int64_t)j->Vh)), dim3(kBlock), 0, s,
+                       j->gf, j->g, j->Vh);
+    LAUNCH_CHECK();
+    return GFC_OK;
+}
+
+// G out of the axial frame at the end of a fix of `sweeps` half-sweeps, with
+// its last reunitarization if `project`.  Without a sweep G is the identity
+// (also for a configuration whose residue is no number).
+int end_frame(gfc_job *j, hipStream_t s, int sweeps, bool project) {
+    if (sweeps == 0) return set_identity(j, s);
+    const int ns = j->geom.ns, ncol = ns * ns * j->geom.nt;
+    hipLaunchKernelGGL(gfc::k_frame_end, dim3((ncol + 63) / 64), dim3(64), 0, s, j->cfg, j->g, ns,
+                       j->Vh, ncol, project);
+    LAUNCH_CHECK();
     return GFC_OK;
 }
 
@@ -704,20 +715,11 @@ int sweep_blocked(gfc_job *j, const StreamSet &ss, bool fp32, int from, int to, 
     return rc;
 }
 
-int promote_g_only(gfc_job *j, hipStream_t s) {
-    const unsigned b = nblocks(2 * (int64_t)j->Vh);
-    hipLaunchKernelGGL(gfc::k_g_promote, dim3(b), dim3(kBlock), 0, s, j->gf, j->g, j->Vh);
-    LAUNCH_CHECK();
-    return GFC_OK;
-}
-
 int promote_g(gfc_job *j, SweepState &st) {
-    RC_TRY(promote_g_only(j, j->ctx->stream));
+    RC_TRY(promote_g(j, j->ctx->stream));
     st.fp32 = false;
     return GFC_OK;
 }
-
-int promote_g_only(gfc_job *j) { return promote_g_only(j, j->ctx->stream); }
 
 struct SweepTimer {
     bool on = false;
@@ -843,10 +845,10 @@ struct SliceTracker {
         gfc_ctx *c = j->ctx;
         const unsigned b = nblocks(2 * (int64_t)j->Vh);
         if (fp32)
-            hipLaunchKernelGGL((gfc::k_obs_factored<double, float>), dim3(b), dim3(kBlock), 0,
+            hipLaunchKernelGGL((gfc::k_obs_factored<float>), dim3(b), dim3(kBlock), 0,
                                c->stream, j->u0, j->gf, j->geom.ns, j->Vh, c->part);
         else
-            hipLaunchKernelGGL((gfc::k_obs_factored<double, double>), dim3(b), dim3(kBlock), 0,
+            hipLaunchKernelGGL((gfc::k_obs_factored<double>), dim3(b), dim3(kBlock), 0,
                                c->stream, j->u0, j->g, j->geom.ns, j->Vh, c->part);
         LAUNCH_CHECK();
         part.resize((size_t)b * 3);
@@ -890,7 +892,6 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
     gfc_report r;
     std::memset(&r, 0, sizeof r);
 
-    RC_TRY(prepare_fix(j, o.precision == GFC_PREC_MIXED));
     const double omega = (double)p->omega_OR;  // float in the reference
     const int hits = (int)p->hits;
     const int which = p->gfix_proxy == GFC_PROXY_THETA ? 1 : 0;
@@ -903,12 +904,15 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
     timer.s = j->ctx->stream;
     SliceTracker sl;
     if (o.retire_slices) {
-        if (j->geom.ns % 8)
+        if (j->geom.ns % 8) {
+            RC_TRY(set_identity(j));
             return fail(GFC_EINVAL, "gfc_job_fix: retire_slices needs ns a multiple of 8");
+        }
         RC_TRY(sl.init(j));
     }
 
-    RC_TRY(obs_factored(j, false, ob));
+    RC_TRY(begin_fix(j, j->ctx->stream, st.fp32));
+    RC_TRY(obs_factored(j, st.fp32, ob));
     r.residue_evals++;
     double res = ob[which];
     r.residue_initial = res;
@@ -1003,10 +1007,10 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
     }
     // left the loop in the FP32 phase (tolerance reached there or max sweeps):
     // hand the state over so that G and U are FP64
-    if (st.fp32) RC_TRY(promote_g(j, st));
+    if (st.fp32 && sweep > 0) RC_TRY(promote_g(j, st));
     // converged: the final reunitarization of G and U (src/gauge_fixing.c:822-823);
     // the max-sweeps and stall exits return before it
-    if (!done) RC_TRY(reunit_g(j, false, 0, 2));
+    RC_TRY(end_frame(j, j->ctx->stream, sweep, !done));
     RC_TRY(materialize(j, !done));
     HIP_TRY(hipStreamSynchronize(j->ctx->stream));
     r.seconds_sweeps = timer.seconds();

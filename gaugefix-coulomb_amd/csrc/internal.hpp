@@ -85,14 +85,13 @@ namespace gfcx {
 // stream, or on j->ctx->stream without one.
 int set_identity(gfc_job *j);
 int set_identity(gfc_job *j, hipStream_t s);
-int build_u0(gfc_job *j);
-int build_u0(gfc_job *j, hipStream_t s);
+int begin_fix(gfc_job *j, hipStream_t s, bool mixed);
+int end_frame(gfc_job *j, hipStream_t s, int sweeps, bool project);
 int materialize(gfc_job *j, bool project);
 int materialize(gfc_job *j, hipStream_t s, bool project);
 int reunit_g(gfc_job *j, bool fp32, int p0, int np);
 int reunit_g(gfc_job *j, hipStream_t s, bool fp32, int p0, int np);
-int promote_g_only(gfc_job *j);
-int promote_g_only(gfc_job *j, hipStream_t s);
+int promote_g(gfc_job *j, hipStream_t s);
 int generate_smooth_device(gfc_job *j, uint64_t seed, double eps);
 int generate_smooth_device(gfc_job *j, hipStream_t s, uint64_t seed, double eps);
 int ensure_partials(gfc_ctx *c, size_t blocks);

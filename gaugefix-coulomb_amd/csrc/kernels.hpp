@@ -5,8 +5,8 @@
 //   u0  : SoA spatial links of the configuration being fixed
 //   g   : SoA gauge transformation
 // u0 and g hold SU(3) matrices as their first two rows (6 complex numbers; an
-// FP64 u0 link as five, see Stored below); row 2 = conj(r0 x r1) is rebuilt in
-// registers on every load.  One tiled field
+// FP64 u0 link as five, see u0 fields below); row 2 = conj(r0 x r1) is rebuilt
+// in registers on every load.  One tiled field
 // (see field_size below) per parity p and, for u0, direction i = Z,Y,X:
 //   u0 field p*3 + i,   g field p.
 // Within a parity the index is h = lex >> 1 with lex = ((t ns + z) ns + y) ns + x
@@ -19,6 +19,25 @@
 // active parity while u0 stays read-only.  w(n) = sum_i U_i(n) + U_i(n-i)^dagger
 // (src/gauge_fixing.c:493-531) becomes w(n) = G(n) W(n) with
 // W(n) = sum_i [u0_i(n) G(n+i)^dagger + u0_i(n-i)^dagger G(n-i)^dagger].
+//
+// The axial frame.  The links G(n) u_i(n) G(n+i)^dagger are, with any field
+// h(n) of SU(3) matrices, also G'(n) u0_i(n) G'(n+i)^dagger with
+// u0_i(n) = h(n) u_i(n) h(n+i)^dagger and G' = G h^dagger, and since an update
+// multiplies G from the left it acts on G' in the same way.  FP64 sweeps take
+// for h the ordered product of the Z links in the site's column below it,
+// h(z+1) = h(z) u_Z(z): then u0_Z = 1 except on the plane z = ns - 1, where it
+// is the product of the whole column.  A sweep reads four links per site
+// instead of six (320 instead of 480 B of u0 per update) and forms four
+// products instead of six; only the sites of the two planes next to the wrap
+// read a Z link.  G = G' h is formed at the end of a fix (k_frame_end).  The
+// sweeps are bound by the rate of their bytes and next by instructions: 768 ->
+// 608 B and 2414 -> about 2080 VALU instructions per update took the 48^3 x 96
+// FP64 fix from 0.652 to 0.547 s, of which entering and leaving the frame are
+// 3.6 ms; 32^3 x 64 from 131 to 110 ms, 8^3 x 16 from 9.4 to 7.9 ms.
+// The FP32 phase of a mixed fix keeps the configuration's own frame: the
+// rounding of its sweeps is carried to the result in the directions that do
+// not change the gauge condition, up to 1e-3 on the odd timeslice, and another
+// frame would give another one.
 #pragma once
 
 #include "su3.hpp"
@@ -127,6 +146,18 @@ __device__ __forceinline__ const cplx<T> *u0_field(const cplx<T> *u0, int Vh, in
 template <typename T>
 __device__ __forceinline__ cplx<T> *u0_field(cplx<T> *u0, int Vh, int p, int i) {
     return u0 + (p * 3 + i) * u0_field_size<T>(Vh);
+}
+// In the axial frame: field of the links u0_i on parity p, i = 1 (Y), 2 (X);
+// and of the Z links of the plane z = ns - 1 on parity p, by their index in
+// the plane, t ns^2/2 + y ns/2 + x/2 (Vh / ns sites).  Together at most 30 of
+// the allocation's 36 planes of Vh numbers.
+template <typename C>
+__device__ __forceinline__ C *axial_field(C *u0, int Vh, int p, int i) {
+    return u0 + (p * 2 + i - 1) * u0_field_size<double>(Vh);
+}
+template <typename C>
+__device__ __forceinline__ C *axial_wrap(C *u0, int Vh, int ns, int p) {
+    return u0 + 4 * u0_field_size<double>(Vh) + p * u0_field_size<double>(Vh / ns);
 }
 template <typename T>
 __device__ __forceinline__ const cplx<T> *g_field(const cplx<T> *g, int Vh, int p) {
@@ -304,9 +335,36 @@ __device__ __forceinline__ Nbr neighbours(const Site &s, int h, int ns) {
     return n;
 }
 
+// W += u0_Z(n) G(n+z)^dagger + u0_Z(n-z)^dagger G(n-z)^dagger in the axial
+// frame, gf = G(n+z) and gb = G(n-z) with all three rows.  u0_Z is 1 but on the plane z = ns - 1,
+// which only the sites of that plane and of z = 0 meet: one plane is ns^2 / 2
+// consecutive parity indices, so most waves skip both branches.
+template <bool STREAM>
+__device__ __forceinline__ void axial_z(mat3<double> &W, const cplx<double> *__restrict__ u0,
+                                        const Site &s, int ns, int Vh, int p,
+                                        const mat3<double> &gf, const mat3<double> &gb) {
+    const int hw = s.t * (ns * (ns >> 1)) + s.y * (ns >> 1) + s.xh;
+    if (s.z + 1 == ns) {
+        mat3<double> u;
+        load_u0_rows01<STREAM>(u, axial_wrap(u0, Vh, ns, p), hw);
+        m_mac_nd_su3(W, u, gf);
+    } else {
+        m_add_dagger(W, gf);
+    }
+    if (s.z == 0) {
+        mat3<double> u;
+        load_u0_rows01<STREAM>(u, axial_wrap(u0, Vh, ns, 1 - p), hw);
+        m_fill_row2(u);
+        m_mac_dagger_su3(W, gb, u);
+    } else {
+        m_add_dagger(W, gb);
+    }
+}
+
 // ---------------------------------------------------------------------------
-// The site update of parity index h on parity p: reads 6 u0 links, 6
-// neighbour G and G(n); writes G(n).  Shared by the single-lattice and the
+// The site update of parity index h on parity p: reads the u0 links (FP64: 4
+// in the axial frame, and a Z link next to the wrap; FP32: 6), 6 neighbour G
+// and G(n); writes G(n).  Shared by the single-lattice and the
 // batched (serving) kernels, so a site computes the same bits in both.
 // POUT projects the new G(n) onto SU(3) (in FP64, project_g) before storing
 // it: the same bits as a reunitarization of this parity's G right after the
@@ -334,20 +392,34 @@ __device__ __forceinline__ void sweep_site(const cplx<T> *__restrict__ u0,
         project_g(gn);
         __builtin_amdgcn_sched_barrier(0);
     }
-    // the six products are SU(3): rows 0, 1 from the stored rows of the left
-    // factor, row 2 by closure (m_mac_nd_su3, m_mac_dagger_su3).  The four
-    // matrices of a direction are loaded together, one memory round trip per
-    // direction rather than the compiler's two (48^3 x 96: FP64 fix 1%, mixed
-    // 2% faster).
+    // the products are SU(3): rows 0, 1 from the stored rows of the left
+    // factor, row 2 by closure (m_mac_nd_su3, m_mac_dagger_su3).  The matrices
+    // of a direction are loaded together, one memory round trip per direction
+    // rather than the compiler's two (48^3 x 96: FP64 fix 1%, mixed 2% faster).
     mat3<T> W;
     m_zero(W);
+    constexpr bool axial = sizeof(T) == sizeof(double);
+    if constexpr (axial) {
+        cplx<T> rgf[kPlanes], rgb[kPlanes];
+        load_raw<false>(rgf, gq, tile_bytes<T>(nb.fwd[0]));
+        load_raw<false>(rgb, gq, tile_bytes<T>(nb.bwd[0]));
+        __builtin_amdgcn_sched_barrier(0);
+        mat3<T> gf, gb;
+        rows01(gf, rgf);
+        m_fill_row2(gf);
+        rows01(gb, rgb);
+        m_fill_row2(gb);
+        axial_z<STREAM>(W, u0, s, ns, Vh, p, gf, gb);
+    }
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
+    for (int i = axial ? 1 : 0; i < 3; i++) {
         constexpr int NU = U0Planes<T>::n;
         cplx<T> ruf[NU], rub[NU], rgf[kPlanes], rgb[kPlanes];
-        load_raw<STREAM>(ruf, u0_field(u0, Vh, p, i), u0_tile_bytes<T>(h));
+        const cplx<T> *fu = axial ? axial_field(u0, Vh, p, i) : u0_field(u0, Vh, p, i);
+        const cplx<T> *bu = axial ? axial_field(u0, Vh, 1 - p, i) : u0_field(u0, Vh, 1 - p, i);
+        load_raw<STREAM>(ruf, fu, u0_tile_bytes<T>(h));
         load_raw<false>(rgf, gq, tile_bytes<T>(nb.fwd[i]));
-        load_raw<STREAM>(rub, u0_field(u0, Vh, 1 - p, i), u0_tile_bytes<T>(nb.bwd[i]));
+        load_raw<STREAM>(rub, bu, u0_tile_bytes<T>(nb.bwd[i]));
         load_raw<false>(rgb, gq, tile_bytes<T>(nb.bwd[i]));
         __builtin_amdgcn_sched_barrier(0);
         mat3<T> uf, gf, ub, gb;
@@ -440,59 +512,185 @@ __global__ __launch_bounds__(kBlock) void k_g_reunit(cplx<T> *__restrict__ g, in
     reunit_site<T>(g, Vh, p0 + idx / count, h0 + idx % count);
 }
 
-// FP32 -> FP64 hand-off of G: promote rows 0, 1 then project in FP64.
-__device__ __forceinline__ void promote_site(const cplx<float> *__restrict__ gf,
-                                             cplx<double> *__restrict__ g, int Vh, int p,
-                                             int h) {
+// FP32 -> FP64 hand-off of G: rows 0, 1 of the FP32 G promoted and projected
+// in FP64, then taken into the axial frame, where g holds h^dagger
+// (k_frame_begin).
+__global__ __launch_bounds__(kBlock) void k_g_promote(const cplx<float> *__restrict__ gf,
+                                                      cplx<double> *__restrict__ g, int Vh) {
+    const int idx = blockIdx.x * kBlock + threadIdx.x;
+    if (idx >= 2 * Vh) return;
+    const int p = idx >= Vh, h = idx - p * Vh;
     const cplx<float> *src = g_field(gf, Vh, p);
     const uint32_t off = tile_bytes<float>(h);
-    mat3<double> m;
+    mat3<double> m, hd, out;
 #pragma unroll
     for (int k = 0; k < kPlanes; k++) {
         cplx<float> v = *elem_ptr(src, off, k);
         m.e[k] = c_make<double>(v.re, v.im);
     }
     m_project_su3(m);
-    store_su3<false>(m, g_field(g, Vh, p), h);
+    load_su3<false>(hd, g_field(static_cast<const cplx<double> *>(g), Vh, p), h);
+    m_mul(m, hd, out);
+    store_su3<false>(out, g_field(g, Vh, p), h);
 }
 
-__global__ __launch_bounds__(kBlock) void k_g_promote(const cplx<float> *__restrict__ gf,
-                                                      cplx<double> *__restrict__ g, int Vh) {
+// Stores a u0 matrix of type T from its rows 0 and 1 in FP64.
+template <typename T>
+__device__ __forceinline__ void store_u0(const mat3<double> &m, cplx<T> *__restrict__ field,
+                                         int h) {
+    cplx<double> e[kPlanes];
+#pragma unroll
+    for (int k = 0; k < kPlanes; k++) e[k] = m.e[k];
+    if constexpr (U0Planes<T>::n == 5) {
+        // row 1 without the element under row 0's pivot (u0_unpack)
+        const int piv = u0_pivot(e);
+        const cplx<double> s0 = csel(piv == 0, e[4], e[3]);
+        const cplx<double> s1 = csel(piv == 2, e[4], e[5]);
+        e[3] = s0;
+        e[4] = s1;
+    }
+    const uint32_t off = u0_tile_bytes<T>(h);
+#pragma unroll
+    for (int k = 0; k < U0Planes<T>::n; k++)
+        *elem_ptr(field, off, k) = c_make<T>((T)e[k].re, (T)e[k].im);
+}
+
+// The axial frame of a column (t, y, x): one thread walks its sites z = 0 ..
+// ns - 1 with d(z) = h(z)^dagger, d(0) = 1 and d(z+1) = u_Z(z)^dagger d(z), one
+// rounding per step, and calls visit(z, d); returns the adjoint of the Z link
+// of the plane z = ns - 1 in the frame.  The next site's link is loaded while
+// this one's product is formed.
+template <typename Visit>
+__device__ __forceinline__ mat3<double> walk_column(const cplx<double> *__restrict__ cfg, int ns,
+                                                    int64_t lex0, Visit visit) {
+    const int64_t stride = (int64_t)ns * ns * 36;  // numbers from one z to the next
+    const cplx<double> *src = cfg + lex0 * 36 + 9;
+    mat3<double> d, u, next, zero;
+    m_zero(zero);
+    m_identity(d);
+#pragma unroll
+    for (int k = 0; k < 9; k++) next.e[k] = src[k];
+    for (int z = 0; z < ns; z++) {
+        u = next;
+        if (z + 1 < ns) {
+            src += stride;
+#pragma unroll
+            for (int k = 0; k < 9; k++) next.e[k] = src[k];
+        }
+        visit(z, d);
+        mat3<double> hi, lo;
+        m_mul2<2>(m_dagger(u), zero, d, hi, lo);
+        m_polish_su3(hi, lo, d);
+    }
+    return d;
+}
+
+// Column index of a thread -> its y, x, t and the site index of its z = 0.
+struct Column {
+    int x, y, t;
+    int64_t lex0;
+};
+
+__device__ __forceinline__ Column column_of(int c, int ns) {
+    Column q;
+    q.x = c % ns;
+    const int r = c / ns;
+    q.y = r % ns;
+    q.t = r / ns;
+    q.lex0 = ((int64_t)q.t * ns * ns + q.y) * ns + q.x;
+    return q;
+}
+
+// G = 1 in the axial frame: G' = h^dagger, and the Z links of the plane
+// z = ns - 1.  One thread per column, ncol = ns^2 nt columns.
+__global__ __launch_bounds__(64) void k_frame_begin(const cplx<double> *__restrict__ cfg,
+                                                    cplx<double> *__restrict__ u0,
+                                                    cplx<double> *__restrict__ g, int ns, int Vh,
+                                                    int ncol) {
+    const int c = blockIdx.x * 64 + threadIdx.x;
+    if (c >= ncol) return;
+    const Column q = column_of(c, ns);
+    const mat3<double> w = walk_column(cfg, ns, q.lex0, [&](int z, const mat3<double> &d) {
+        const int p = (q.x + q.y + z + q.t) & 1;
+        store_su3<false>(d, g_field(g, Vh, p), (int)((q.lex0 + (int64_t)z * ns * ns) >> 1));
+    });
+    const int p = (q.x + q.y + ns - 1 + q.t) & 1;
+    const int hw = (q.t * ns + q.y) * (ns >> 1) + (q.x >> 1);
+    store_u0(m_dagger(w), axial_wrap(u0, Vh, ns, p), hw);
+}
+
+// End of a fix: G = G' h, projected onto SU(3) if `project` (the last
+// reunitarization of G).
+__global__ __launch_bounds__(64) void k_frame_end(const cplx<double> *__restrict__ cfg,
+                                                  cplx<double> *__restrict__ g, int ns, int Vh,
+                                                  int ncol, bool project) {
+    const int c = blockIdx.x * 64 + threadIdx.x;
+    if (c >= ncol) return;
+    const Column q = column_of(c, ns);
+    walk_column(cfg, ns, q.lex0, [&](int z, const mat3<double> &d) {
+        cplx<double> *field = g_field(g, Vh, (q.x + q.y + z + q.t) & 1);
+        const int h = (int)((q.lex0 + (int64_t)z * ns * ns) >> 1);
+        mat3<double> gp, zero, out, lo;
+        m_zero(zero);
+        load_su3<false>(gp, static_cast<const cplx<double> *>(field), h);
+        m_mul2<2>(gp, zero, m_dagger(d), out, lo);
+#pragma unroll
+        for (int k = 0; k < kPlanes; k++)
+            out.e[k] = c_make<double>(out.e[k].re + lo.e[k].re, out.e[k].im + lo.e[k].im);
+        if (project) m_project_su3(out);
+        store_su3<false>(out, field, h);
+    });
+}
+
+// The Y and X links of cfg (AoS FP64) in the axial frame, u0_i(n) =
+// h(n) u_i(n) h(n+i)^dagger with h = G'^dagger (k_frame_begin).  One thread per
+// site.
+__global__ __launch_bounds__(kBlock) void k_axial_u0(const cplx<double> *__restrict__ cfg,
+                                                     const cplx<double> *__restrict__ g,
+                                                     cplx<double> *__restrict__ u0, int ns,
+                                                     int Vh) {
     const int idx = blockIdx.x * kBlock + threadIdx.x;
     if (idx >= 2 * Vh) return;
-    const int p = idx >= Vh;
-    promote_site(gf, g, Vh, p, idx - p * Vh);
+    const int p = idx >= Vh, h = idx - p * Vh;
+    const Site s = site_of(h, p, ns);
+    const Nbr nb = neighbours(s, h, ns);
+    const int64_t lex = (int64_t)2 * s.row + s.x;
+    mat3<double> gn;
+    load_su3<false>(gn, g_field(g, Vh, p), h);
+#pragma unroll
+    for (int i = 1; i < 3; i++) {
+        const cplx<double> *src = cfg + (lex * 4 + 1 + i) * 9;
+        mat3<double> u, gm, zero, a, alo, out, lo;
+        m_zero(zero);
+#pragma unroll
+        for (int k = 0; k < 9; k++) u.e[k] = src[k];
+        load_su3<false>(gm, g_field(g, Vh, 1 - p), nb.fwd[i]);
+        m_mul2<2>(m_dagger(gn), zero, u, a, alo);
+        m_mul2<2>(a, alo, gm, out, lo);
+        m_polish_su3(out, lo, out);
+        store_u0(out, axial_field(u0, Vh, p, i), h);
+    }
 }
 
-// cfg (AoS FP64) spatial links -> u0 planes of type T (rows 0 and 1).
-template <typename T>
+// cfg (AoS FP64) spatial links -> u0 fields in FP64 and FP32 in the
+// configuration's own frame, for the FP32 phase of a mixed fix.
 __global__ __launch_bounds__(kBlock) void k_build_u0(const cplx<double> *__restrict__ cfg,
-                                                     cplx<T> *__restrict__ u0, int ns,
+                                                     cplx<double> *__restrict__ u0,
+                                                     cplx<float> *__restrict__ u0f, int ns,
                                                      int Vh) {
     const int idx = blockIdx.x * kBlock + threadIdx.x;
     if (idx >= 2 * Vh) return;
     const int p = idx >= Vh, h = idx - p * Vh;
     const Site s = site_of(h, p, ns);
     const int64_t lex = (int64_t)2 * s.row + s.x;
-    const uint32_t off = u0_tile_bytes<T>(h);
 #pragma unroll
     for (int i = 0; i < 3; i++) {
         const cplx<double> *src = cfg + (lex * 4 + 1 + i) * 9;
-        cplx<T> *dst = u0_field(u0, Vh, p, i);
-        cplx<double> e[kPlanes];
+        mat3<double> m;
 #pragma unroll
-        for (int k = 0; k < kPlanes; k++) e[k] = src[k];
-        if constexpr (U0Planes<T>::n == 5) {
-            // row 1 without the element under row 0's pivot (u0_unpack)
-            const int piv = u0_pivot(e);
-            const cplx<double> s0 = csel(piv == 0, e[4], e[3]);
-            const cplx<double> s1 = csel(piv == 2, e[4], e[5]);
-            e[3] = s0;
-            e[4] = s1;
-        }
-#pragma unroll
-        for (int k = 0; k < U0Planes<T>::n; k++)
-            *elem_ptr(dst, off, k) = c_make<T>((T)e[k].re, (T)e[k].im);
+        for (int k = 0; k < kPlanes; k++) m.e[k] = src[k];
+        store_u0(m, u0_field(u0, Vh, p, i), h);
+        store_u0(m, u0_field(u0f, Vh, p, i), h);
     }
 }
 
@@ -678,16 +876,17 @@ __device__ __forceinline__ void block_reduce3(Obs o, double *__restrict__ part, 
 }
 
 // Observables of the factored state at site index idx in [0, 2 Vh) (parity
-// idx >= Vh); u0 of type TU, G of type TG, arithmetic in FP64.  They come
+// idx >= Vh); u0 in FP64 (in the axial frame with an FP64 G, in the
+// configuration's own with an FP32 one), arithmetic in FP64.  They come
 // from the site's w = G(n) W(n), formed as the sweep forms it:
 // w = sum_i [U_i(n) + U_i(n-i)^dagger], so w - w^dagger is the divergence
 // sum_i [(U - U^dagger)_i(n) - (U - U^dagger)_i(n-i)] that e2 and theta
 // measure (calculateA, divergenceA: src/four_potential.c), and
 // Re Tr w / 2 summed over all sites is the sum over links of Re Tr U that F
-// measures (calculateF, src/gauge_fixing.c).  Seven products instead of the
-// twelve of forming every link.
-template <typename TU, typename TG>
-__device__ __forceinline__ Obs obs_site(const cplx<TU> *__restrict__ u0,
+// measures (calculateF, src/gauge_fixing.c).  Seven products (five in the axial
+// frame) instead of the twelve of forming every link.
+template <typename TG>
+__device__ __forceinline__ Obs obs_site(const cplx<double> *__restrict__ u0,
                                         const cplx<TG> *__restrict__ g, int ns, int Vh,
                                         int idx) {
     Obs o = {0, 0, 0};
@@ -698,12 +897,21 @@ __device__ __forceinline__ Obs obs_site(const cplx<TU> *__restrict__ u0,
         const cplx<TG> *gq = g_field(g, Vh, 1 - p);
         mat3<double> W;
         m_zero(W);
+        constexpr bool axial = sizeof(TG) == sizeof(double);
+        if constexpr (axial) {
+            mat3<double> gf, gb;
+            load_su3_d(gf, gq, nb.fwd[0]);
+            load_su3_d(gb, gq, nb.bwd[0]);
+            axial_z<false>(W, u0, s, ns, Vh, p, gf, gb);
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
-        for (int i = 0; i < 3; i++) {
+        for (int i = axial ? 1 : 0; i < 3; i++) {
             mat3<double> uf, gf, ub, gb;
-            load_u0_d(uf, u0_field(u0, Vh, p, i), h);
+            load_u0_d(uf, axial ? axial_field(u0, Vh, p, i) : u0_field(u0, Vh, p, i), h);
             load_su3_d(gf, gq, nb.fwd[i]);
-            load_u0_d(ub, u0_field(u0, Vh, 1 - p, i), nb.bwd[i]);
+            load_u0_d(ub, axial ? axial_field(u0, Vh, 1 - p, i) : u0_field(u0, Vh, 1 - p, i),
+                      nb.bwd[i]);
             load_su3_d(gb, gq, nb.bwd[i]);
             m_mac_nd_su3(W, uf, gf);      // u0_i(n) G(n+i)^dagger
             m_mac_dagger_su3(W, gb, ub);  // (G(n-i) u0_i(n-i))^dagger
@@ -725,14 +933,14 @@ __device__ __forceinline__ Obs obs_site(const cplx<TU> *__restrict__ u0,
 // site order.  The workgroups run in XCD-contiguous order (xcd_order), so that
 // the neighbour G and backward u0 links a site reads were mostly brought into
 // its XCD's L2 by the sites next to it.
-template <typename TU, typename TG>
-__global__ __launch_bounds__(kBlock) void k_obs_factored(const cplx<TU> *__restrict__ u0,
+template <typename TG>
+__global__ __launch_bounds__(kBlock, 3) void k_obs_factored(const cplx<double> *__restrict__ u0,
                                                          const cplx<TG> *__restrict__ g,
                                                          int ns, int Vh,
                                                          double *__restrict__ part) {
     const unsigned b = xcd_order(blockIdx.x, gridDim.x);
     const int idx = (int)(b * kBlock + threadIdx.x);
-    block_reduce3(obs_site<TU, TG>(u0, g, ns, Vh, idx), part, b);
+    block_reduce3(obs_site<TG>(u0, g, ns, Vh, idx), part, b);
 }
 
 // Observables of an AoS FP64 configuration; one thread per site.
@@ -918,9 +1126,9 @@ __global__ __launch_bounds__(kBlock) void k_obs_batch(const BatchJob *__restrict
     const BatchJob J = jobs[it.x];
     const int idx = it.y * kBlock + (int)threadIdx.x;
     const cplx<double> *u0 = static_cast<const cplx<double> *>(J.u0d);
-    Obs o = it.z ? obs_site<double, float>(u0, static_cast<const cplx<float> *>(J.gf), J.ns,
+    Obs o = it.z ? obs_site<float>(u0, static_cast<const cplx<float> *>(J.gf), J.ns,
                                            J.Vh, idx)
-                 : obs_site<double, double>(u0, static_cast<const cplx<double> *>(J.gd), J.ns,
+                 : obs_site<double>(u0, static_cast<const cplx<double> *>(J.gd), J.ns,
                                             J.Vh, idx);
     block_reduce3(o, part + 3 * (int64_t)J.part_off, it.y);
 }

@@ -272,9 +272,8 @@ int admit_one(gfc_server *s, Lane &L, Req &r, bool &admitted) {
     hipLaunchKernelGGL(gfc::k_reunit_aos, dim3(nblocks(job->V * 4)), dim3(kBlock), 0, L.st,
                        job->cfg, job->V * 4, L.d_flags + slot);
     LAUNCH_CHECK();
-    RC_TRY(gfcx::build_u0(job, L.st));
-    RC_TRY(gfcx::set_identity(job, L.st));
     r.fp32 = r.o.precision == GFC_PREC_MIXED;
+    RC_TRY(gfcx::begin_fix(job, L.st, r.fp32));
     r.state = INIT;
     r.t_admit = s->clock();
     fill_desc(L, r);
@@ -296,8 +295,7 @@ int evaluate(gfc_server *s, Lane &L, std::vector<Req *> &which) {
         Req *r = which[q];
         L.h_jobs[r->slot].part_off = (int)k;
         const int nb = (int)nblocks(2 * (int64_t)r->job->Vh);
-        // the initial residue reads the FP64 G, like run_fix (engine.hip)
-        const int g32 = r->state == RUN && r->fp32 ? 1 : 0;
+        const int g32 = r->fp32 ? 1 : 0;
         for (int b = 0; b < nb; b++) L.h_oitems[k++] = make_int4(r->slot, b, g32, 0);
         L.h_sel[q] = r->slot;
     }
@@ -330,7 +328,7 @@ int evaluate(gfc_server *s, Lane &L, std::vector<Req *> &which) {
 }
 
 int promote(Lane &L, Req &r) {
-    RC_TRY(gfcx::promote_g_only(r.job, L.st));
+    RC_TRY(gfcx::promote_g(r.job, L.st));
     r.fp32 = false;
     fill_desc(L, r);
     L.plan_sig.clear();
@@ -340,8 +338,8 @@ int promote(Lane &L, Req &r) {
 // End of gaugefixOverrelaxation for r: hand-off, final reunitarization (unless
 // it stopped on max sweeps or a stalled residue), U = G U0 G^dagger.
 int finish(Lane &L, Req &r, int rc) {
-    if (r.fp32) RC_TRY(promote(L, r));
-    if (rc >= 0) RC_TRY(gfcx::reunit_g(r.job, L.st, false, 0, 2));
+    if (r.fp32 && r.sweep > 0) RC_TRY(promote(L, r));
+    RC_TRY(gfcx::end_frame(r.job, L.st, r.sweep, rc >= 0));
     RC_TRY(gfcx::materialize(r.job, L.st, rc >= 0));
     r.rc = rc >= 0 ? r.sweep : rc;
     r.state = DONE;
@@ -349,10 +347,12 @@ int finish(Lane &L, Req &r, int rc) {
 }
 
 // A request that cannot be fixed (its input could not be reunitarized): no
-// sweep, no result, the error code as its status.
-void fail_request(Req &r, int code) {
+// sweep, G = 1, the error code as its status.
+int fail_request(Lane &L, Req &r, int code) {
+    RC_TRY(gfcx::set_identity(r.job, L.st));
     r.rc = code;
     r.state = DONE;
+    return GFC_OK;
 }
 
 int next_multiple(int s, int m) { return (s / m + 1) * m; }
@@ -597,7 +597,7 @@ int poll_lane(gfc_server *s, int li) {
             // the lane)
             std::vector<char>().swap(r.host_cfg);
             if (L.h_flags[r.slot]) {
-                fail_request(r, GFC_EPROJECT);
+                RC_TRY(fail_request(L, r, GFC_EPROJECT));
                 continue;
             }
             r.res = r.res0 = r.obs[which];

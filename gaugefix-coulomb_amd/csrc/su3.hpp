@@ -92,15 +92,27 @@ __device__ __forceinline__ void m_mac_nd(mat3<T> &acc, const mat3<T> &a, const m
             for (int k = 0; k < 3; k++) c_mac_cb(acc.e[3 * i + j], a.e[3 * i + k], b.e[3 * j + k]);
 }
 
-// acc += a^dagger * b^dagger  (= (b a)^dagger)
 template <typename T>
-__device__ __forceinline__ void m_mac_dd(mat3<T> &acc, const mat3<T> &a, const mat3<T> &b) {
+__device__ __forceinline__ mat3<T> m_dagger(const mat3<T> &a) {
+    mat3<T> d;
 #pragma unroll
     for (int i = 0; i < 3; i++)
 #pragma unroll
         for (int j = 0; j < 3; j++)
+            d.e[3 * i + j] = c_make<T>(a.e[3 * j + i].re, -a.e[3 * j + i].im);
+    return d;
+}
+
+// acc += a^dagger
+template <typename T>
+__device__ __forceinline__ void m_add_dagger(mat3<T> &acc, const mat3<T> &a) {
 #pragma unroll
-            for (int k = 0; k < 3; k++) c_mac_cc(acc.e[3 * i + j], a.e[3 * k + i], b.e[3 * j + k]);
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            acc.e[3 * i + j].re += a.e[3 * j + i].re;
+            acc.e[3 * i + j].im -= a.e[3 * j + i].im;
+        }
 }
 
 // c = a * b^dagger
@@ -244,6 +256,103 @@ __device__ __forceinline__ bool m_project_su3(mat3<T> &m) {
     m.e[4] = c_make<T>(c1.re - d1.re, c1.im - d1.im);
     m.e[5] = c_make<T>(c2.re - d2.re, c2.im - d2.im);
     return ok;
+}
+
+// Compensated products (two-product and two-sum error terms kept beside the
+// sum), for the change of frame at the two ends of a fix: each matrix then
+// carries one rounding, as the links of the input do.  FMA contraction is off,
+// since the error terms hold for the rounded product.
+struct sum2 {
+    double hi, lo;
+};
+
+__device__ __forceinline__ void s2_mac(sum2 &s, double a, double b) {
+#pragma clang fp contract(off)
+    const double p = a * b, e = __builtin_fma(a, b, -p);
+    const double t = s.hi + p, v = t - s.hi;
+    s.lo += e + ((s.hi - (t - v)) + (p - v));
+    s.hi = t;
+}
+
+// re, im += a * b
+__device__ __forceinline__ void s2_cmac(sum2 &re, sum2 &im, const cplx<double> &a,
+                                        const cplx<double> &b) {
+    s2_mac(re, a.re, b.re);
+    s2_mac(re, -a.im, b.im);
+    s2_mac(im, a.re, b.im);
+    s2_mac(im, a.im, b.re);
+}
+
+// Rows [0, R) of hi + lo = (a + alo) b.
+template <int R>
+__device__ __forceinline__ void m_mul2(const mat3<double> &a, const mat3<double> &alo,
+                                       const mat3<double> &b, mat3<double> &hi,
+                                       mat3<double> &lo) {
+#pragma unroll
+    for (int i = 0; i < R; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            sum2 re = {0, 0}, im = {0, 0};
+            cplx<double> l = c_make<double>(0, 0);
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                s2_cmac(re, im, a.e[3 * i + k], b.e[3 * k + j]);
+                c_mac(l, alo.e[3 * i + k], b.e[3 * k + j]);
+            }
+            hi.e[3 * i + j] = c_make<double>(re.hi, im.hi);
+            lo.e[3 * i + j] = c_make<double>(re.lo + l.re, im.lo + l.im);
+        }
+}
+
+// The SU(3) matrix nearest hi + lo, whose rows 0 and 1 are orthonormal to
+// within some roundings, rounded once: first-order corrections of the rows'
+// norms and overlap from compensated sums, row 2 = conj(r0 x r1).  Matrices
+// further from SU(3) are projected as elsewhere.
+__device__ __forceinline__ void m_polish_su3(const mat3<double> &hi, const mat3<double> &lo,
+                                             mat3<double> &m) {
+    const cplx<double> *r0 = hi.e, *r1 = hi.e + 3, *l0 = lo.e, *l1 = lo.e + 3;
+    sum2 n0 = {-1, 0}, n1 = {-1, 0}, sre = {0, 0}, sim = {0, 0};
+    double c0 = 0, c1 = 0;
+    cplx<double> cs = c_make<double>(0, 0);
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+        s2_mac(n0, r0[b].re, r0[b].re);
+        s2_mac(n0, r0[b].im, r0[b].im);
+        s2_mac(n1, r1[b].re, r1[b].re);
+        s2_mac(n1, r1[b].im, r1[b].im);
+        s2_cmac(sre, sim, r1[b], c_make<double>(r0[b].re, -r0[b].im));
+        c0 += 2 * (r0[b].re * l0[b].re + r0[b].im * l0[b].im);
+        c1 += 2 * (r1[b].re * l1[b].re + r1[b].im * l1[b].im);
+        c_mac_cb(cs, r1[b], l0[b]);
+        c_mac_cb(cs, l1[b], r0[b]);
+    }
+    const double d0 = -0.5 * (n0.hi + (n0.lo + c0)), d1 = -0.5 * (n1.hi + (n1.lo + c1));
+    const cplx<double> s = c_make<double>(-(sre.hi + (sre.lo + cs.re)), -(sim.hi + (sim.lo + cs.im)));
+    const double off = 1e-10;
+    if (!(fabs(d0) < off && fabs(d1) < off && fabs(s.re) < off && fabs(s.im) < off)) {
+        m = hi;
+        m_project_su3(m);
+        return;
+    }
+    mat3<double> o;
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+        cplx<double> k0 = c_make<double>(l0[b].re + d0 * r0[b].re, l0[b].im + d0 * r0[b].im);
+        cplx<double> k1 = c_make<double>(l1[b].re + d1 * r1[b].re, l1[b].im + d1 * r1[b].im);
+        c_mac(k1, s, r0[b]);
+        o.e[b] = c_make<double>(r0[b].re + k0.re, r0[b].im + k0.im);
+        o.e[3 + b] = c_make<double>(r1[b].re + k1.re, r1[b].im + k1.im);
+    }
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+        const cplx<double> x0 = o.e[(b + 1) % 3], x1 = o.e[3 + (b + 2) % 3];
+        const cplx<double> y0 = o.e[(b + 2) % 3], y1 = o.e[3 + (b + 1) % 3];
+        sum2 re = {0, 0}, im = {0, 0};
+        s2_cmac(re, im, x0, x1);
+        s2_cmac(re, im, c_make<double>(-y0.re, -y0.im), y1);
+        o.e[6 + b] = c_make<double>(re.hi + re.lo, -(im.hi + im.lo));
+    }
+    m = o;
 }
 
 // determinant3x3 (src/SU3_ops.c:251-281), Leibniz expansion along row 0.

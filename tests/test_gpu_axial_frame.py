@@ -1,0 +1,59 @@
+"""The axial frame the sweeps run in (u0_Z = 1 but on the plane z = ns - 1).
+
+Haar-random links, so that the column products are general SU(3) matrices, on
+the smallest extents and on timeslices that are no whole number of tiles or
+waves: G and U after a few half-sweeps against the CPU oracle, which keeps
+every link.  Rounding of G: a column product is projected onto SU(3) at each
+step and enters G twice (G' = G h^dagger and back), a few 1e-16 each; the
+bound of 1e-11 is that of the drop-in tests (1e-10) less a decade.  A fix
+that needs no sweep leaves G = 1 exactly."""
+import numpy as np
+import pytest
+
+import gfc
+import oracle as orc
+from test_gpu_u0_pivot import _haar_su3
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ns,nt", [(2, 2), (2, 6), (4, 2), (6, 4), (10, 2), (18, 2)])
+def test_frame_matches_oracle(ctx, ns, nt):
+    geom = gfc.Geometry(ns, nt)
+    V = geom.volume
+    U = _haar_su3(np.random.default_rng(ns * 100 + nt), 4 * V).reshape(V, 4, 3, 3)
+    k = 11  # past a reunitarization
+    p = gfc.Params(tolerance=1e-300, estimate_sweeps_to_gf_progress=100000000,
+                   max_sweeps_to_fix=k, sweeps_to_reunitarization=10)
+    with gfc.Job(ctx, geom) as job:
+        job.upload_config(U)
+        assert job.reunitarize() == 0
+        rc, rep, tr = job.fix(p, trace_len=k)
+        G, Uf = job.download_gauge(), job.download_config()
+    Uo, Go = U.copy(), np.zeros((V, 3, 3), np.complex128)
+    orc.reunitarize(Uo)
+    rc_o, tr_o = orc.gaugefix(Uo, Go, orc.geom(ns, nt),
+                              orc.params(tolerance=1e-300, max_sweeps=k, estimate=100000000,
+                                         reunit_every=10), trace_len=k)
+    assert rc == rc_o == gfc.ENOTCONVERGED and rep.sweeps == k
+    dG, dU = np.max(np.abs(G - Go)), np.max(np.abs(Uf - Uo))
+    rel = np.max(np.abs(tr - tr_o) / tr_o)
+    print(f"{ns}^3x{nt}: max|dG| {dG:.2e}, max|dU| {dU:.2e}, e2 rel {rel:.2e}")
+    assert dG < 1e-11 and dU < 1e-11 and rel < 1e-12
+
+
+@pytest.mark.parametrize("precision", [gfc.PREC_FP64, gfc.PREC_MIXED])
+def test_no_sweep_leaves_identity(ctx, precision):
+    geom = gfc.Geometry(6, 4)
+    one = np.broadcast_to(np.eye(3, dtype=np.complex128), (geom.volume, 3, 3))
+    U = gfc.generate_smooth(geom, 3, 0.3)
+    bad = U.copy()
+    bad[5, 2] = np.nan
+    o = gfc.Options(precision=precision)
+    with gfc.Job(ctx, geom, precision) as job:
+        # a tolerance the input already meets, and a residue that is no number
+        for cfg, tol in ((U, 1e6), (bad, 1e-16)):
+            job.upload_config(cfg)
+            rc, rep = job.fix(gfc.Params(tolerance=tol), o)
+            assert rc == 0 and rep.sweeps == 0
+            assert np.array_equal(job.download_gauge(), one)
