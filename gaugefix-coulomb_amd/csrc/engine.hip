@@ -561,42 +561,42 @@ int lane_count(const gfc_job *j, const gfc_options &o, bool fp32) {
 }
 
 template <typename T, bool POUT, bool STREAM>
-void launch_sweep_pin(const cplx<T> *u0, cplx<T> *g, hipStream_t s, int ns, int Vh, int p,
+void launch_sweep_pin(const cplx<T> *u0, cplx<T> *g, hipStream_t s, const gfc::Extents &x, int p,
                       T omega, int hits, int h0, int count, bool pin) {
     const unsigned b = nblocks(count);
     if (pin)
         hipLaunchKernelGGL((gfc::k_sweep<T, POUT, STREAM, true>), dim3(b), dim3(kBlock), 0, s,
-                           u0, g, ns, Vh, p, omega, hits, h0, count);
+                           u0, g, x, p, omega, hits, h0, count);
     else
         hipLaunchKernelGGL((gfc::k_sweep<T, POUT, STREAM, false>), dim3(b), dim3(kBlock), 0, s,
-                           u0, g, ns, Vh, p, omega, hits, h0, count);
+                           u0, g, x, p, omega, hits, h0, count);
 }
 
 // A half-sweep launch: pout projects the swept parity's new G on output, pin
 // its G on input (see sweep_site), stream selects non-temporal loads.
 template <typename T>
-int launch_sweep(const cplx<T> *u0, cplx<T> *g, hipStream_t s, int ns, int Vh, int p, T omega,
-                 int hits, int h0, int count, bool pout, bool stream, bool pin = false) {
+int launch_sweep(const cplx<T> *u0, cplx<T> *g, hipStream_t s, const gfc::Extents &x, int p,
+                 T omega, int hits, int h0, int count, bool pout, bool stream, bool pin = false) {
     if (pout && stream)
-        launch_sweep_pin<T, true, true>(u0, g, s, ns, Vh, p, omega, hits, h0, count, pin);
+        launch_sweep_pin<T, true, true>(u0, g, s, x, p, omega, hits, h0, count, pin);
     else if (pout)
-        launch_sweep_pin<T, true, false>(u0, g, s, ns, Vh, p, omega, hits, h0, count, pin);
+        launch_sweep_pin<T, true, false>(u0, g, s, x, p, omega, hits, h0, count, pin);
     else if (stream)
-        launch_sweep_pin<T, false, true>(u0, g, s, ns, Vh, p, omega, hits, h0, count, pin);
+        launch_sweep_pin<T, false, true>(u0, g, s, x, p, omega, hits, h0, count, pin);
     else
-        launch_sweep_pin<T, false, false>(u0, g, s, ns, Vh, p, omega, hits, h0, count, pin);
+        launch_sweep_pin<T, false, false>(u0, g, s, x, p, omega, hits, h0, count, pin);
     LAUNCH_CHECK();
     return GFC_OK;
 }
 
 int half_sweep(gfc_job *j, SweepState &st, int parity, double omega, int hits) {
     hipStream_t s = j->ctx->stream;
-    const int ns = j->geom.ns, Vh = j->Vh;
+    const int Vh = j->Vh;
+    const gfc::Extents x = gfc::make_extents(j->geom.ns, Vh);
     const bool stream = stream_loads(j, st.fp32, 0, 1);
     if (st.fp32)
-        return launch_sweep(j->u0f, j->gf, s, ns, Vh, parity, (float)omega, hits, 0, Vh, false,
-                            stream);
-    return launch_sweep(j->u0, j->g, s, ns, Vh, parity, omega, hits, 0, Vh, false, stream);
+        return launch_sweep(j->u0f, j->gf, s, x, parity, (float)omega, hits, 0, Vh, false, stream);
+    return launch_sweep(j->u0, j->g, s, x, parity, omega, hits, 0, Vh, false, stream);
 }
 
 // Projects G on parities [p0, p0 + np) of the live array.
@@ -662,7 +662,8 @@ StreamSet ctx_streams(gfc_ctx *c) {
 int sweep_blocked(gfc_job *j, const StreamSet &ss, bool fp32, int from, int to, int group,
                   int max_lanes, double omega, int hits, unsigned R,
                   const std::vector<char> *active) {
-    const int ns = j->geom.ns, nt = j->geom.nt, Vh = j->Vh;
+    const int ns = j->geom.ns, nt = j->geom.nt;
+    const gfc::Extents x = gfc::make_extents(ns, j->Vh);
     const int S = ns * ns * ns / 2;  // parity sites per timeslice
     const int ngroups = (nt + group - 1) / group;
     // the groups to sweep: all, or (one timeslice per group) the active slices
@@ -693,10 +694,10 @@ int sweep_blocked(gfc_job *j, const StreamSet &ss, bool fp32, int from, int to, 
                     const int h0 = t0 * S;
                     const int count = (t0 + group <= nt ? group : nt - t0) * S;
                     if (fp32)
-                        RC_TRY(launch_sweep(j->u0f, j->gf, s, ns, Vh, k & 1, (float)omega, hits,
+                        RC_TRY(launch_sweep(j->u0f, j->gf, s, x, k & 1, (float)omega, hits,
                                             h0, count, pout, stream, pin));
                     else
-                        RC_TRY(launch_sweep(j->u0, j->g, s, ns, Vh, k & 1, omega, hits, h0,
+                        RC_TRY(launch_sweep(j->u0, j->g, s, x, k & 1, omega, hits, h0,
                                             count, pout, stream, pin));
                 }
             }
@@ -802,8 +803,7 @@ struct SliceTracker {
             b.u0 = fp32 ? (const void *)j->u0f : (const void *)j->u0;
             b.g = fp32 ? (void *)j->gf : (void *)j->g;
             b.omega = omega;
-            b.ns = j->geom.ns;
-            b.Vh = j->Vh;
+            b.x = gfc::make_extents(j->geom.ns, j->Vh);
             b.hits = hits;
             std::vector<int4> it[2];
             for (int t = 0; t < nt; t++)

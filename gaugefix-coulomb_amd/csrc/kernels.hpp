@@ -76,7 +76,7 @@ __device__ __forceinline__ void st_stream(cplx<float> *p, const cplx<float> &c) 
 
 // Tiled layout of a matrix field over n parity sites: the six stored complex
 // numbers of 32 consecutive sites form one 6 x 32 tile, element k of site h at
-// tile_elem(h) + 32 k.  One 32-bit offset (on a uniform base) plus immediate
+// (h / 32) 192 + h % 32 + 32 k.  One 32-bit offset (on a uniform base) plus immediate
 // steps of 32 elements addresses a whole matrix, and 32 lanes with
 // consecutive h read 32 consecutive numbers.  A field holds field_size(n)
 // complex numbers (n rounded up to whole tiles) and must stay below 4 GiB.
@@ -86,8 +86,15 @@ __host__ __device__ constexpr int64_t field_size(int64_t n) {
     return (n + kTile - 1) / kTile * kTile * kPlanes;
 }
 
-__device__ __forceinline__ uint32_t tile_elem(int h) {
-    return (uint32_t)(h >> 5) * (uint32_t)(kTile * kPlanes) + (uint32_t)(h & (kTile - 1));
+// (FP64: h < 2^26, so the tile number takes a full-rate 24-bit product)
+template <typename T>
+__device__ __forceinline__ uint32_t tile_bytes_of(int h, int planes) {
+    if constexpr (sizeof(T) == sizeof(double))
+        return __umul24((unsigned)(h >> 5), (unsigned)(kTile * planes * sizeof(cplx<T>))) +
+               (uint32_t)(h & (kTile - 1)) * (uint32_t)sizeof(cplx<T>);
+    else
+        return ((uint32_t)(h >> 5) * (uint32_t)(kTile * planes) + (uint32_t)(h & (kTile - 1))) *
+               (uint32_t)sizeof(cplx<T>);
 }
 
 template <typename T>
@@ -104,7 +111,7 @@ __device__ __forceinline__ cplx<T> *elem_ptr(cplx<T> *field, uint32_t byte_off, 
 
 template <typename T>
 __device__ __forceinline__ uint32_t tile_bytes(int h) {
-    return tile_elem(h) * (uint32_t)sizeof(cplx<T>);
+    return tile_bytes_of<T>(h, kPlanes);
 }
 
 // u0 fields.  The sweeps read all six u0 links of a site per update, two
@@ -134,8 +141,7 @@ __host__ __device__ constexpr int64_t u0_field_size(int64_t n) {
 
 template <typename T>
 __device__ __forceinline__ uint32_t u0_tile_bytes(int h) {
-    return ((uint32_t)(h >> 5) * (uint32_t)(kTile * U0Planes<T>::n) +
-            (uint32_t)(h & (kTile - 1))) * (uint32_t)sizeof(cplx<T>);
+    return tile_bytes_of<T>(h, U0Planes<T>::n);
 }
 
 // Field of the spatial links u0_i on parity p; field of G on parity p.
@@ -317,6 +323,60 @@ __device__ __forceinline__ Site site_of(int h, int p, int ns) {
     return s;
 }
 
+// Division of numbers below 2^26 by a fixed divisor d: n / d = n m >> s with
+// m = ceil(2^s / d), s = 26 + ceil(log2 d) (exact: m d - 2^s < d <= 2^(s - 26)).
+struct Divisor {
+    uint32_t d, m, s;
+};
+
+inline Divisor make_divisor(uint32_t d) {
+    uint32_t l = 0;
+    while ((1u << l) < d) l++;
+    return {d, (uint32_t)((((uint64_t)1 << (26 + l)) + d - 1) / d), 26 + l};
+}
+
+__device__ __forceinline__ uint32_t divide(uint32_t n, const Divisor &v) {
+    return (uint32_t)(((uint64_t)n * v.m) >> v.s);
+}
+
+// Extents of a lattice as the sweeps' index arithmetic uses them.
+struct Extents {
+    int ns, Vh;
+    Divisor nh, n;  // ns / 2, ns
+};
+
+inline Extents make_extents(int ns, int Vh) {
+    return {ns, Vh, make_divisor((uint32_t)ns / 2), make_divisor((uint32_t)ns)};
+}
+
+// n / d and n % d for n below 2^16 and d = inv^-1 below 2^15, in FP32:
+// (n + 1/2) / d is 1 / (2 d) or more from a whole number, further than its
+// rounding (3 2^-24 n / d).
+__device__ __forceinline__ int small_div(int &n, int d, float inv) {
+    const int q = (int)(((float)n + 0.5f) * inv);
+    n -= __mul24(q, d);
+    return q;
+}
+
+// site_of for the workgroups of a sweep: the first index of a workgroup, which
+// is uniform, is split by whole-number products on the scalar unit, and a
+// lane's offset of at most 255 carried over with small quotients (three 32-bit
+// divisions per lane took 75 vector instructions, 15 of them quarter-rate
+// products, of about 2050 in the FP32 update).
+__device__ __forceinline__ Site site_in_block(uint32_t first, int lane, int p, const Extents &x) {
+    const int ns = x.ns, nh = ns >> 1;
+    const uint32_t r0 = divide(first, x.nh), z0 = divide(r0, x.n), t0 = divide(z0, x.n);
+    const float inv_nh = __builtin_amdgcn_rcpf((float)nh), inv_n = 0.5f * inv_nh;
+    Site s;
+    s.xh = (int)(first - r0 * x.nh.d) + lane;
+    s.y = (int)(r0 - z0 * x.n.d) + small_div(s.xh, nh, inv_nh);
+    s.z = (int)(z0 - t0 * x.n.d) + small_div(s.y, ns, inv_n);
+    s.t = (int)t0 + small_div(s.z, ns, inv_n);
+    s.x = 2 * s.xh + ((s.y + s.z + s.t + p) & 1);
+    s.row = (int)first + lane - s.xh;
+    return s;
+}
+
 // Parity indices (in the other parity) of the six spatial neighbours, in the
 // direction order i = 0 (Z), 1 (Y), 2 (X).
 struct Nbr {
@@ -362,7 +422,7 @@ __device__ __forceinline__ void axial_z(mat3<double> &W, const cplx<double> *__r
 }
 
 // ---------------------------------------------------------------------------
-// The site update of parity index h on parity p: reads the u0 links (FP64: 4
+// The site update of parity index h = first + lane on parity p: reads the u0 links (FP64: 4
 // in the axial frame, and a Z link next to the wrap; FP32: 6), 6 neighbour G
 // and G(n); writes G(n).  Shared by the single-lattice and the
 // batched (serving) kernels, so a site computes the same bits in both.
@@ -375,10 +435,14 @@ __device__ __forceinline__ void axial_z(mat3<double> &W, const cplx<double> *__r
 // reads u0 and G(n) with non-temporal loads (data read once per sweep);
 // without it they are cached, for sweeps whose data stays in the Infinity
 // Cache from one half-sweep to the next.
-template <typename T, bool POUT = false, bool STREAM = true, bool PIN = false>
-__device__ __forceinline__ void sweep_site(const cplx<T> *__restrict__ u0,
-                                           cplx<T> *__restrict__ g, int ns, int Vh, int p,
-                                           T omega, int hits, int h) {
+//
+// FP32, in the configuration's own frame: the four matrices of a direction are
+// loaded together, one memory round trip per direction rather than the
+// compiler's two.
+template <typename T, bool POUT, bool STREAM, bool PIN>
+__device__ __forceinline__ void sweep_own(const cplx<T> *__restrict__ u0,
+                                          cplx<T> *__restrict__ g, int ns, int Vh, int p,
+                                          T omega, int hits, int h) {
     const Site s = site_of(h, p, ns);
     const Nbr nb = neighbours(s, h, ns);
     const cplx<T> *gq = g_field(static_cast<const cplx<T> *>(g), Vh, 1 - p);  // other parity
@@ -398,28 +462,13 @@ __device__ __forceinline__ void sweep_site(const cplx<T> *__restrict__ u0,
     // rather than the compiler's two (48^3 x 96: FP64 fix 1%, mixed 2% faster).
     mat3<T> W;
     m_zero(W);
-    constexpr bool axial = sizeof(T) == sizeof(double);
-    if constexpr (axial) {
-        cplx<T> rgf[kPlanes], rgb[kPlanes];
-        load_raw<false>(rgf, gq, tile_bytes<T>(nb.fwd[0]));
-        load_raw<false>(rgb, gq, tile_bytes<T>(nb.bwd[0]));
-        __builtin_amdgcn_sched_barrier(0);
-        mat3<T> gf, gb;
-        rows01(gf, rgf);
-        m_fill_row2(gf);
-        rows01(gb, rgb);
-        m_fill_row2(gb);
-        axial_z<STREAM>(W, u0, s, ns, Vh, p, gf, gb);
-    }
 #pragma unroll
-    for (int i = axial ? 1 : 0; i < 3; i++) {
+    for (int i = 0; i < 3; i++) {
         constexpr int NU = U0Planes<T>::n;
         cplx<T> ruf[NU], rub[NU], rgf[kPlanes], rgb[kPlanes];
-        const cplx<T> *fu = axial ? axial_field(u0, Vh, p, i) : u0_field(u0, Vh, p, i);
-        const cplx<T> *bu = axial ? axial_field(u0, Vh, 1 - p, i) : u0_field(u0, Vh, 1 - p, i);
-        load_raw<STREAM>(ruf, fu, u0_tile_bytes<T>(h));
+        load_raw<STREAM>(ruf, u0_field(u0, Vh, p, i), u0_tile_bytes<T>(h));
         load_raw<false>(rgf, gq, tile_bytes<T>(nb.fwd[i]));
-        load_raw<STREAM>(rub, bu, u0_tile_bytes<T>(nb.bwd[i]));
+        load_raw<STREAM>(rub, u0_field(u0, Vh, 1 - p, i), u0_tile_bytes<T>(nb.bwd[i]));
         load_raw<false>(rgb, gq, tile_bytes<T>(nb.bwd[i]));
         __builtin_amdgcn_sched_barrier(0);
         mat3<T> uf, gf, ub, gb;
@@ -442,6 +491,89 @@ __device__ __forceinline__ void sweep_site(const cplx<T> *__restrict__ u0,
     m_mul(upd, gn, out);
     if (POUT) project_g(out);
     store_su3<true>(out, gp, h);
+}
+
+// FP64, in the axial frame: the matrices of Z and Y come in one memory round
+// trip, those of X and G(n) in another, in 214 registers (2 waves per SIMD).
+// us per half-sweep at 64^3 x 128 / 48^3 x 96 / 32^3 x 64 / 24^3 x 48: 1475 /
+// 479 / 92 / 31.4; with a round trip per direction in 168 registers (3 waves),
+// three integer divisions per lane, and the compiler's contraction and branches
+// in the local update 1600 / 498 / 96.5 / 33.3.  Of the same update, X's loads
+// ahead of Y's products cost 0.3 to 2% and all loads first (one wave per SIMD)
+// 35 to 50%.
+template <bool POUT, bool STREAM, bool PIN>
+__device__ __forceinline__ void sweep_axial(const cplx<double> *__restrict__ u0,
+                                            cplx<double> *__restrict__ g, const Extents &x, int p,
+                                            double omega, int hits, int first, int lane) {
+    typedef cplx<double> C;
+    const int ns = x.ns, Vh = x.Vh, h = first + lane;
+    const Site s = site_in_block((uint32_t)first, lane, p, x);
+    const Nbr nb = neighbours(s, h, ns);
+    const C *gq = g_field(static_cast<const C *>(g), Vh, 1 - p);  // other parity
+    C *gp = g_field(g, Vh, p);
+    mat3<double> gn;
+    if (PIN) {
+        load_rows01<STREAM>(gn, static_cast<const C *>(gp), h);
+        project_g(gn);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    struct Raw {
+        C uf[5], gf[kPlanes], ub[5], gb[kPlanes];
+    };
+    auto load_dir = [&](Raw &r, int i) {
+        load_raw<STREAM>(r.uf, axial_field(u0, Vh, p, i), u0_tile_bytes<double>(h));
+        load_raw<false>(r.gf, gq, tile_bytes<double>(nb.fwd[i]));
+        load_raw<STREAM>(r.ub, axial_field(u0, Vh, 1 - p, i), u0_tile_bytes<double>(nb.bwd[i]));
+        load_raw<false>(r.gb, gq, tile_bytes<double>(nb.bwd[i]));
+    };
+    mat3<double> W, gf, gb;
+    m_zero(W);
+    auto use_dir = [&](const Raw &r) {
+        mat3<double> u;
+        u0_rows01(u, r.uf);
+        rows01(gf, r.gf);
+        m_fill_row2(gf);
+        m_mac_nd_su3(W, u, gf);  // u0_i(n) G(n+i)^dagger
+        u0_rows01(u, r.ub);
+        m_fill_row2(u);
+        rows01(gb, r.gb);
+        m_mac_dagger_su3(W, gb, u);  // (G(n-i) u0_i(n-i))^dagger
+    };
+    C zf[kPlanes], zb[kPlanes];
+    Raw y;
+    load_raw<false>(zf, gq, tile_bytes<double>(nb.fwd[0]));
+    load_raw<false>(zb, gq, tile_bytes<double>(nb.bwd[0]));
+    load_dir(y, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    rows01(gf, zf);
+    m_fill_row2(gf);
+    rows01(gb, zb);
+    m_fill_row2(gb);
+    axial_z<STREAM>(W, u0, s, ns, Vh, p, gf, gb);
+    __builtin_amdgcn_sched_barrier(0);
+    use_dir(y);
+    Raw r;
+    load_dir(r, 2);
+    if (!PIN) load_rows01<STREAM>(gn, static_cast<const C *>(gp), h);
+    __builtin_amdgcn_sched_barrier(0);
+    use_dir(r);
+    m_fill_row2(gn);  // with PIN, the third row a store and reload would give
+    mat3<double> w, upd, out;
+    m_mul(gn, W, w);
+    la_or_update(w, hits, omega, upd);
+    m_mul(upd, gn, out);
+    if (POUT) project_g(out);
+    store_su3<true>(out, gp, h);
+}
+
+template <typename T, bool POUT = false, bool STREAM = true, bool PIN = false>
+__device__ __forceinline__ void sweep_site(const cplx<T> *__restrict__ u0,
+                                           cplx<T> *__restrict__ g, const Extents &x, int p,
+                                           T omega, int hits, int first, int lane) {
+    if constexpr (sizeof(T) == sizeof(double))
+        sweep_axial<POUT, STREAM, PIN>(u0, g, x, p, omega, hits, first, lane);
+    else
+        sweep_own<T, POUT, STREAM, PIN>(u0, g, x.ns, x.Vh, p, omega, hits, first + lane);
 }
 
 // Workgroup order.  The hardware hands workgroup i of a launch to XCD i % 8,
@@ -467,13 +599,12 @@ __device__ __forceinline__ unsigned xcd_order(unsigned i, unsigned n) {
 // One red/black half-sweep on parity p over parity indices [h0, h0 + count).
 template <typename T, bool POUT = false, bool STREAM = true, bool PIN = false>
 __global__ __launch_bounds__(kBlock) void k_sweep(const cplx<T> *__restrict__ u0,
-                                                  cplx<T> *__restrict__ g, int ns, int Vh,
-                                                  int p, T omega, int hits, int h0,
-                                                  int count) {
+                                                  cplx<T> *__restrict__ g, Extents x, int p,
+                                                  T omega, int hits, int h0, int count) {
     const unsigned b = STREAM ? blockIdx.x : xcd_order(blockIdx.x, gridDim.x);
-    const int tid = (int)(b * kBlock + threadIdx.x);
-    if (tid >= count) return;
-    sweep_site<T, POUT, STREAM, PIN>(u0, g, ns, Vh, p, omega, hits, h0 + tid);
+    const int lane = (int)threadIdx.x;
+    if ((int)(b * kBlock) + lane >= count) return;
+    sweep_site<T, POUT, STREAM, PIN>(u0, g, x, p, omega, hits, h0 + (int)(b * kBlock), lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -1096,7 +1227,8 @@ struct BatchJob {
     const void *gd;   // FP64 G, for FP64-state observables
     const void *gf;   // FP32 G (MIXED only, else null), for FP32-state observables
     double omega;
-    int ns, Vh, hits;
+    Extents x;
+    int hits;
     int part_off;     // first partial-sum slot of this lattice (observables)
 };
 
@@ -1111,11 +1243,11 @@ __global__ __launch_bounds__(kBlock) void k_sweep_batch(const BatchJob *__restri
     if (i >= nitems) return;
     const int4 it = items[i];
     const BatchJob J = jobs[it.x];
-    const int h = it.y + (int)threadIdx.x;
-    if (h < J.Vh)
+    const int lane = (int)threadIdx.x;
+    if (it.y + lane < J.x.Vh)
         sweep_site<T, false, STREAM>(static_cast<const cplx<T> *>(J.u0),
-                                     static_cast<cplx<T> *>(J.g), J.ns, J.Vh, it.z, (T)J.omega,
-                                     J.hits, h);
+                                     static_cast<cplx<T> *>(J.g), J.x, it.z, (T)J.omega, J.hits,
+                                     it.y, lane);
 }
 
 // item = (job index, block index within the lattice's [0, 2 Vh) range, fp32 G?, _)
@@ -1126,10 +1258,10 @@ __global__ __launch_bounds__(kBlock) void k_obs_batch(const BatchJob *__restrict
     const BatchJob J = jobs[it.x];
     const int idx = it.y * kBlock + (int)threadIdx.x;
     const cplx<double> *u0 = static_cast<const cplx<double> *>(J.u0d);
-    Obs o = it.z ? obs_site<float>(u0, static_cast<const cplx<float> *>(J.gf), J.ns,
-                                           J.Vh, idx)
-                 : obs_site<double>(u0, static_cast<const cplx<double> *>(J.gd), J.ns,
-                                            J.Vh, idx);
+    Obs o = it.z ? obs_site<float>(u0, static_cast<const cplx<float> *>(J.gf), J.x.ns,
+                                           J.x.Vh, idx)
+                 : obs_site<double>(u0, static_cast<const cplx<double> *>(J.gd), J.x.ns,
+                                            J.x.Vh, idx);
     block_reduce3(o, part + 3 * (int64_t)J.part_off, it.y);
 }
 
@@ -1139,7 +1271,7 @@ __global__ __launch_bounds__(kBlock) void k_reduce_batch(const BatchJob *__restr
                                                          const double *__restrict__ part,
                                                          double *__restrict__ out) {
     const BatchJob J = jobs[sel[blockIdx.x]];
-    const int nb = (2 * J.Vh + kBlock - 1) / kBlock;
+    const int nb = (2 * J.x.Vh + kBlock - 1) / kBlock;
     reduce_parts(part + 3 * (int64_t)J.part_off, nb, out + 3 * blockIdx.x);
 }
 
@@ -1150,9 +1282,9 @@ __global__ __launch_bounds__(kBlock) void k_reunit_batch(const BatchJob *__restr
     const int4 it = items[blockIdx.x];
     const BatchJob J = jobs[it.x];
     const int idx = it.y * kBlock + (int)threadIdx.x;
-    if (idx >= 2 * J.Vh) return;
-    const int p = idx >= J.Vh;
-    reunit_site<T>(static_cast<cplx<T> *>(J.g), J.Vh, p, idx - p * J.Vh);
+    if (idx >= 2 * J.x.Vh) return;
+    const int p = idx >= J.x.Vh;
+    reunit_site<T>(static_cast<cplx<T> *>(J.g), J.x.Vh, p, idx - p * J.x.Vh);
 }
 
 // ---------------------------------------------------------------------------

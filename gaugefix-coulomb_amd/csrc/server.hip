@@ -205,8 +205,7 @@ void fill_desc(Lane &L, Req &r) {
     b.gd = j->g;
     b.gf = j->gf;
     b.omega = (double)r.p.omega_OR;
-    b.ns = j->geom.ns;
-    b.Vh = j->Vh;
+    b.x = gfc::make_extents(j->geom.ns, j->Vh);
     b.hits = (int)r.p.hits;
 }
 

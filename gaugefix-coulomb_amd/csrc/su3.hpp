@@ -55,6 +55,46 @@ __device__ __forceinline__ void c_mac_cc(cplx<T> &acc, const cplx<T> &a, const c
     acc.im -= a.im * b.re;
 }
 
+// FP64 in explicit FMAs, so that every kernel variant that forms the same
+// expression gives the same bits: left to the compiler, the contraction depends
+// on the code around it.  (FP32 leaves it to the compiler.)
+__device__ __forceinline__ void c_mac(cplx<double> &acc, const cplx<double> &a,
+                                      const cplx<double> &b) {
+    acc.re = __builtin_fma(-a.im, b.im, __builtin_fma(a.re, b.re, acc.re));
+    acc.im = __builtin_fma(a.im, b.re, __builtin_fma(a.re, b.im, acc.im));
+}
+__device__ __forceinline__ void c_mac_cb(cplx<double> &acc, const cplx<double> &a,
+                                         const cplx<double> &b) {
+    acc.re = __builtin_fma(a.im, b.im, __builtin_fma(a.re, b.re, acc.re));
+    acc.im = __builtin_fma(-a.re, b.im, __builtin_fma(a.im, b.re, acc.im));
+}
+
+// a b - c d, and its conjugate
+__device__ __forceinline__ cplx<double> c_det2(const cplx<double> &a, const cplx<double> &b,
+                                               const cplx<double> &c, const cplx<double> &d) {
+    cplx<double> r = c_make<double>(a.re * b.re, a.re * b.im);
+    r.re = __builtin_fma(-a.im, b.im, r.re);
+    r.re = __builtin_fma(-c.re, d.re, r.re);
+    r.re = __builtin_fma(c.im, d.im, r.re);
+    r.im = __builtin_fma(a.im, b.re, r.im);
+    r.im = __builtin_fma(-c.re, d.im, r.im);
+    r.im = __builtin_fma(-c.im, d.re, r.im);
+    return r;
+}
+__device__ __forceinline__ cplx<double> c_conj(const cplx<double> &a) {
+    return c_make<double>(a.re, -a.im);
+}
+
+// Squared norm of a row.
+__device__ __forceinline__ double row_norm(const cplx<double> *r) {
+    double n = r[0].re * r[0].re;
+    n = __builtin_fma(r[0].im, r[0].im, n);
+    n = __builtin_fma(r[1].re, r[1].re, n);
+    n = __builtin_fma(r[1].im, r[1].im, n);
+    n = __builtin_fma(r[2].re, r[2].re, n);
+    return __builtin_fma(r[2].im, r[2].im, n);
+}
+
 template <typename T>
 __device__ __forceinline__ void m_zero(mat3<T> &m) {
 #pragma unroll
@@ -139,6 +179,13 @@ __device__ __forceinline__ void m_fill_row2(mat3<T> &m) {
     m.e[8] = c_make<T>(c2.re - d2.re, c2.im - d2.im);
 }
 
+__device__ __forceinline__ void m_fill_row2(mat3<double> &m) {
+    const cplx<double> *r0 = m.e, *r1 = m.e + 3;
+    m.e[6] = c_conj(c_det2(r0[1], r1[2], r0[2], r1[1]));
+    m.e[7] = c_conj(c_det2(r0[2], r1[0], r0[0], r1[2]));
+    m.e[8] = c_conj(c_det2(r0[0], r1[1], r0[1], r1[0]));
+}
+
 template <typename T>
 __device__ __forceinline__ T inv_sqrt(T x);
 // FP64: the hardware estimate (v_rsq_f64) and two Newton steps
@@ -214,6 +261,15 @@ __device__ __forceinline__ void m_mac_dagger_su3(mat3<T> &acc, const mat3<T> &a,
                                          acc.e[3 * i + j].im - Q.e[3 * j + i].im);
 }
 
+// Row r of squared norm n normalised, or left as it is (false) when n is 0.
+__device__ __forceinline__ bool scale_row(cplx<double> *r, double n) {
+    const bool ok = n != 0.0;
+    const double s = inv_sqrt(ok ? n : 1.0);
+#pragma unroll
+    for (int b = 0; b < 3; b++) r[b] = c_make<double>(r[b].re * s, r[b].im * s);
+    return ok;
+}
+
 // projectSU3 (src/SU3_ops.c:994-1049): normalise row 0; row 2 = conj(r0 x r1)
 // normalised; row 1 = conj(r2 x r0).  Returns false when row 0 or the cross
 // product is null; the rows are then written unnormalised, as in the
@@ -256,6 +312,17 @@ __device__ __forceinline__ bool m_project_su3(mat3<T> &m) {
     m.e[4] = c_make<T>(c1.re - d1.re, c1.im - d1.im);
     m.e[5] = c_make<T>(c2.re - d2.re, c2.im - d2.im);
     return ok;
+}
+
+__device__ __forceinline__ bool m_project_su3(mat3<double> &m) {
+    const bool ok0 = scale_row(m.e, row_norm(m.e));
+    m_fill_row2(m);
+    const bool ok2 = scale_row(m.e + 6, row_norm(m.e + 6));
+    const cplx<double> *r0 = m.e, *r2 = m.e + 6;
+    m.e[3] = c_conj(c_det2(r2[1], r0[2], r2[2], r0[1]));
+    m.e[4] = c_conj(c_det2(r2[2], r0[0], r2[0], r0[2]));
+    m.e[5] = c_conj(c_det2(r2[0], r0[1], r2[1], r0[0]));
+    return ok0 && ok2;
 }
 
 // Compensated products (two-product and two-sum error terms kept beside the
@@ -377,11 +444,24 @@ __device__ __forceinline__ cplx<T> m_det(const mat3<T> &m) {
     return r;
 }
 
+__device__ __forceinline__ cplx<double> m_det(const mat3<double> &m) {
+    const cplx<double> *e = m.e;
+    cplx<double> r = c_make<double>(0, 0);
+    c_mac(r, e[0], c_det2(e[4], e[8], e[5], e[7]));
+    c_mac(r, e[1], c_det2(e[5], e[6], e[3], e[8]));
+    c_mac(r, e[2], c_det2(e[3], e[7], e[4], e[6]));
+    return r;
+}
+
 // The SU(2) element of a Cabibbo-Marinari step on rows (A, B) of w
 // (updateSubLosAlamos, src/SU3_ops.c:776-840 with projectSU2,
 // src/SU2_ops.c:369-402): x = a/|a| with a = (Re(w_AA + w_BB),
 // -Im(w_AB + w_BA), -Re(w_AB - w_BA), -Im(w_AA - w_BB)) maximises
-// Re Tr(x w_sub).  False for a null a (the step is then skipped).
+// Re Tr(x w_sub).  For a null a the reference skips the step: false (FP32), or
+// x = 1, which leaves the rows as they are (FP64).  A branch around the step
+// costs 84 register moves per update with two hits, where its paths join; the
+// FP32 sweeps wait for their bytes either way, and straight code would contract
+// into other FMAs there and so change their rounding.
 template <typename T, int A, int B>
 __device__ __forceinline__ bool cm_su2(const mat3<T> &w, T &a0, T &a1, T &a2, T &a3) {
     const cplx<T> waa = w.e[3 * A + A], wbb = w.e[3 * B + B];
@@ -390,6 +470,16 @@ __device__ __forceinline__ bool cm_su2(const mat3<T> &w, T &a0, T &a1, T &a2, T 
     a1 = -(wab.im + wba.im);
     a2 = -(wab.re - wba.re);
     a3 = -(waa.im - wbb.im);
+    if constexpr (sizeof(T) == sizeof(double)) {
+        const double n = __builtin_fma(a0, a0, __builtin_fma(a1, a1, __builtin_fma(a2, a2, a3 * a3)));
+        const bool null = n == 0.0;
+        const double r = inv_sqrt(null ? 1.0 : n);
+        a0 = null ? 1.0 : a0 * r;
+        a1 *= r;
+        a2 *= r;
+        a3 *= r;
+        return true;
+    }
     const T s = a0 * a0 + a1 * a1 + a2 * a2 + a3 * a3;
     if (s == T(0)) return false;
     const T r = inv_sqrt(s);
@@ -414,14 +504,38 @@ __device__ __forceinline__ void cm_rows(mat3<T> &m, T a0, T a1, T a2, T a3) {
     }
 }
 
+template <int A, int B>
+__device__ __forceinline__ void cm_rows(mat3<double> &m, double a0, double a1, double a2,
+                                        double a3) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        const cplx<double> p = m.e[3 * A + c], q = m.e[3 * B + c];
+        cplx<double> u, v;
+        u.re = __builtin_fma(a0, p.re, __builtin_fma(-a3, p.im, __builtin_fma(a2, q.re, -(a1 * q.im))));
+        u.im = __builtin_fma(a0, p.im, __builtin_fma(a3, p.re, __builtin_fma(a2, q.im, a1 * q.re)));
+        v.re = __builtin_fma(-a2, p.re, __builtin_fma(-a1, p.im, __builtin_fma(a0, q.re, a3 * q.im)));
+        v.im = __builtin_fma(-a2, p.im, __builtin_fma(a1, p.re, __builtin_fma(a0, q.im, -(a3 * q.re))));
+        m.e[3 * A + c] = u;
+        m.e[3 * B + c] = v;
+    }
+}
+
+template <typename T, int A, int B>
+__device__ __forceinline__ void cm_apply(mat3<T> &m, T a0, T a1, T a2, T a3) {
+    if constexpr (sizeof(T) == sizeof(double))
+        cm_rows<A, B>(m, a0, a1, a2, a3);
+    else
+        cm_rows<T, A, B>(m, a0, a1, a2, a3);
+}
+
 // One Cabibbo-Marinari step on rows (A, B): rows A, B of w and of the
 // accumulated update g are left-multiplied by the step's SU(2) element.
 template <typename T, int A, int B>
 __device__ __forceinline__ void cm_step(mat3<T> &w, mat3<T> &g) {
     T a0, a1, a2, a3;
     if (!cm_su2<T, A, B>(w, a0, a1, a2, a3)) return;
-    cm_rows<T, A, B>(w, a0, a1, a2, a3);
-    cm_rows<T, A, B>(g, a0, a1, a2, a3);
+    cm_apply<T, A, B>(w, a0, a1, a2, a3);
+    cm_apply<T, A, B>(g, a0, a1, a2, a3);
 }
 
 // The first two steps of the first hit, from g = 1 (what cm_step<0, 1> then
@@ -434,21 +548,28 @@ __device__ __forceinline__ void cm_first_two(mat3<T> &w, mat3<T> &g) {
     m_identity(g);
     T a0, a1, a2, a3;
     if (cm_su2<T, 0, 1>(w, a0, a1, a2, a3)) {
-        cm_rows<T, 0, 1>(w, a0, a1, a2, a3);
+        cm_apply<T, 0, 1>(w, a0, a1, a2, a3);
         g.e[0] = c_make<T>(a0, a3);
         g.e[1] = c_make<T>(a2, a1);
         g.e[3] = c_make<T>(-a2, a1);
         g.e[4] = c_make<T>(a0, -a3);
     }
     if (!cm_su2<T, 0, 2>(w, a0, a1, a2, a3)) return;
-    cm_rows<T, 0, 2>(w, a0, a1, a2, a3);
+    cm_apply<T, 0, 2>(w, a0, a1, a2, a3);
     // g rows 0 and 2: columns 0, 1 from row 0 alone (row 2 is 0 there),
     // column 2 from row 2 alone (row 0 is 0 there, row 2 is 1)
 #pragma unroll
     for (int c = 0; c < 2; c++) {
         const cplx<T> p = g.e[c];
-        g.e[c] = c_make<T>(a0 * p.re - a3 * p.im, a0 * p.im + a3 * p.re);
-        g.e[6 + c] = c_make<T>(-a2 * p.re - a1 * p.im, -a2 * p.im + a1 * p.re);
+        if constexpr (sizeof(T) == sizeof(double)) {
+            g.e[c] = c_make<T>(__builtin_fma(a0, p.re, -(a3 * p.im)),
+                               __builtin_fma(a0, p.im, a3 * p.re));
+            g.e[6 + c] = c_make<T>(__builtin_fma(-a2, p.re, -(a1 * p.im)),
+                                   __builtin_fma(-a2, p.im, a1 * p.re));
+        } else {
+            g.e[c] = c_make<T>(a0 * p.re - a3 * p.im, a0 * p.im + a3 * p.re);
+            g.e[6 + c] = c_make<T>(-a2 * p.re - a1 * p.im, -a2 * p.im + a1 * p.re);
+        }
     }
     g.e[2] = c_make<T>(a2, a1);
     g.e[8] = c_make<T>(a0, -a3);
@@ -497,7 +618,9 @@ __device__ __forceinline__ void la_or_update(mat3<T> &w, int hits, T omega, mat3
 #pragma unroll
     for (int k = 0; k < 9; k++) {
         T re = g.e[k].re, im = g.e[k].im;
-        if (k % 4 == 0)
+        if (k % 4 == 0 && sizeof(T) == sizeof(double))
+            g.e[k] = c_make<T>(__builtin_fma(omega, re - T(1), T(1)), omega * im);
+        else if (k % 4 == 0)
             g.e[k] = c_make<T>(T(1) + omega * (re - T(1)), omega * im);
         else
             g.e[k] = c_make<T>(omega * re, omega * im);
