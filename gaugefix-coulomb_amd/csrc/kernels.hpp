@@ -299,7 +299,7 @@ __device__ __forceinline__ void project_g(mat3<float> &m) {
     mat3<double> d;
 #pragma unroll
     for (int k = 0; k < kPlanes; k++) d.e[k] = c_make<double>(m.e[k].re, m.e[k].im);
-    m_project_su3(d);
+    m_project_su3<double>(d);  // the rounding it always had: FP32 results hang on it
 #pragma unroll
     for (int k = 0; k < kPlanes; k++) m.e[k] = c_make<float>((float)d.e[k].re, (float)d.e[k].im);
 }

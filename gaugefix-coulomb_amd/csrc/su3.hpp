@@ -287,7 +287,7 @@ __device__ __forceinline__ bool m_project_su3(mat3<T> &m) {
     } else {
         ok = false;
     }
-    m_fill_row2(m);
+    m_fill_row2<T>(m);
     T n2 = 0;
 #pragma unroll
     for (int b = 6; b < 9; b++) n2 += m.e[b].re * m.e[b].re + m.e[b].im * m.e[b].im;
