@@ -132,6 +132,9 @@ void gfc_ctx_destroy(gfc_ctx *c) {
         if (c->pin[k]) hipHostFree(c->pin[k]);
         if (c->pin_ev[k]) hipEventDestroy(c->pin_ev[k]);
     }
+    hipHostFree(c->ring);
+    for (hipEvent_t e : c->slot_ev)
+        if (e) hipEventDestroy(e);
     if (c->fork) hipEventDestroy(c->fork);
     for (int k = 0; k < gfc_ctx::kLanes; k++)
         if (c->join[k]) hipEventDestroy(c->join[k]);
@@ -332,12 +335,12 @@ extern "C" int gfc_job_upload_config(gfc_job *j, const void *U, int in_precision
     hipStream_t s = j->ctx->stream;
     const int64_t nreal = j->V * 4 * 18;
     if (in_precision == 8) {
-        HIP_TRY(hipMemcpyAsync(j->cfg, U, nreal * sizeof(double), hipMemcpyHostToDevice, s));
+        RC_TRY(copy_from_host(j->ctx, s, j->cfg, U, nreal * sizeof(double)));
     } else {
         // FP32 staging lands in the u0 planes: 18V complex doubles = 288V bytes,
         // exactly the 4V x 18 floats of an FP32 configuration
         float *stage = reinterpret_cast<float *>(j->u0);
-        HIP_TRY(hipMemcpyAsync(stage, U, nreal * sizeof(float), hipMemcpyHostToDevice, s));
+        RC_TRY(copy_from_host(j->ctx, s, stage, U, nreal * sizeof(float)));
         hipLaunchKernelGGL(gfc::k_f32_to_f64, dim3(nblocks(nreal)), dim3(kBlock), 0, s, stage,
                            reinterpret_cast<double *>(j->cfg), nreal);
         LAUNCH_CHECK();
@@ -1067,10 +1070,8 @@ extern "C" int gfc_job_plaquette(gfc_job *j, double *spatial, double *temporal) 
 extern "C" int gfc_job_download_config(gfc_job *j, double *U) {
     if (j == nullptr || U == nullptr) return fail(GFC_EINVAL, "gfc_job_download_config: NULL");
     HIP_TRY(hipSetDevice(j->ctx->device));
-    HIP_TRY(hipMemcpyAsync(U, j->cfg, (size_t)j->V * 4 * 18 * sizeof(double),
-                           hipMemcpyDeviceToHost, j->ctx->stream));
-    HIP_TRY(hipStreamSynchronize(j->ctx->stream));
-    return GFC_OK;
+    return copy_to_host(j->ctx, j->ctx->stream, U, j->cfg,
+                        (size_t)j->V * 4 * 18 * sizeof(double));
 }
 
 extern "C" int gfc_job_save_config(gfc_job *j) {
@@ -1120,10 +1121,7 @@ extern "C" int gfc_job_download_gauge(gfc_job *j, double *G) {
     hipLaunchKernelGGL(gfc::k_g_to_aos, dim3(nblocks(j->V)), dim3(kBlock), 0, s, j->g, stage,
                        j->geom.ns, j->Vh);
     LAUNCH_CHECK();
-    HIP_TRY(hipMemcpyAsync(G, stage, (size_t)j->V * 18 * sizeof(double), hipMemcpyDeviceToHost,
-                           s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return GFC_OK;
+    return copy_to_host(j->ctx, s, G, stage, (size_t)j->V * 18 * sizeof(double));
 }
 
 extern "C" int gfc_fix_coulomb_or(gfc_ctx *ctx, const gfc_geom *g, const gfc_params *p,

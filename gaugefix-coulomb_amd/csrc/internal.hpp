@@ -6,6 +6,7 @@
 
 #include <cmath>
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -60,9 +61,15 @@ struct gfc_ctx {
     hipStream_t lane[kLanes] = {};
     hipEvent_t fork = nullptr;
     hipEvent_t join[kLanes] = {};
-    // pinned host blocks of the file streams (io_device.hip), made on first use
+    // pinned host blocks of the transfers to and from files, and the ring of
+    // those to and from host arrays (io_device.hip), made on first use; one
+    // transfer at a time
+    std::mutex pin_mu;
     void *pin[2] = {nullptr, nullptr};
     hipEvent_t pin_ev[2] = {nullptr, nullptr};
+    static constexpr int kSlots = 4;
+    char *ring = nullptr;
+    hipEvent_t slot_ev[kSlots] = {};
 };
 
 struct gfc_job {
@@ -95,6 +102,11 @@ int promote_g(gfc_job *j, hipStream_t s);
 int generate_smooth_device(gfc_job *j, uint64_t seed, double eps);
 int generate_smooth_device(gfc_job *j, hipStream_t s, uint64_t seed, double eps);
 int ensure_partials(gfc_ctx *c, size_t blocks);
+
+// Transfers of host arrays (io_device.hip).
+int copy_to_host(gfc_ctx *c, hipStream_t s, void *dst, const void *src, size_t total);
+int copy_from_host(gfc_ctx *c, hipStream_t s, void *dst, const void *src, size_t total);
+void copy_host(void *dst, const void *src, size_t total);
 
 // Streams over which timeslice groups run at once; lane[0] is the stream the
 // work is forked from and joined back into.

@@ -43,6 +43,7 @@
 #include <deque>
 #include <map>
 #include <memory>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -86,7 +87,7 @@ struct Req {
     double eps = 0;
     // a caller-supplied configuration (4V x 18 reals of in_prec bytes), kept
     // until its copy to the device has completed; empty: synthesise from seed
-    std::vector<char> host_cfg;
+    std::unique_ptr<char[]> host_cfg;
     int in_prec = 0;
     gfc_params p{};
     gfc_options o{};
@@ -250,16 +251,16 @@ int admit_one(gfc_server *s, Lane &L, Req &r, bool &admitted) {
     r.slot = slot;
     // input: the caller's configuration or one synthesised in HBM,
     // reunitarized like the CLI does after loading (gauge_fix_coulomb.c:126)
-    if (!r.host_cfg.empty()) {
+    if (r.host_cfg) {
         const int64_t nreal = job->V * 4 * 18;
         if (r.in_prec == 8) {
-            HIP_TRY(hipMemcpyAsync(job->cfg, r.host_cfg.data(), nreal * sizeof(double),
-                                   hipMemcpyHostToDevice, L.st));
+            RC_TRY(gfcx::copy_from_host(s->ctx, L.st, job->cfg, r.host_cfg.get(),
+                                        nreal * sizeof(double)));
         } else {
             // FP32 staging in the u0 planes (rebuilt below), as gfc_job_upload_config
             float *stage = reinterpret_cast<float *>(job->u0);
-            HIP_TRY(hipMemcpyAsync(stage, r.host_cfg.data(), nreal * sizeof(float),
-                                   hipMemcpyHostToDevice, L.st));
+            RC_TRY(gfcx::copy_from_host(s->ctx, L.st, stage, r.host_cfg.get(),
+                                        nreal * sizeof(float)));
             hipLaunchKernelGGL(gfc::k_f32_to_f64, dim3(nblocks(nreal)), dim3(kBlock), 0, L.st,
                                stage, reinterpret_cast<double *>(job->cfg), nreal);
             LAUNCH_CHECK();
@@ -594,7 +595,7 @@ int poll_lane(gfc_server *s, int li) {
         if (r.state == INIT) {
             // the input's copy to the device has completed (evaluate synchronised
             // the lane)
-            std::vector<char>().swap(r.host_cfg);
+            r.host_cfg.reset();
             if (L.h_flags[r.slot]) {
                 RC_TRY(fail_request(L, r, GFC_EPROJECT));
                 continue;
@@ -843,11 +844,10 @@ int64_t gfc_server_submit_config(gfc_server *s, const gfc_geom *g, const void *U
         if (in_precision != 4 && in_precision != 8)
             return fail(GFC_EINVAL, "gfc_server_submit_config: precision must be 4 or 8");
         const size_t bytes = (size_t)gfc_geom_volume(g) * 4 * 18 * (size_t)in_precision;
-        try {
-            r.host_cfg.assign(static_cast<const char *>(U), static_cast<const char *>(U) + bytes);
-        } catch (const std::bad_alloc &) {
+        r.host_cfg.reset(new (std::nothrow) char[bytes]);
+        if (!r.host_cfg)
             return fail(GFC_ENOMEM, "gfc_server_submit_config: host copy of the input");
-        }
+        gfcx::copy_host(r.host_cfg.get(), U, bytes);
         r.in_prec = in_precision;
         return GFC_OK;
     });

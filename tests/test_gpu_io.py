@@ -81,3 +81,35 @@ def test_write_gauge_transf_matches_host_writer(ctx, tmp_path, U):
     assert data == open(host, "rb").read()
     rc, G2 = gfc.load_gauge_transf(dev, GEOM)
     assert rc == 0 and np.array_equal(G2, G)
+
+
+@pytest.mark.parametrize("ns,nt", [(12, 100), (16, 100), (16, 102), (18, 256)])
+def test_host_arrays_round_trip(ctx, ns, nt):
+    """Uploads and downloads of host arrays, plain and through the ring of
+    pinned slots: sizes below and above its thresholds, and around whole slots
+    and pieces.  An FP64 image must come back as it was, bit for bit, an FP32
+    one as its promotion; and two threads may move different jobs at once."""
+    import threading
+    geom = gfc.Geometry(ns, nt)
+    rng = np.random.default_rng(ns * nt)
+    U = rng.standard_normal((geom.volume, 4, 3, 3, 2)).view(np.complex128)[..., 0]
+    with gfc.Job(ctx, geom) as job, gfc.Job(ctx, geom) as other:
+        job.upload_config(U)
+        assert np.array_equal(job.download_config(), U)
+        U4 = U.astype(np.complex64)
+        got = [None, None]
+
+        def move(k, j, a):
+            j.upload_config(a)
+            got[k] = j.download_config()
+
+        th = [threading.Thread(target=move, args=(0, job, U4)),
+              threading.Thread(target=move, args=(1, other, U))]
+        for t in th:
+            t.start()
+        for t in th:
+            t.join()
+        assert np.array_equal(got[0], U4.astype(np.complex128))
+        assert np.array_equal(got[1], U)
+        one = np.broadcast_to(np.eye(3, dtype=np.complex128), (geom.volume, 3, 3))
+        assert np.array_equal(job.download_gauge(), one)
