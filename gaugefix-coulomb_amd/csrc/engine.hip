@@ -543,14 +543,19 @@ bool stream_loads(const gfc_job *j, bool fp32, int group, int lanes) {
 }
 
 // Lattices of at least this many parity sites that fit in kCacheBytes whole
-// are swept as three concurrent groups rather than one whole-lattice launch.
-constexpr int64_t kSplitMinSites = 1 << 17;
+// are swept as three concurrent groups, smaller ones of more than kOneGroup
+// parity sites (one workgroup per CU) as two, the others as one.
+constexpr int kSplitMinSites = 1 << 17;
+constexpr int kOneGroup = 256 * kBlock;
 
 // Streams over which the timeslice groups of precision fp32 run at once
 // (gfc_options.slice_lanes, or by default, measured on full fixes):
-// * three for a lattice of at least kSplitMinSites parity sites that fits the
-//   cache whole (three groups of nt/3 timeslices: 20^3 x 40 FP64 and FP32 23%
-//   and 18% faster than one whole-lattice launch, 24^3 x 48 FP32 20%);
+// * for a lattice that fits the cache whole, by its parity sites, in one, two
+//   or three groups (us per half-sweep, one / two / three streams, in FP64:
+//   16^3 x 32 8.1 / 8.9 / 10.3, 18^3 x 36 14.7 / 11.5 / 12.4, 20^3 x 40 21.3 /
+//   17.2 / 16.0; in FP32 7.2 / 8.6 / 9.5, 10.4 / 9.6 / 9.9, 15.0 / 13.1 / 11.4).
+//   One group is a launch per half-sweep, as in whole-lattice sweeps, but with
+//   the reunitarizations folded in (16^3 x 32: 10.8 -> 8.1 us with R = 10);
 // * two for FP64 single timeslices too large for a cache-resident wave
 //   (64^3 x 128: 6% faster than four);
 // * four otherwise.
@@ -558,7 +563,8 @@ int lane_count(const gfc_job *j, const gfc_options &o, bool fp32) {
     if (o.slice_lanes >= 1 && o.slice_lanes <= gfc_ctx::kLanes) return o.slice_lanes;
     if (o.slice_group != 0) return gfc_ctx::kLanes;
     const int64_t ts = slice_bytes(j, fp32);
-    if ((int64_t)j->geom.nt * ts <= kCacheBytes) return j->Vh >= kSplitMinSites ? 3 : 1;
+    if ((int64_t)j->geom.nt * ts <= kCacheBytes)
+        return j->Vh >= kSplitMinSites ? 3 : j->Vh > kOneGroup ? 2 : 1;
     if (!fp32 && gfc_ctx::kLanes * ts > kCacheBytes) return 2;
     return gfc_ctx::kLanes;
 }
@@ -623,8 +629,8 @@ int reunit_g(gfc_job *j, hipStream_t s, bool fp32, int p0, int np) {
 // precision fp32.  The groups are spread over the context's streams, a wave
 // of one group per stream at a time, so that one group's kernel tail overlaps
 // the others' work.  By default (slice_group = 0), with L = lane_count:
-// * a lattice whose u0 and G fit in kCacheBytes: nt / L timeslices per group,
-//   or the whole lattice in one launch when L = 1; from the cache;
+// * a lattice whose u0 and G fit in kCacheBytes: nt / L timeslices per group;
+//   from the cache;
 // * otherwise, if a wave of L single timeslices fits, the largest groups whose
 //   wave fits, evened out so that every wave fills all streams (64^3 x 128 in
 //   FP64: single timeslices on two streams, from the cache);
@@ -637,8 +643,7 @@ int group_size(const gfc_job *j, const gfc_options &o, bool fp32) {
     if (o.slice_group > 0) return o.slice_group < nt ? o.slice_group : nt;
     const int64_t ts = slice_bytes(j, fp32);
     const int64_t L = lane_count(j, o, fp32);
-    if ((int64_t)nt * ts <= kCacheBytes)
-        return L > 1 && nt >= L ? (int)((nt + L - 1) / L) : 0;
+    if ((int64_t)nt * ts <= kCacheBytes) return (int)((nt + L - 1) / L);
     const int64_t nmax = kCacheBytes / (L * ts);
     if (nmax < 1) return 1;
     const int64_t waves = (nt + L * nmax - 1) / (L * nmax);
@@ -653,6 +658,38 @@ StreamSet ctx_streams(gfc_ctx *c) {
     }
     ss.fork = c->fork;
     return ss;
+}
+
+// Lattices of at most this many parity sites per timeslice (ns <= 10) run their
+// FP64 sweeps between two host decisions in one launch (k_sweep_slices).  At
+// ns = 10 a workgroup fills a CU, so more than 256 timeslices take turns: us
+// per half-sweep at nt = 300 18.8 against 16.4 in groups of timeslices, at
+// nt = 1024 41 against 50.  At ns <= 8 it is the faster one at every nt.
+constexpr int kSliceSites = 512;
+
+bool whole_slices(const gfc_job *j, const gfc_options &o, bool fp32) {
+    const int ns = j->geom.ns, nt = j->geom.nt;
+    return !fp32 && o.slice_group == 0 && ns <= 10 && (ns <= 8 || nt <= 256 || nt >= 1024);
+}
+
+int sweep_slices(gfc_job *j, int from, int to, double omega, int hits, unsigned R) {
+    const int ns = j->geom.ns, S = ns * ns * ns / 2;
+    const gfc::Extents x = gfc::make_extents(ns, j->Vh);
+    const dim3 grid((unsigned)j->geom.nt);
+    hipStream_t s = j->ctx->stream;
+    // at most some 20 ms a launch
+    constexpr int kMost = 2000;
+    for (int a = from; a < to; a += kMost) {
+        const int b = std::min(to, a + kMost);
+        if (S <= 256)
+            hipLaunchKernelGGL((gfc::k_sweep_slices<256>), grid, dim3(256), 0, s, j->u0, j->g, x,
+                               omega, hits, a, b, to, R);
+        else
+            hipLaunchKernelGGL((gfc::k_sweep_slices<kSliceSites>), grid, dim3(kSliceSites), 0, s,
+                               j->u0, j->g, x, omega, hits, a, b, to, R);
+        LAUNCH_CHECK();
+    }
+    return GFC_OK;
 }
 
 // Half-sweeps [from, to) (parity = sweep number & 1), timeslice group by
@@ -928,14 +965,18 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
     bool done = false;
     // per-sweep traces need the state after every sweep of the whole lattice;
     // the other sweeps run timeslice-blocked, with slice retirement one
-    // timeslice per group so that retired slices are left out
+    // timeslice per group so that retired slices are left out (small lattices:
+    // in whole-lattice launches over the active slices)
     const bool may_block = trace == nullptr;
+    const bool per_slice = o.slice_group > 0 || j->Vh >= kSplitMinSites ||
+                           j->geom.nt * slice_bytes(j, st.fp32) > kCacheBytes;
     while (res > p->tolerance) {
         int group = may_block ? group_size(j, o, st.fp32) : 0;
-        if (sl.on && group > 0) group = 1;
+        if (sl.on && group > 0) group = per_slice ? 1 : 0;
         const bool in32 = st.fp32;
+        const bool slices = may_block && !sl.on && whole_slices(j, o, st.fp32);
         timer.before();
-        if (group > 0) {
+        if (group > 0 || slices) {
             // the next sweep after which the host looks at the state
             int64_t stop = due;
             const int64_t pe = o.mixed_probe_every;
@@ -944,9 +985,13 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
             if (st.fp32 && ho.switch_at > sweep) stop = std::min<int64_t>(stop, ho.switch_at);
             stop = std::min<int64_t>(stop, (int64_t)p->max_sweeps_to_fix);
             if (stop <= sweep) stop = sweep + 1;
-            RC_TRY(sweep_blocked(j, ctx_streams(j->ctx), st.fp32, sweep, (int)stop, group,
-                                 lane_count(j, o, st.fp32), omega, hits,
-                                 p->sweeps_to_reunitarization, sl.on ? &sl.active : nullptr));
+            if (slices)
+                RC_TRY(sweep_slices(j, sweep, (int)stop, omega, hits,
+                                    p->sweeps_to_reunitarization));
+            else
+                RC_TRY(sweep_blocked(j, ctx_streams(j->ctx), st.fp32, sweep, (int)stop, group,
+                                     lane_count(j, o, st.fp32), omega, hits,
+                                     p->sweeps_to_reunitarization, sl.on ? &sl.active : nullptr));
             if (sl.on) sl.slice_sweeps += (double)(stop - sweep) * sl.n_active / sl.nt;
             if (in32) r.sweeps_fp32 += (int)stop - sweep;
             sweep = (int)stop;

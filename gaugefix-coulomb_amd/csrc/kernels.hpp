@@ -501,6 +501,23 @@ __device__ __forceinline__ void sweep_own(const cplx<T> *__restrict__ u0,
 // in the local update 1600 / 498 / 96.5 / 33.3.  Of the same update, X's loads
 // ahead of Y's products cost 0.3 to 2% and all loads first (one wave per SIMD)
 // 35 to 50%.
+struct AxialDir {
+    cplx<double> uf[5], gf[kPlanes], ub[5], gb[kPlanes];
+};
+
+// W += u0_i(n) G(n+i)^dagger + u0_i(n-i)^dagger G(n-i)^dagger
+__device__ __forceinline__ void axial_dir(mat3<double> &W, const AxialDir &r) {
+    mat3<double> u, m;
+    u0_rows01(u, r.uf);
+    rows01(m, r.gf);
+    m_fill_row2(m);
+    m_mac_nd_su3(W, u, m);
+    u0_rows01(u, r.ub);
+    m_fill_row2(u);
+    rows01(m, r.gb);
+    m_mac_dagger_su3(W, m, u);  // (G(n-i) u0_i(n-i))^dagger
+}
+
 template <bool POUT, bool STREAM, bool PIN>
 __device__ __forceinline__ void sweep_axial(const cplx<double> *__restrict__ u0,
                                             cplx<double> *__restrict__ g, const Extents &x, int p,
@@ -517,10 +534,7 @@ __device__ __forceinline__ void sweep_axial(const cplx<double> *__restrict__ u0,
         project_g(gn);
         __builtin_amdgcn_sched_barrier(0);
     }
-    struct Raw {
-        C uf[5], gf[kPlanes], ub[5], gb[kPlanes];
-    };
-    auto load_dir = [&](Raw &r, int i) {
+    auto load_dir = [&](AxialDir &r, int i) {
         load_raw<STREAM>(r.uf, axial_field(u0, Vh, p, i), u0_tile_bytes<double>(h));
         load_raw<false>(r.gf, gq, tile_bytes<double>(nb.fwd[i]));
         load_raw<STREAM>(r.ub, axial_field(u0, Vh, 1 - p, i), u0_tile_bytes<double>(nb.bwd[i]));
@@ -528,35 +542,20 @@ __device__ __forceinline__ void sweep_axial(const cplx<double> *__restrict__ u0,
     };
     mat3<double> W, gf, gb;
     m_zero(W);
-    auto use_dir = [&](const Raw &r) {
-        mat3<double> u;
-        u0_rows01(u, r.uf);
-        rows01(gf, r.gf);
-        m_fill_row2(gf);
-        m_mac_nd_su3(W, u, gf);  // u0_i(n) G(n+i)^dagger
-        u0_rows01(u, r.ub);
-        m_fill_row2(u);
-        rows01(gb, r.gb);
-        m_mac_dagger_su3(W, gb, u);  // (G(n-i) u0_i(n-i))^dagger
-    };
-    C zf[kPlanes], zb[kPlanes];
-    Raw y;
-    load_raw<false>(zf, gq, tile_bytes<double>(nb.fwd[0]));
-    load_raw<false>(zb, gq, tile_bytes<double>(nb.bwd[0]));
+    load_rows01<false>(gf, gq, nb.fwd[0]);
+    load_rows01<false>(gb, gq, nb.bwd[0]);
+    AxialDir y, r;
     load_dir(y, 1);
     __builtin_amdgcn_sched_barrier(0);
-    rows01(gf, zf);
     m_fill_row2(gf);
-    rows01(gb, zb);
     m_fill_row2(gb);
     axial_z<STREAM>(W, u0, s, ns, Vh, p, gf, gb);
     __builtin_amdgcn_sched_barrier(0);
-    use_dir(y);
-    Raw r;
+    axial_dir(W, y);
     load_dir(r, 2);
     if (!PIN) load_rows01<STREAM>(gn, static_cast<const C *>(gp), h);
     __builtin_amdgcn_sched_barrier(0);
-    use_dir(r);
+    axial_dir(W, r);
     m_fill_row2(gn);  // with PIN, the third row a store and reload would give
     mat3<double> w, upd, out;
     m_mul(gn, W, w);
@@ -605,6 +604,89 @@ __global__ __launch_bounds__(kBlock) void k_sweep(const cplx<T> *__restrict__ u0
     const int lane = (int)threadIdx.x;
     if ((int)(b * kBlock) + lane >= count) return;
     sweep_site<T, POUT, STREAM, PIN>(u0, g, x, p, omega, hits, h0 + (int)(b * kBlock), lane);
+}
+
+// Half-sweeps [from, to) of a small lattice in FP64, one workgroup per
+// timeslice and one thread per site of each parity (S = ns^3 / 2 <= N sites):
+// timeslices do not interact, so a workgroup runs through all the sweeps by
+// itself, its G in LDS, with a workgroup barrier where the other path has a
+// launch boundary.  Reunitarizations after the sweeps s + 1 < end that are
+// multiples of R, as in the timeslice-blocked sweeps; the same bits.
+//
+// Bound by one wave's chain of instructions: a half-sweep launch of 8^3 x 16
+// lasts 8.5 us alone (9.4 from one to the next) whatever its loads and code
+// size, a half-sweep here 4.7 us, at 8^3 x 2048 39 against 50 us; 10^3 x 20 8.0
+// against 10.1.  (Loading the next sweep's links before the local update:
+// 5.0 us, and with 512 threads the registers spill.)
+template <int N>
+__global__ __launch_bounds__(N) void k_sweep_slices(const cplx<double> *__restrict__ u0,
+                                                    cplx<double> *__restrict__ g, Extents x,
+                                                    double omega, int hits, int from, int to,
+                                                    int end, unsigned R) {
+    typedef cplx<double> C;
+    __shared__ C sh[2][N * kPlanes];
+    const int ns = x.ns, Vh = x.Vh, S = ns * ns * (ns >> 1), lane = (int)threadIdx.x;
+    const int first = (int)blockIdx.x * S, h = first + lane;
+    const bool on = lane < S;
+    auto copy = [&](bool in) {
+        if (!on) return;
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            mat3<double> m;
+            load_rows01<false>(m, in ? g_field(static_cast<const C *>(g), Vh, p)
+                                     : static_cast<const C *>(sh[p]), in ? h : lane);
+            store_su3<false>(m, in ? sh[p] : g_field(g, Vh, p), in ? lane : h);
+        }
+    };
+    copy(true);
+    __syncthreads();
+    for (int k = from; k < to; k++) {
+        const int p = k & 1;
+        if (on) {
+            const Site s = site_in_block((uint32_t)first, lane, p, x);
+            const Nbr nb = neighbours(s, h, ns);
+            const C *gq = sh[1 - p];
+            AxialDir d[2];
+#pragma unroll
+            for (int i = 1; i < 3; i++) {
+                load_raw<false>(d[i - 1].uf, axial_field(u0, Vh, p, i), u0_tile_bytes<double>(h));
+                load_raw<false>(d[i - 1].ub, axial_field(u0, Vh, 1 - p, i),
+                                u0_tile_bytes<double>(nb.bwd[i]));
+            }
+            mat3<double> W, gf, gb, gn, w, upd, out;
+            m_zero(W);
+            load_rows01<false>(gf, gq, nb.fwd[0] - first);
+            load_rows01<false>(gb, gq, nb.bwd[0] - first);
+            m_fill_row2(gf);
+            m_fill_row2(gb);
+            axial_z<false>(W, u0, s, ns, Vh, p, gf, gb);
+#pragma unroll
+            for (int i = 1; i < 3; i++) {
+                load_raw<false>(d[i - 1].gf, gq, tile_bytes<double>(nb.fwd[i] - first));
+                load_raw<false>(d[i - 1].gb, gq, tile_bytes<double>(nb.bwd[i] - first));
+                axial_dir(W, d[i - 1]);
+            }
+            load_su3<false>(gn, static_cast<const C *>(sh[p]), lane);
+            m_mul(gn, W, w);
+            la_or_update(w, hits, omega, upd);
+            m_mul(upd, gn, out);
+            store_su3<false>(out, sh[p], lane);
+        }
+        __syncthreads();
+        if (k + 1 < end && (unsigned)(k + 1) % R == 0) {
+            if (on) {
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    mat3<double> m;
+                    load_rows01<false>(m, static_cast<const C *>(sh[q]), lane);
+                    project_g(m);
+                    store_su3<false>(m, sh[q], lane);
+                }
+            }
+            __syncthreads();
+        }
+    }
+    copy(false);
 }
 
 // ---------------------------------------------------------------------------

@@ -160,15 +160,15 @@ typedef struct {
                                (one group per stream) stays in 192 MiB of the
                                Infinity Cache between half-sweeps (read with
                                cached loads); a lattice that fits in it whole
-                               is swept as three groups of nt/3 timeslices
-                               when it has at least 2^17 sites per parity,
-                               whole otherwise; single timeslices when a wave
+                               is swept as one, two or three groups, by its
+                               size, in FP64 with ns <= 10 in one launch
+                               between decisions; single timeslices when a wave
                                of them does not fit; -1: whole-lattice
                                sweeps.  With retire_slices, one timeslice per
                                group.                                         */
     int slice_lanes;        /* streams over which the timeslice groups run
-                               concurrently: 1-4, or 0 (default): three for a
-                               lattice that fits the cache whole, two for
+                               concurrently: 1-4, or 0 (default): up to three
+                               for a lattice that fits the cache whole, two for
                                FP64 timeslices too large for a cache-resident
                                wave of four, four otherwise                   */
 } gfc_options;
