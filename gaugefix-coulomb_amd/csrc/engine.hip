@@ -93,7 +93,6 @@ int gfc_ctx_create(int device, gfc_ctx **out) {
     gfc_ctx *c = new gfc_ctx();
     c->device = device;
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipMalloc(&c->res_dev, 4 * sizeof(double));
     if (e == hipSuccess) e = hipHostMalloc(&c->res_host, 8 * sizeof(double), hipHostMallocDefault);
     if (e == hipSuccess) e = hipMalloc(&c->flag_dev, sizeof(int));
     c->lane[0] = c->stream;
@@ -120,7 +119,6 @@ void gfc_ctx_destroy(gfc_ctx *c) {
     hipSetDevice(c->device);
     if (c->stream) hipStreamSynchronize(c->stream);
     hipFree(c->part);
-    hipFree(c->res_dev);
     hipHostFree(c->res_host);
     hipFree(c->flag_dev);
     for (int k = 1; k < gfc_ctx::kLanes; k++)
@@ -397,14 +395,19 @@ extern "C" int gfc_job_reunitarize(gfc_job *j) {
 
 namespace gfcx {
 
-// Reduces the per-block partials of the last observable kernel and returns the
-// three sums on the host.
-int finish_reduction(gfc_ctx *c, unsigned blocks, double out[3]) {
+// Reduces the per-block partials of the last observable kernel into out (device
+// or pinned host memory).
+int reduce_to(gfc_ctx *c, unsigned blocks, double *out) {
     hipLaunchKernelGGL(gfc::k_reduce_final, dim3(1), dim3(kBlock), 0, c->stream, c->part,
-                       (int)blocks, c->res_dev);
+                       (int)blocks, out);
     LAUNCH_CHECK();
-    HIP_TRY(hipMemcpyAsync(c->res_host, c->res_dev, 3 * sizeof(double), hipMemcpyDeviceToHost,
-                           c->stream));
+    return GFC_OK;
+}
+
+// ... and returns the three sums on the host.  The kernel writes them to pinned
+// memory itself: a copy behind it cost another 10 us of launch.
+int finish_reduction(gfc_ctx *c, unsigned blocks, double out[3]) {
+    RC_TRY(reduce_to(c, blocks, c->res_host));
     HIP_TRY(hipStreamSynchronize(c->stream));
     out[0] = c->res_host[0];
     out[1] = c->res_host[1];
@@ -412,25 +415,34 @@ int finish_reduction(gfc_ctx *c, unsigned blocks, double out[3]) {
     return GFC_OK;
 }
 
-// e2, theta, F of the factored state; fp32 selects the FP32 G (MIXED phase 1)
-// and the FP64 u0 in the configuration's own frame.
-int obs_factored(gfc_job *j, bool fp32, double out[3]) {
+// Per-block partials of e2, theta, F of the factored state; fp32 selects the
+// FP32 G (MIXED phase 1) and the FP64 u0 in the configuration's own frame.
+int obs_partials(gfc_job *j, bool fp32) {
     gfc_ctx *c = j->ctx;
     const unsigned b = nblocks(2 * (int64_t)j->Vh);
     if (fp32)
-        hipLaunchKernelGGL((gfc::k_obs_factored<float>), dim3(b), dim3(kBlock), 0,
-                           c->stream, j->u0, j->gf, j->geom.ns, j->Vh, c->part);
+        hipLaunchKernelGGL((gfc::k_obs_factored<float>), dim3(b), dim3(kBlock), 0, c->stream,
+                           j->u0, j->gf, j->geom.ns, j->Vh, c->part);
     else
-        hipLaunchKernelGGL((gfc::k_obs_factored<double>), dim3(b), dim3(kBlock), 0,
-                           c->stream, j->u0, j->g, j->geom.ns, j->Vh, c->part);
+        hipLaunchKernelGGL((gfc::k_obs_factored<double>), dim3(b), dim3(kBlock), 0, c->stream,
+                           j->u0, j->g, j->geom.ns, j->Vh, c->part);
     LAUNCH_CHECK();
-    double s[3];
-    int rc = finish_reduction(c, b, s);
-    if (rc) return rc;
+    return GFC_OK;
+}
+
+// e2, theta, F from their sums over the lattice.
+void obs_means(const gfc_job *j, const double s[3], double out[3]) {
     const double V = (double)j->V;
     out[0] = s[0] / V;
     out[1] = s[1] / (3.0 * V);
     out[2] = s[2] / (9.0 * V);
+}
+
+int obs_factored(gfc_job *j, bool fp32, double out[3]) {
+    RC_TRY(obs_partials(j, fp32));
+    double s[3];
+    RC_TRY(finish_reduction(j->ctx, nblocks(2 * (int64_t)j->Vh), s));
+    obs_means(j, s, out);
     return GFC_OK;
 }
 
@@ -441,12 +453,8 @@ int obs_aos(gfc_job *j, double out[3]) {
                        j->V, c->part);
     LAUNCH_CHECK();
     double s[3];
-    int rc = finish_reduction(c, b, s);
-    if (rc) return rc;
-    const double V = (double)j->V;
-    out[0] = s[0] / V;
-    out[1] = s[1] / (3.0 * V);
-    out[2] = s[2] / (9.0 * V);
+    RC_TRY(finish_reduction(c, b, s));
+    obs_means(j, s, out);
     return GFC_OK;
 }
 
@@ -762,6 +770,39 @@ int promote_g(gfc_job *j, SweepState &st) {
     return GFC_OK;
 }
 
+// The sums behind a per-sweep trace, one triple per half-sweep, kept on the
+// device until the fix ends: a host round trip after every sweep took 25 of the
+// 57 us of a traced sweep at 16^3 x 32.
+struct TraceSums {
+    double *dev = nullptr;
+    int n = 0;
+    ~TraceSums() { hipFree(dev); }
+    int init(int len) {
+        HIP_TRY(hipMalloc(&dev, sizeof(double) * 3 * (size_t)len));
+        return GFC_OK;
+    }
+    // After half-sweep k (1, 2, ...).
+    int add(gfc_job *j, bool fp32, int k) {
+        RC_TRY(obs_partials(j, fp32));
+        RC_TRY(reduce_to(j->ctx, nblocks(2 * (int64_t)j->Vh), dev + 3 * (size_t)(k - 1)));
+        n = k;
+        return GFC_OK;
+    }
+    int finish(gfc_job *j, int which, double *trace) {
+        if (n == 0) return GFC_OK;
+        std::vector<double> s(3 * (size_t)n);
+        HIP_TRY(hipMemcpyAsync(s.data(), dev, sizeof(double) * s.size(), hipMemcpyDeviceToHost,
+                               j->ctx->stream));
+        HIP_TRY(hipStreamSynchronize(j->ctx->stream));
+        for (int k = 0; k < n; k++) {
+            double ob[3];
+            obs_means(j, &s[3 * (size_t)k], ob);
+            trace[k] = ob[which];
+        }
+        return GFC_OK;
+    }
+};
+
 struct SweepTimer {
     bool on = false;
     std::vector<hipEvent_t> ev;
@@ -884,13 +925,7 @@ struct SliceTracker {
     int probe(gfc_job *j, bool fp32, int which, double tol, double *global) {
         gfc_ctx *c = j->ctx;
         const unsigned b = nblocks(2 * (int64_t)j->Vh);
-        if (fp32)
-            hipLaunchKernelGGL((gfc::k_obs_factored<float>), dim3(b), dim3(kBlock), 0,
-                               c->stream, j->u0, j->gf, j->geom.ns, j->Vh, c->part);
-        else
-            hipLaunchKernelGGL((gfc::k_obs_factored<double>), dim3(b), dim3(kBlock), 0,
-                               c->stream, j->u0, j->g, j->geom.ns, j->Vh, c->part);
-        LAUNCH_CHECK();
+        RC_TRY(obs_partials(j, fp32));
         part.resize((size_t)b * 3);
         HIP_TRY(hipMemcpyAsync(part.data(), c->part, sizeof(double) * part.size(),
                                hipMemcpyDeviceToHost, c->stream));
@@ -951,6 +986,11 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
         RC_TRY(sl.init(j));
     }
 
+    TraceSums sums;
+    if (trace && trace_len > 0)
+        RC_TRY(sums.init((int)std::min<unsigned>((unsigned)trace_len,
+                                                 std::max(1u, p->max_sweeps_to_fix))));
+
     RC_TRY(begin_fix(j, j->ctx->stream, st.fp32));
     RC_TRY(obs_factored(j, st.fp32, ob));
     r.residue_evals++;
@@ -1004,10 +1044,7 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
             if (in32) r.sweeps_fp32++;
         }
         timer.after();
-        if (trace && sweep <= trace_len) {
-            RC_TRY(obs_factored(j, st.fp32, ob));
-            trace[sweep - 1] = ob[which];
-        }
+        if (trace && sweep <= trace_len) RC_TRY(sums.add(j, st.fp32, sweep));
         if (((st.fp32 && !ho.at_floor) || sl.on) && sweep != due &&
             sweep % o.mixed_probe_every == 0) {
             double g = 0;
@@ -1060,6 +1097,7 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
     // the max-sweeps and stall exits return before it
     RC_TRY(end_frame(j, j->ctx->stream, sweep, !done));
     RC_TRY(materialize(j, !done));
+    if (trace) RC_TRY(sums.finish(j, which, trace));
     HIP_TRY(hipStreamSynchronize(j->ctx->stream));
     r.seconds_sweeps = timer.seconds();
     r.sweeps = sweep;
@@ -1251,8 +1289,7 @@ extern "C" int gfc_config_observables_noalloc(gfc_ctx *ctx, const gfc_geom *g,
     hipLaunchKernelGGL(gfc::k_reduce_final, dim3(1), dim3(kBlock), 0, s, ptr, (int)b,
                        ptr + kNoallocOut);
     LAUNCH_CHECK();
-    hipLaunchKernelGGL(gfc::k_plaquette_aos, dim3(b), dim3(kBlock), 0, s, cfg, g->ns, g->nt, V,
-                       ptr);
+    hipLaunchKernelGGL(gfc::k_plaquette_aos, dim3(b), dim3(kBlock), 0, s, cfg, g->ns, g->nt, V, ptr);
     LAUNCH_CHECK();
     hipLaunchKernelGGL(gfc::k_reduce_final, dim3(1), dim3(kBlock), 0, s, ptr, (int)b,
                        ptr + kNoallocOut + 3);

@@ -51,7 +51,6 @@ struct gfc_ctx {
     hipStream_t stream = nullptr;
     double *part = nullptr;  // per-block partial sums
     size_t part_cap = 0;     // in blocks
-    double *res_dev = nullptr;
     double *res_host = nullptr;  // pinned, 8 doubles
     int *flag_dev = nullptr;
     // extra streams (default priority) over which independent timeslice
