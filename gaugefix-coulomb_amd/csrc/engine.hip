@@ -315,7 +315,7 @@ extern "C" int gfc_job_create(gfc_ctx *ctx, const gfc_geom *g, int precision, gf
         gfc_job_destroy(j);
         return fail(GFC_ENOMEM, std::string("gfc_job_create: ") + hipGetErrorString(e));
     }
-    int rc = ensure_partials(ctx, nblocks(V));
+    int rc = ensure_partials(ctx, std::max(nblocks(V), gfc::aos_blocks(V)));
     if (rc == GFC_OK) rc = set_identity(j);
     if (rc != GFC_OK) {
         gfc_job_destroy(j);
@@ -448,9 +448,9 @@ int obs_factored(gfc_job *j, bool fp32, double out[3]) {
 
 int obs_aos(gfc_job *j, double out[3]) {
     gfc_ctx *c = j->ctx;
-    const unsigned b = nblocks(j->V);
+    const unsigned b = gfc::aos_blocks(j->V);
     hipLaunchKernelGGL(gfc::k_obs_aos, dim3(b), dim3(kBlock), 0, c->stream, j->cfg, j->geom.ns,
-                       j->V, c->part);
+                       j->V, gfc::aos_groups(j->V), c->part);
     LAUNCH_CHECK();
     double s[3];
     RC_TRY(finish_reduction(c, b, s));
@@ -1139,9 +1139,9 @@ extern "C" int gfc_job_plaquette(gfc_job *j, double *spatial, double *temporal) 
     if (j == nullptr) return fail(GFC_EINVAL, "gfc_job_plaquette: NULL");
     HIP_TRY(hipSetDevice(j->ctx->device));
     gfc_ctx *c = j->ctx;
-    const unsigned b = nblocks(j->V);
+    const unsigned b = gfc::aos_blocks(j->V);
     hipLaunchKernelGGL(gfc::k_plaquette_aos, dim3(b), dim3(kBlock), 0, c->stream, j->cfg,
-                       j->geom.ns, j->geom.nt, j->V, c->part);
+                       j->geom.ns, j->geom.nt, j->V, gfc::aos_groups(j->V), c->part);
     LAUNCH_CHECK();
     double s[3];
     RC_TRY(finish_reduction(c, b, s));
@@ -1272,7 +1272,7 @@ extern "C" int gfc_config_observables_noalloc(gfc_ctx *ctx, const gfc_geom *g,
     if (gfc_geom_check(g))
         return fail(GFC_EGEOMETRY, "gfc_config_observables_noalloc: bad geometry");
     const int64_t V = gfc_geom_volume(g);
-    const unsigned b = nblocks(V);
+    const unsigned b = gfc::aos_blocks(V);
     if (b > (unsigned)kNoallocBlocks)
         return fail(GFC_EINVAL, "gfc_config_observables_noalloc: lattice larger than the "
                                 "scratch allows (at most 11182080 sites)");
@@ -1284,12 +1284,14 @@ extern "C" int gfc_config_observables_noalloc(gfc_ctx *ctx, const gfc_geom *g,
     const cplx<double> *cfg = reinterpret_cast<const cplx<double> *>(U_dev);
     // the same kernels and block decomposition as gfc_job_observables and
     // gfc_job_plaquette, with the partials and sums in the scratch
-    hipLaunchKernelGGL(gfc::k_obs_aos, dim3(b), dim3(kBlock), 0, s, cfg, g->ns, V, ptr);
+    hipLaunchKernelGGL(gfc::k_obs_aos, dim3(b), dim3(kBlock), 0, s, cfg, g->ns, V,
+                       gfc::aos_groups(V), ptr);
     LAUNCH_CHECK();
     hipLaunchKernelGGL(gfc::k_reduce_final, dim3(1), dim3(kBlock), 0, s, ptr, (int)b,
                        ptr + kNoallocOut);
     LAUNCH_CHECK();
-    hipLaunchKernelGGL(gfc::k_plaquette_aos, dim3(b), dim3(kBlock), 0, s, cfg, g->ns, g->nt, V, ptr);
+    hipLaunchKernelGGL(gfc::k_plaquette_aos, dim3(b), dim3(kBlock), 0, s, cfg, g->ns, g->nt, V,
+                       gfc::aos_groups(V), ptr);
     LAUNCH_CHECK();
     hipLaunchKernelGGL(gfc::k_reduce_final, dim3(1), dim3(kBlock), 0, s, ptr, (int)b,
                        ptr + kNoallocOut + 3);

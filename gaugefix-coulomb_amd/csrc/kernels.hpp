@@ -1156,92 +1156,226 @@ __global__ __launch_bounds__(kBlock, 3) void k_obs_factored(const cplx<double> *
     block_reduce3(obs_site<TG>(u0, g, ns, Vh, idx), part, b);
 }
 
-// Observables of an AoS FP64 configuration; one thread per site.
-__global__ __launch_bounds__(kBlock) void k_obs_aos(const cplx<double> *__restrict__ cfg,
-                                                    int ns, int64_t V,
-                                                    double *__restrict__ part) {
-    const int64_t lex = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    Obs o = {0, 0, 0};
-    if (lex < V) {
-        const int x = (int)(lex % ns);
-        int64_t r = lex / ns;
-        const int y = (int)(r % ns);
-        r /= ns;
-        const int z = (int)(r % ns);
-        const int t = (int)(r / ns);
-        mat3<double> D;
-        m_zero(D);
-        double f = 0;
+// The kernels over an AoS configuration.  A thread reading the 144 bytes of a
+// matrix by itself leaves the lanes of a load 144 to 576 bytes apart, a cache
+// line each, and the kernel waits for the address units; so the links of 64
+// sites are brought into LDS in consecutive 16-byte pieces, and four threads
+// work on a site, one per direction.  48^3 x 96: residues 2.15 -> 1.19 ms,
+// plaquettes 4.86 -> 3.3 ms (the configuration's 6.1 GB take 0.98 ms at 6.25
+// TB/s; the plaquettes read 16 links per site, the T neighbours' and part of
+// the Z neighbours' from beyond the L2).
+constexpr int kAosSites = 64;
+
+// Matrix of nine pieces in LDS.
+__device__ __forceinline__ void lds_mat(mat3<double> &m, const double2 *__restrict__ s) {
 #pragma unroll
-        for (int mu = 1; mu <= 3; mu++) {
-            int c[4] = {t, z, y, x};
-            c[mu] = c[mu] == 0 ? ns - 1 : c[mu] - 1;
-            const int64_t lb = (((int64_t)c[0] * ns + c[1]) * ns + c[2]) * ns + c[3];
-            mat3<double> u;
-            const cplx<double> *pf = cfg + (lex * 4 + mu) * 9;
+    for (int k = 0; k < 9; k++) m.e[k] = c_make<double>(s[k].x, s[k].y);
+}
+
+// The value of the lane whose number differs in the bits X (1 to 3).
+template <int X>
+__device__ __forceinline__ double quad_xor(double v) {
+    constexpr int ctrl = X == 1 ? 0xB1 : X == 2 ? 0x4E : 0x1B;  // quad_perm
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, ctrl, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), ctrl, 0xf, 0xf, true);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
+                                            (unsigned)lo));
+}
+
+// tile[k] = src[at(k)] for the P pieces of each of kAosSites sites, moved
+// straight to LDS, 64 pieces by a wave's load, all of them in flight together
+// (through registers, a piece at a time, they arrived one after the other:
+// 4.6 ms for the plaquettes).  Pieces from n on, of sites past the end, get
+// src[at(0)].  Complete on return; the tile must have been read before.
+template <int P, typename At>
+__device__ __forceinline__ void stage_tile(double2 *tile, const double2 *src, int n, At at) {
+    typedef __attribute__((address_space(3))) void *lds_ptr;
+    typedef const __attribute__((address_space(1))) void *global_ptr;
+    static_assert(kAosSites == 64, "P chunks of 64 pieces");
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
 #pragma unroll
-            for (int k = 0; k < 9; k++) u.e[k] = pf[k];
-            accum_link(D, u, 1.0);
-            f += u.e[0].re + u.e[4].re + u.e[8].re;
-            const cplx<double> *pb = cfg + (lb * 4 + mu) * 9;
-#pragma unroll
-            for (int k = 0; k < 9; k++) u.e[k] = pb[k];
-            accum_link(D, u, -1.0);
-        }
-        o = site_obs(D, f);
+    for (int j = 0; j < (P + 3) / 4; j++) {
+        const int c = wave + 4 * j, k = c * 64 + ((int)threadIdx.x & 63);
+        if (c < P)
+            __builtin_amdgcn_global_load_lds((global_ptr)(src + at(k < n ? k : 0)),
+                                             (lds_ptr)(tile + c * 64), 16, 0, 0);
     }
-    block_reduce3(o, part, blockIdx.x);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
+// Groups of kAosSites sites a workgroup takes: four, so that its partial sums
+// are those of kBlock sites, or for a small lattice, whose workgroups do not
+// fill the GPU, one.
+inline int aos_groups(int64_t V) { return V <= 1024 * kBlock ? 1 : kBlock / kAosSites; }
+inline unsigned aos_blocks(int64_t V) {
+    const int64_t sites = (int64_t)aos_groups(V) * kAosSites;
+    return (unsigned)((V + sites - 1) / sites);
+}
+
+// First site of the q-th of workgroup b's groups: runs of 64 workgroups (one
+// XCD's, xcd_order) go through their groups side by side, 4096 consecutive
+// sites at a time, so that a site's Y and Z neighbours are read by the same XCD
+// at about the same time.
+__device__ __forceinline__ int aos_group(unsigned b, unsigned nb, int q, int groups) {
+    const unsigned run = b / 64, m = min(64u, nb - run * 64);
+    return (int)(run * 64 * (unsigned)groups + (unsigned)q * m + b % 64) * kAosSites;
+}
+
+// lex index of the site one step from lex in direction mu, forward or backward.
+__device__ __forceinline__ int aos_neighbour(int lex, int mu, bool fwd, int ns, int nt) {
+    int c[4];  // t, z, y, x
+    c[3] = lex % ns;
+    int r = lex / ns;
+    c[2] = r % ns;
+    r /= ns;
+    c[1] = r % ns;
+    c[0] = r / ns;
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        if (k == mu) {
+            const int n = k == 0 ? nt : ns;
+            c[k] = fwd ? (c[k] + 1 == n ? 0 : c[k] + 1) : (c[k] == 0 ? n - 1 : c[k] - 1);
+        }
+    return ((c[0] * ns + c[1]) * ns + c[2]) * ns + c[3];
+}
+
+// Observables of an AoS FP64 configuration.  Thread i (1 to 3) of a site adds
+// its direction's U_i(n) - U_i(n-i); thread 0 takes the sum.
+__global__ __launch_bounds__(kBlock) void k_obs_aos(const cplx<double> *__restrict__ cfg, int ns,
+                                                    int64_t V, int groups,
+                                                    double *__restrict__ part) {
+    __shared__ double2 tile[kAosSites * 27];
+    __shared__ int nbr[kAosSites * 3];
+    const double2 *src = reinterpret_cast<const double2 *>(cfg);
+    const unsigned b = xcd_order(blockIdx.x, gridDim.x);
+    const int site = threadIdx.x >> 2, i = threadIdx.x & 3, n = (int)V;
+    Obs o = {0, 0, 0};
+#pragma unroll 1
+    for (int q = 0; q < groups; q++) {
+        const int lex0 = aos_group(b, gridDim.x, q, groups), count = min(kAosSites, n - lex0);
+        if (count <= 0) break;
+        const bool on = i > 0 && site < count;
+        const double2 *mine = tile + site * 27 + (i - 1) * 9;
+        mat3<double> u, v;
+        if (on) nbr[site * 3 + i - 1] = aos_neighbour(lex0 + site, i, false, ns, 1 << 30);
+        stage_tile<27>(tile, src, count * 27,
+                       [&](int k) { return (int64_t)lex0 * 36 + 9 + k + k / 27 * 9; });
+        if (on) lds_mat(u, mine);
+        __syncthreads();
+        stage_tile<27>(tile, src, count * 27,
+                       [&](int k) { return (int64_t)nbr[k / 9] * 36 + 9 + k % 27; });
+        // D = sum_i (E_i - E_i^dagger), E_i = U_i(n) - U_i(n-i): the imaginary
+        // parts of its diagonal, D01, D02, D12, and Re Tr U
+        double d[10];
+#pragma unroll
+        for (int k = 0; k < 10; k++) d[k] = 0;
+        if (on) {
+            lds_mat(v, mine);
+            d[9] = u.e[0].re + u.e[4].re + u.e[8].re;
+#pragma unroll
+            for (int k = 0; k < 9; k++)
+                u.e[k] = c_make<double>(u.e[k].re - v.e[k].re, u.e[k].im - v.e[k].im);
+            d[0] = 2 * u.e[0].im;
+            d[1] = 2 * u.e[4].im;
+            d[2] = 2 * u.e[8].im;
+            d[3] = u.e[1].re - u.e[3].re;
+            d[4] = u.e[1].im + u.e[3].im;
+            d[5] = u.e[2].re - u.e[6].re;
+            d[6] = u.e[2].im + u.e[6].im;
+            d[7] = u.e[5].re - u.e[7].re;
+            d[8] = u.e[5].im + u.e[7].im;
+        }
+#pragma unroll
+        for (int k = 0; k < 10; k++) d[k] += quad_xor<1>(d[k]);
+#pragma unroll
+        for (int k = 0; k < 10; k++) d[k] += quad_xor<2>(d[k]);
+        if (i == 0 && site < count) {
+            mat3<double> D;
+            D.e[0] = c_make<double>(0, d[0]);
+            D.e[4] = c_make<double>(0, d[1]);
+            D.e[8] = c_make<double>(0, d[2]);
+            D.e[1] = c_make<double>(d[3], d[4]);
+            D.e[3] = c_make<double>(-d[3], d[4]);
+            D.e[2] = c_make<double>(d[5], d[6]);
+            D.e[6] = c_make<double>(-d[5], d[6]);
+            D.e[5] = c_make<double>(d[7], d[8]);
+            D.e[7] = c_make<double>(-d[7], d[8]);
+            const Obs s = site_obs(D, d[9]);
+            o.e2 += s.e2;
+            o.theta += s.theta;
+            o.f += s.f;
+        }
+        __syncthreads();
+    }
+    block_reduce3(o, part, b);
+}
+
+// Re Tr of the plaquette in the plane of directions r (this thread) and
+// d = r ^ X (the thread X lanes over): a = U_d(n) U_r(n+d) here and
+// U_r(n) U_d(n+r) there, Re Tr(a_here a_there^dagger).
+template <int X>
+__device__ __forceinline__ double plaquette_trace(const mat3<double> &a) {
+    double tr = 0;
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        tr = __builtin_fma(a.e[k].re, quad_xor<X>(a.e[k].re), tr);
+        tr = __builtin_fma(a.e[k].im, quad_xor<X>(a.e[k].im), tr);
+    }
+    return tr;
 }
 
 // Plaquettes of an AoS FP64 configuration (TrPlaquette, src/measurement.c:38-84):
 // Re Tr[U_mu(n) U_nu(n+mu) U_mu(n+nu)^dag U_nu(n)^dag] / 3, spatial planes
 // (XY, XZ, YZ) into slot 0 and temporal planes (TZ, TY, TX) into slot 1.
+// Thread r of a site meets each other direction d = r ^ X once, X = 1, 2, 3;
+// both threads of a plane find its trace, and each counts half.
 __global__ __launch_bounds__(kBlock) void k_plaquette_aos(const cplx<double> *__restrict__ cfg,
-                                                          int ns, int nt, int64_t V,
+                                                          int ns, int nt, int64_t V, int groups,
                                                           double *__restrict__ part) {
-    const int64_t lex = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    __shared__ double2 tile[kAosSites * 36];
+    __shared__ int nbr[kAosSites * 4];
+    const double2 *src = reinterpret_cast<const double2 *>(cfg);
+    const unsigned b = xcd_order(blockIdx.x, gridDim.x);
+    const int site = threadIdx.x >> 2, r = threadIdx.x & 3, n = (int)V;
     Obs o = {0, 0, 0};
-    if (lex < V) {
-        const int x = (int)(lex % ns);
-        int64_t r = lex / ns;
-        const int y = (int)(r % ns);
-        r /= ns;
-        const int z = (int)(r % ns);
-        const int t = (int)(r / ns);
-        const int planes[6][2] = {{3, 2}, {3, 1}, {2, 1}, {0, 1}, {0, 2}, {0, 3}};
+#pragma unroll 1
+    for (int q = 0; q < groups; q++) {
+        const int lex0 = aos_group(b, gridDim.x, q, groups), count = min(kAosSites, n - lex0);
+        if (count <= 0) break;
+        if (site < count) nbr[threadIdx.x] = aos_neighbour(lex0 + site, r, true, ns, nt);
+        stage_tile<36>(tile, src, count * 36, [&](int k) { return (int64_t)lex0 * 36 + k; });
+        mat3<double> own;  // U_r(n)
+        m_zero(own);
+        if (site < count) lds_mat(own, tile + threadIdx.x * 9);
 #pragma unroll
-        for (int q = 0; q < 6; q++) {
-            const int mu = planes[q][0], nu = planes[q][1];
-            int cm[4] = {t, z, y, x}, cn[4] = {t, z, y, x};
-            cm[mu] += 1;
-            if (cm[mu] == (mu == 0 ? nt : ns)) cm[mu] = 0;
-            cn[nu] += 1;
-            if (cn[nu] == (nu == 0 ? nt : ns)) cn[nu] = 0;
-            const int64_t lm = (((int64_t)cm[0] * ns + cm[1]) * ns + cm[2]) * ns + cm[3];
-            const int64_t ln = (((int64_t)cn[0] * ns + cn[1]) * ns + cn[2]) * ns + cn[3];
-            mat3<double> a, b, c, d, ab, abc;
-            const cplx<double> *pa = cfg + (lex * 4 + mu) * 9, *pb = cfg + (lm * 4 + nu) * 9;
-            const cplx<double> *pc = cfg + (ln * 4 + mu) * 9, *pd = cfg + (lex * 4 + nu) * 9;
+        for (int X = 1; X < 4; X++) {
+            __syncthreads();  // the tile has been read
+            stage_tile<36>(tile, src, count * 36,
+                           [&](int k) { return (int64_t)nbr[(k / 9) ^ X] * 36 + k % 36; });
+            mat3<double> u, v, a;
 #pragma unroll
-            for (int k = 0; k < 9; k++) {
-                a.e[k] = pa[k];
-                b.e[k] = pb[k];
-                c.e[k] = pc[k];
-                d.e[k] = pd[k];
-            }
-            m_mul(a, b, ab);
-            m_mul_nd(ab, c, abc);
-            // Re Tr(abc d^dag) = sum_ij Re(abc_ij conj(d_ij))
-            double tr = 0;
-#pragma unroll
-            for (int k = 0; k < 9; k++) tr += abc.e[k].re * d.e[k].re + abc.e[k].im * d.e[k].im;
-            if (q < 3)
-                o.e2 += tr / 3.0;
+            for (int k = 0; k < 9; k++)
+                u.e[k] = X == 1   ? c_make<double>(quad_xor<1>(own.e[k].re), quad_xor<1>(own.e[k].im))
+                         : X == 2 ? c_make<double>(quad_xor<2>(own.e[k].re), quad_xor<2>(own.e[k].im))
+                                  : c_make<double>(quad_xor<3>(own.e[k].re), quad_xor<3>(own.e[k].im));
+            m_zero(v);
+            if (site < count) lds_mat(v, tile + threadIdx.x * 9);
+            m_mul(u, v, a);
+            double tr = (X == 1   ? plaquette_trace<1>(a)
+                         : X == 2 ? plaquette_trace<2>(a)
+                                  : plaquette_trace<3>(a)) / 6.0;
+            // formed here: the compiler would keep the three products for later
+            asm volatile("" : "+v"(tr));
+            if (r == 0 || (r ^ X) == 0)
+                o.theta += tr;
             else
-                o.theta += tr / 3.0;
+                o.e2 += tr;
         }
+        __syncthreads();
     }
-    block_reduce3(o, part, blockIdx.x);
+    block_reduce3(o, part, b);
 }
 
 // Streaming copy of n 16-byte elements (bandwidth probe / counter calibration).
