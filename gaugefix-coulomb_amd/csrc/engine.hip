@@ -523,12 +523,11 @@ struct SweepState {
     bool fp32 = false;
 };
 
-// Bytes of one timeslice as the cache-budget policy counts them: u0 (3 links)
-// and G at six complex numbers each (an FP64 u0 link reads five; the policy
-// below was measured with this count).
+// Bytes of one timeslice that its sweeps touch: in FP64 two links of five
+// complex numbers and G of six, in FP32 three links and G of six.
 int64_t slice_bytes(const gfc_job *j, bool fp32) {
     const int64_t S = (int64_t)j->geom.ns * j->geom.ns * j->geom.ns;
-    return S * 4 * 6 * (fp32 ? 8 : 16);
+    return S * (fp32 ? 24 * 8 : 16 * 16);
 }
 
 // Part of the 256 MiB Infinity Cache that the data of concurrent sweep
@@ -564,16 +563,20 @@ constexpr int kOneGroup = 256 * kBlock;
 //   17.2 / 16.0; in FP32 7.2 / 8.6 / 9.5, 10.4 / 9.6 / 9.9, 15.0 / 13.1 / 11.4).
 //   One group is a launch per half-sweep, as in whole-lattice sweeps, but with
 //   the reunitarizations folded in (16^3 x 32: 10.8 -> 8.1 us with R = 10);
-// * two for FP64 single timeslices too large for a cache-resident wave
-//   (64^3 x 128: 6% faster than four);
-// * four otherwise.
+// * in FP64, three if two timeslices each fit in the cache together, else two
+//   (groups x streams, us per half-sweep: 48^3 x 96 2 x 3 463, 3 x 2 469, 2 x 2
+//   and 1 x 4 475, 1 x 3 508; 40^3 x 80 4 x 3 225, 4 x 2 223, 3 x 4 232;
+//   32^3 x 64 8 x 3 91.2, 6 x 4 93.4; 56^3 x 112 2 x 2 872, 1 x 4 882, 1 x 2
+//   970; 64^3 x 128 1 x 2 1474, 1 x 3 1495, 1 x 4 1725; 72^3 x 72 1 x 2 1217,
+//   1 x 4 1475);
+// * four in FP32.
 int lane_count(const gfc_job *j, const gfc_options &o, bool fp32) {
     if (o.slice_lanes >= 1 && o.slice_lanes <= gfc_ctx::kLanes) return o.slice_lanes;
     if (o.slice_group != 0) return gfc_ctx::kLanes;
     const int64_t ts = slice_bytes(j, fp32);
     if ((int64_t)j->geom.nt * ts <= kCacheBytes)
         return j->Vh >= kSplitMinSites ? 3 : j->Vh > kOneGroup ? 2 : 1;
-    if (!fp32 && gfc_ctx::kLanes * ts > kCacheBytes) return 2;
+    if (!fp32) return 6 * ts <= kCacheBytes ? 3 : 2;
     return gfc_ctx::kLanes;
 }
 
@@ -640,11 +643,9 @@ int reunit_g(gfc_job *j, hipStream_t s, bool fp32, int p0, int np) {
 // * a lattice whose u0 and G fit in kCacheBytes: nt / L timeslices per group;
 //   from the cache;
 // * otherwise, if a wave of L single timeslices fits, the largest groups whose
-//   wave fits, evened out so that every wave fills all streams (64^3 x 128 in
-//   FP64: single timeslices on two streams, from the cache);
+//   wave fits, evened out so that every wave fills all streams;
 // * otherwise single timeslices with non-temporal loads (a timeslice is then
-//   large enough that a launch still fills the GPU; single timeslices on four
-//   streams were 8-10% faster than groups of 8 timeslices at 64^3 x 128).
+//   large enough that a launch still fills the GPU).
 int group_size(const gfc_job *j, const gfc_options &o, bool fp32) {
     if (o.slice_group < 0) return 0;
     const int nt = j->geom.nt;

@@ -61,7 +61,7 @@ enum State { QUEUED, INIT, RUN, DONE };
 
 constexpr int kLanes = gfc_ctx::kLanes;
 
-// A lane whose runners' u0 and G (192 B per site in FP32, 384 B in FP64) fit
+// A lane whose runners' u0 and G (192 B per site in FP32, 256 B in FP64) fit
 // in this share of the 256 MiB Infinity Cache sweeps with cached loads, so
 // that its data stays in the cache from one half-sweep to the next; larger
 // lanes stream with non-temporal loads.
@@ -423,7 +423,7 @@ int plan_and_run(gfc_server *s, Lane &L) {
     }
     if (run.empty()) return GFC_OK;
     int64_t bytes = 0;
-    for (Req *r : run) bytes += r->job->V * (r->fp32 ? 192 : 384);
+    for (Req *r : run) bytes += r->job->V * (r->fp32 ? 192 : 256);
     const bool cached = bytes <= kLaneCacheBytes;
     // plan signature: load policy, then (slot, job, fp32, steps, parity) of
     // every runner

@@ -168,9 +168,9 @@ typedef struct {
                                group.                                         */
     int slice_lanes;        /* streams over which the timeslice groups run
                                concurrently: 1-4, or 0 (default): up to three
-                               for a lattice that fits the cache whole, two for
-                               FP64 timeslices too large for a cache-resident
-                               wave of four, four otherwise                   */
+                               for a lattice that fits the cache whole, two or
+                               three in FP64, by the size of a timeslice, four
+                               in FP32 otherwise                              */
 } gfc_options;
 
 typedef struct {
