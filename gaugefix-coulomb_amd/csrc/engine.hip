@@ -858,8 +858,9 @@ struct SliceTracker {
     int n_items[2] = {0, 0};
     bool dirty = true;
     bool desc_fp32 = false;
-    std::vector<double> part;
+    double *sums = nullptr;  // pinned: the three sums of every timeslice
     ~SliceTracker() {
+        hipHostFree(sums);
         hipFree(d_job);
         hipFree(d_items[0]);
         hipFree(d_items[1]);
@@ -870,6 +871,7 @@ struct SliceTracker {
         S = j->geom.ns * j->geom.ns * j->geom.ns / 2;
         active.assign(nt, 1);
         n_active = nt;
+        HIP_TRY(hipHostMalloc(&sums, sizeof(double) * 3 * (size_t)nt, hipHostMallocDefault));
         HIP_TRY(hipMalloc(&d_job, sizeof(gfc::BatchJob)));
         for (int p = 0; p < 2; p++)
             HIP_TRY(hipMalloc(&d_items[p], sizeof(int4) * (size_t)(j->Vh / kBlock + 1)));
@@ -925,20 +927,15 @@ struct SliceTracker {
     // tol.  Returns the global proxy (mean over slices) in *global.
     int probe(gfc_job *j, bool fp32, int which, double tol, double *global) {
         gfc_ctx *c = j->ctx;
-        const unsigned b = nblocks(2 * (int64_t)j->Vh);
         RC_TRY(obs_partials(j, fp32));
-        part.resize((size_t)b * 3);
-        HIP_TRY(hipMemcpyAsync(part.data(), c->part, sizeof(double) * part.size(),
-                               hipMemcpyDeviceToHost, c->stream));
+        hipLaunchKernelGGL(gfc::k_slice_sums, dim3(nt), dim3(kBlock), 0, c->stream, c->part,
+                           j->Vh / kBlock, S / kBlock, sums);
+        LAUNCH_CHECK();
         HIP_TRY(hipStreamSynchronize(c->stream));
-        const int bps = S / kBlock, half = j->Vh / kBlock;
         const double vt = 2.0 * S;  // sites per slice
         double sum = 0;
         for (int t = 0; t < nt; t++) {
-            double acc = 0;
-            for (int q = 0; q < 2; q++)
-                for (int k = 0; k < bps; k++) acc += part[3 * (q * half + t * bps + k) + which];
-            const double pt = acc / (which == 1 ? 3.0 * vt : vt);
+            const double pt = sums[3 * t + which] / (which == 1 ? 3.0 * vt : vt);
             sum += pt;
             if (active[t] && pt <= tol) {
                 active[t] = 0;

@@ -1142,18 +1142,42 @@ __device__ __forceinline__ Obs obs_site(const cplx<double> *__restrict__ u0,
     return o;
 }
 
+// The b-th block of n to be worked on, in the order of the site index: the
+// first and the second half of the blocks, i.e. the two parities of the same
+// sites, in turn.  A link is read as a site's forward link by one parity and as
+// a backward link by the other; in index order the second read came when the
+// first was long out of the caches (us at 48^3 x 96 with an FP32 / FP64 G: 1020
+// / 1240 -> XXX / YYY).
+__host__ __device__ inline unsigned parity_order(unsigned b, unsigned n) {
+    return (b & 1) ? (n + 1) / 2 + b / 2 : b / 2;
+}
+
 // One thread per site, both parities; per-block partial sums in part, in
 // site order.  The workgroups run in XCD-contiguous order (xcd_order), so that
 // the neighbour G and backward u0 links a site reads were mostly brought into
 // its XCD's L2 by the sites next to it.
 template <typename TG>
 __global__ __launch_bounds__(kBlock, 3) void k_obs_factored(const cplx<double> *__restrict__ u0,
-                                                         const cplx<TG> *__restrict__ g,
-                                                         int ns, int Vh,
-                                                         double *__restrict__ part) {
-    const unsigned b = xcd_order(blockIdx.x, gridDim.x);
+                                                            const cplx<TG> *__restrict__ g,
+                                                            int ns, int Vh,
+                                                            double *__restrict__ part) {
+    const unsigned b = parity_order(xcd_order(blockIdx.x, gridDim.x), gridDim.x);
     const int idx = (int)(b * kBlock + threadIdx.x);
     block_reduce3(obs_site<TG>(u0, g, ns, Vh, idx), part, b);
+}
+
+// The sums of each timeslice t (one workgroup), out[3 t + j]: partials
+// t bps + [0, bps) of either parity, which begin at 0 and half.
+__global__ __launch_bounds__(kBlock) void k_slice_sums(const double *__restrict__ part, int half,
+                                                       int bps, double *__restrict__ out) {
+    Obs o = {0, 0, 0};
+    for (int k = threadIdx.x; k < 2 * bps; k += kBlock) {
+        const double *v = part + 3 * ((k < bps ? k : half + k - bps) + (int64_t)blockIdx.x * bps);
+        o.e2 += v[0];
+        o.theta += v[1];
+        o.f += v[2];
+    }
+    block_reduce3(o, out, blockIdx.x);
 }
 
 // The kernels over an AoS configuration.  A thread reading the 144 bytes of a
@@ -1488,7 +1512,7 @@ __global__ __launch_bounds__(kBlock) void k_sweep_batch(const BatchJob *__restri
 __global__ __launch_bounds__(kBlock) void k_obs_batch(const BatchJob *__restrict__ jobs,
                                                       const int4 *__restrict__ items,
                                                       double *__restrict__ part) {
-    const int4 it = items[blockIdx.x];
+    const int4 it = items[xcd_order(blockIdx.x, gridDim.x)];
     const BatchJob J = jobs[it.x];
     const int idx = it.y * kBlock + (int)threadIdx.x;
     const cplx<double> *u0 = static_cast<const cplx<double> *>(J.u0d);

@@ -296,7 +296,9 @@ int evaluate(gfc_server *s, Lane &L, std::vector<Req *> &which) {
         L.h_jobs[r->slot].part_off = (int)k;
         const int nb = (int)nblocks(2 * (int64_t)r->job->Vh);
         const int g32 = r->fp32 ? 1 : 0;
-        for (int b = 0; b < nb; b++) L.h_oitems[k++] = make_int4(r->slot, b, g32, 0);
+        for (int b = 0; b < nb; b++)
+            L.h_oitems[k++] =
+                make_int4(r->slot, (int)gfc::parity_order((unsigned)b, (unsigned)nb), g32, 0);
         L.h_sel[q] = r->slot;
     }
     hipStream_t st = L.st;
