@@ -13,11 +13,11 @@ value        site updates per second of the FP64 drop-in path
 fp64_seconds wall time to e2 < 1e-16, FP64 path
 mixed_*      the FP32 -> FP64 path on the same input and schedule
 roofline     the kernel of the timed fix, k_sweep<double> in cache-resident
-             timeslice waves: the factored update's algorithmic bytes (768 B
-             per site update: the 6 spatial u0 links in five stored complex
-             numbers, G(n) read and written, one neighbour G per update) per lattice
-             half-sweep over the half-sweep's duration measured with HIP
-             events on the job's stream (fork to join of the waves), and the
+             timeslice waves: the factored update's algorithmic bytes (608 B
+             per site update: four spatial u0 links, in the axial frame, in
+             five stored complex numbers, G(n) read and written, one neighbour
+             G per update) per lattice half-sweep over the half-sweep's
+             duration measured with HIP events on the job's stream (fork to join of the waves), and the
              copy-calibrated L2-miss traffic of the same launches from the
              committed rocprofv3 counters (profiles/sweep_fix_48x96_pmc.txt)
 cpu_baseline the reference's OpenMP CPU path (compiled from its sources into
@@ -44,7 +44,7 @@ sys.path.insert(0, os.path.join(ROOT, "gaugefix-coulomb_amd"))
 # queues some of them share a queue, and kernels on one queue run in order: a
 # lone 48^3x96 request then takes 0.92 s instead of 0.72 s.  Eight queues
 # (read when the HIP runtime starts, so set before any HIP call) give each
-# stream its own; the single-lattice fixes use four streams either way.
+# stream its own; a single-lattice fix uses at most four streams either way.
 os.environ.setdefault("GPU_MAX_HW_QUEUES", "8")
 
 # bytes per site update credited to the reference's update: 6 spatial links
@@ -52,11 +52,12 @@ os.environ.setdefault("GPU_MAX_HW_QUEUES", "8")
 # for reference-equivalent rates
 REF_BYTES_PER_UPDATE_FP64 = 2016
 REF_BYTES_PER_UPDATE_FP32 = 1008
-# the factored update's algorithmic bytes in the engine's storage: the 6
-# spatial u0 links (FP64: five complex numbers, 80 B; FP32: two rows, 48 B),
-# G(n) read and written and one neighbour G (two rows: 96 B in FP64, 48 B in
-# FP32; each of the 6 neighbour G read by an update is shared by 6 updates)
-ALG_BYTES_PER_UPDATE_FP64 = 6 * 80 + 96 + 96 + 96
+# the factored update's algorithmic bytes in the engine's storage: the u0 links
+# (FP64: four in the axial frame, of five complex numbers, 80 B; FP32: six, of
+# two rows, 48 B), G(n) read and written and one neighbour G (two rows: 96 B in
+# FP64, 48 B in FP32; each of the 6 neighbour G read by an update is shared by 6
+# updates)
+ALG_BYTES_PER_UPDATE_FP64 = 4 * 80 + 96 + 96 + 96
 ALG_BYTES_PER_UPDATE_FP32 = 6 * 48 + 48 + 48 + 48
 HBM_PEAK_GBS = 8000.0
 # VALU issue peak: 256 CUs x 4 SIMDs, a wave64 FP64 (or unpacked FP32)
@@ -622,8 +623,8 @@ def main():
             "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": round(traffic_upd * vh) if traffic_upd else None,
             "kernel": "k_sweep<double> of the timed fix in its default grouping "
-                      "(48^3x96: 96 single-timeslice launches of 55296 site updates per "
-                      "half-sweep, cache-resident waves on 4 streams)",
+                      "(48^3x96: 48 two-timeslice launches of 110592 site updates per "
+                      "half-sweep, cache-resident waves on 3 streams)",
             "per": f"lattice half-sweep ({vh} site updates)",
             "algorithmic_bytes_per_update": ALG_BYTES_PER_UPDATE_FP64,
             "traffic_bytes_per_update": traffic_upd,

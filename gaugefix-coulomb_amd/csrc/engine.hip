@@ -537,8 +537,8 @@ constexpr int64_t kCacheBytes = 192ll << 20;
 // Whether sweeps over groups of `group` timeslices (0: the whole lattice)
 // read u0 and G(n) with non-temporal loads: unless what the concurrent
 // launches sweep fits in kCacheBytes.  Measured at 48^3 x 96 with groups of
-// 1 (FP64) and 2 (FP32) timeslices on four streams: cached loads make a
-// half-sweep 1% (FP64) and 9% (FP32) faster than the best streamed grouping;
+// 1 (FP64, before its axial frame) and 2 (FP32) timeslices on four streams:
+// cached loads make a half-sweep 1% (FP64) and 9% (FP32) faster than the best streamed grouping;
 // on sets larger than the cache they are 4-5% slower.
 bool stream_loads(const gfc_job *j, bool fp32, int group, int lanes) {
     const int64_t ts = slice_bytes(j, fp32);

@@ -152,7 +152,7 @@ typedef struct {
                                the lattice is cut into groups of slice_group
                                timeslices, and each group runs all those
                                sweeps (with its reunitarizations) on one of
-                               four streams, concurrently with the other
+                               up to four streams, concurrently with the other
                                groups, so that kernel tails overlap.
                                Timeslices do not interact, so the result is
                                bit-identical to whole-lattice sweeps.
