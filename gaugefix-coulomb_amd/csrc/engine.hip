@@ -486,17 +486,26 @@ int begin_fix(gfc_job *j, hipStream_t s, bool mixed) {
 // FP32 -> FP64 hand-off: u0 and G go into the axial frame.
 int promote_g(gfc_job *j, hipStream_t s) {
     RC_TRY(begin_frame(j, s));
-    hipLaunchKernelGGL(gfc::k_g_promote, dim3(nblocks(2 * (int64_t)j->Vh)), dim3(kBlock), 0, s,
-                       j->gf, j->g, j->Vh);
+    hipLaunchKernelGGL(gfc::k_g_promote<true>, dim3(nblocks(2 * (int64_t)j->Vh)), dim3(kBlock), 0,
+                       s, j->gf, j->g, j->Vh);
     LAUNCH_CHECK();
     return GFC_OK;
 }
 
-// G out of the axial frame at the end of a fix of `sweeps` half-sweeps, with
-// its last reunitarization if `project`.  Without a sweep G is the identity
-// (also for a configuration whose residue is no number).
-int end_frame(gfc_job *j, hipStream_t s, int sweeps, bool project) {
+// G at the end of a fix of `sweeps` half-sweeps: out of the axial frame, with
+// its last reunitarization if `project`; if it ended in the FP32 phase, promoted
+// (and so projected) in the configuration's own frame, which that phase keeps
+// (mixed fixes stopped in it, through the axial frame and without: 16^3 x 32
+// after 100 half-sweeps 0.996 and 0.837 ms, 56^3 x 56 after 60 27.1 and 23.7).  Without a sweep G is the identity (also for a configuration whose
+// residue is no number).
+int end_frame(gfc_job *j, hipStream_t s, bool fp32, int sweeps, bool project) {
     if (sweeps == 0) return set_identity(j, s);
+    if (fp32) {
+        hipLaunchKernelGGL(gfc::k_g_promote<false>, dim3(nblocks(2 * (int64_t)j->Vh)),
+                           dim3(kBlock), 0, s, j->gf, j->g, j->Vh);
+        LAUNCH_CHECK();
+        return GFC_OK;
+    }
     const int ns = j->geom.ns, ncol = ns * ns * j->geom.nt;
     hipLaunchKernelGGL(gfc::k_frame_end, dim3((ncol + 63) / 64), dim3(64), 0, s, j->cfg, j->g, ns,
                        j->Vh, ncol, project);
@@ -1088,12 +1097,10 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
         if (!((unsigned)sweep % p->sweeps_to_reunitarization))
             RC_TRY(reunit_g(j, st.fp32, 0, 2));
     }
-    // left the loop in the FP32 phase (tolerance reached there or max sweeps):
-    // hand the state over so that G and U are FP64
-    if (st.fp32 && sweep > 0) RC_TRY(promote_g(j, st));
     // converged: the final reunitarization of G and U (src/gauge_fixing.c:822-823);
-    // the max-sweeps and stall exits return before it
-    RC_TRY(end_frame(j, j->ctx->stream, sweep, !done));
+    // the max-sweeps and stall exits return before it.  The loop may be left in
+    // the FP32 phase (tolerance reached there or max sweeps).
+    RC_TRY(end_frame(j, j->ctx->stream, st.fp32, sweep, !done));
     RC_TRY(materialize(j, !done));
     if (trace) RC_TRY(sums.finish(j, which, trace));
     HIP_TRY(hipStreamSynchronize(j->ctx->stream));

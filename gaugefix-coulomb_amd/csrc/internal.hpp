@@ -92,7 +92,7 @@ namespace gfcx {
 int set_identity(gfc_job *j);
 int set_identity(gfc_job *j, hipStream_t s);
 int begin_fix(gfc_job *j, hipStream_t s, bool mixed);
-int end_frame(gfc_job *j, hipStream_t s, int sweeps, bool project);
+int end_frame(gfc_job *j, hipStream_t s, bool fp32, int sweeps, bool project);
 int materialize(gfc_job *j, bool project);
 int materialize(gfc_job *j, hipStream_t s, bool project);
 int reunit_g(gfc_job *j, bool fp32, int p0, int np);

@@ -728,8 +728,9 @@ __global__ __launch_bounds__(kBlock) void k_g_reunit(cplx<T> *__restrict__ g, in
 }
 
 // FP32 -> FP64 hand-off of G: rows 0, 1 of the FP32 G promoted and projected
-// in FP64, then taken into the axial frame, where g holds h^dagger
+// in FP64, then, with FRAME, taken into the axial frame, where g holds h^dagger
 // (k_frame_begin).
+template <bool FRAME>
 __global__ __launch_bounds__(kBlock) void k_g_promote(const cplx<float> *__restrict__ gf,
                                                       cplx<double> *__restrict__ g, int Vh) {
     const int idx = blockIdx.x * kBlock + threadIdx.x;
@@ -744,8 +745,12 @@ __global__ __launch_bounds__(kBlock) void k_g_promote(const cplx<float> *__restr
         m.e[k] = c_make<double>(v.re, v.im);
     }
     m_project_su3(m);
-    load_su3<false>(hd, g_field(static_cast<const cplx<double> *>(g), Vh, p), h);
-    m_mul(m, hd, out);
+    if (FRAME) {
+        load_su3<false>(hd, g_field(static_cast<const cplx<double> *>(g), Vh, p), h);
+        m_mul(m, hd, out);
+    } else {
+        out = m;
+    }
     store_su3<false>(out, g_field(g, Vh, p), h);
 }
 

@@ -329,19 +329,24 @@ int evaluate(gfc_server *s, Lane &L, std::vector<Req *> &which) {
     return GFC_OK;
 }
 
-int promote(Lane &L, Req &r) {
-    RC_TRY(gfcx::promote_g(r.job, L.st));
+// r's G is in FP64 from here on.
+void in_fp64(Lane &L, Req &r) {
     r.fp32 = false;
     fill_desc(L, r);
     L.plan_sig.clear();
+}
+
+int promote(Lane &L, Req &r) {
+    RC_TRY(gfcx::promote_g(r.job, L.st));
+    in_fp64(L, r);
     return GFC_OK;
 }
 
 // End of gaugefixOverrelaxation for r: hand-off, final reunitarization (unless
 // it stopped on max sweeps or a stalled residue), U = G U0 G^dagger.
 int finish(Lane &L, Req &r, int rc) {
-    if (r.fp32 && r.sweep > 0) RC_TRY(promote(L, r));
-    RC_TRY(gfcx::end_frame(r.job, L.st, r.sweep, rc >= 0));
+    RC_TRY(gfcx::end_frame(r.job, L.st, r.fp32, r.sweep, rc >= 0));
+    if (r.fp32 && r.sweep > 0) in_fp64(L, r);
     RC_TRY(gfcx::materialize(r.job, L.st, rc >= 0));
     r.rc = rc >= 0 ? r.sweep : rc;
     r.state = DONE;

@@ -57,3 +57,34 @@ def test_no_sweep_leaves_identity(ctx, precision):
             rc, rep = job.fix(gfc.Params(tolerance=tol), o)
             assert rc == 0 and rep.sweeps == 0
             assert np.array_equal(job.download_gauge(), one)
+
+
+@pytest.mark.parametrize("ns,nt", [(2, 2), (6, 4), (18, 2)])
+def test_mixed_stopped_in_fp32(ctx, ns, nt):
+    """A mixed fix that ends in its FP32 phase never enters the axial frame: G is
+    the FP32 G projected in FP64 (SU(3), and U = G U0 G^dagger, to 1e-13) and
+    within 20 sweeps of some 50 FP32 roundings each, 6e-8 * 1000, of the FP64 G."""
+    geom = gfc.Geometry(ns, nt)
+    U0 = gfc.generate_smooth(geom, 5, 0.3)
+    p = gfc.Params(tolerance=1e-300, estimate_sweeps_to_gf_progress=100000000,
+                   max_sweeps_to_fix=20)
+    out = {}
+    for prec in (gfc.PREC_FP64, gfc.PREC_MIXED):
+        with gfc.Job(ctx, geom, precision=prec) as job:
+            job.upload_config(U0)
+            assert job.reunitarize() == 0
+            rc, rep = job.fix(p, gfc.Options(precision=prec))[:2]
+            assert rc == gfc.ENOTCONVERGED and rep.sweeps == 20
+            out[prec] = job.download_gauge(), job.download_config()
+    assert rep.sweeps_fp32 == 20
+    G, U = out[gfc.PREC_MIXED]
+    Gt, Ut = G.reshape(nt, ns, ns, ns, 3, 3), U.reshape(nt, ns, ns, ns, 4, 3, 3)
+    dag = lambda m: np.conj(np.swapaxes(m, -1, -2))  # noqa: E731
+    assert np.abs(G @ dag(G) - np.eye(3)).max() < 1e-13
+    V0 = U0.copy()
+    orc.reunitarize(V0)
+    V0 = V0.reshape(Ut.shape)
+    for mu in range(4):
+        assert np.abs(Ut[..., mu, :, :] - Gt @ V0[..., mu, :, :]
+                      @ dag(np.roll(Gt, -1, axis=mu))).max() < 1e-13
+    assert np.abs(G - out[gfc.PREC_FP64][0]).max() < 1000 * 6e-8
