@@ -595,10 +595,10 @@ void launch_sweep_pin(const cplx<T> *u0, cplx<T> *g, hipStream_t s, const gfc::E
     const unsigned b = nblocks(count);
     if (pin)
         hipLaunchKernelGGL((gfc::k_sweep<T, POUT, STREAM, true>), dim3(b), dim3(kBlock), 0, s,
-                           u0, g, x, p, omega, hits, h0, count);
+                           u0, g, p, omega, hits, h0, count, x);
     else
         hipLaunchKernelGGL((gfc::k_sweep<T, POUT, STREAM, false>), dim3(b), dim3(kBlock), 0, s,
-                           u0, g, x, p, omega, hits, h0, count);
+                           u0, g, p, omega, hits, h0, count, x);
 }
 
 // A half-sweep launch: pout projects the swept parity's new G on output, pin
