@@ -134,7 +134,7 @@ char *slot(gfc_ctx *c, int k) { return c->ring + (size_t)k * kSlot; }
 
 // The ring of the context, allocated on first use, with no copy of an earlier
 // call still running in it.  The caller holds c->pin_mu.
-int ring(gfc_ctx *c) {
+int make_ring(gfc_ctx *c) {
     if (c->ring == nullptr) {
         void *p = nullptr;
         HIP_TRY(hipHostMalloc(&p, kSlots * kSlot, hipHostMallocDefault));
@@ -145,6 +145,17 @@ int ring(gfc_ctx *c) {
         HIP_TRY(hipEventSynchronize(e));
     }
     return GFC_OK;
+}
+
+// Whether the context has its ring.  When it cannot have one the caller takes
+// another way, so the failed request must not be reported by the next launch
+// check (HIP keeps an error until it is read) nor by gfc_last_error.
+bool ring(gfc_ctx *c) {
+    const std::string message = gfcx::last_error;
+    if (make_ring(c) == GFC_OK) return true;
+    (void)hipGetLastError();
+    gfcx::last_error = message;
+    return false;
 }
 
 // Host threads that take the pieces of a transfer in turn and copy each once
@@ -242,7 +253,7 @@ int stream_out(gfc_ctx *c, int fd, const char *src, size_t total) {
 // copy_to_host and copy_from_host through the ring; > 0 if it is not to be had.
 int ring_to_host(gfc_ctx *c, hipStream_t s, char *dst, const char *src, size_t total) {
     std::lock_guard<std::mutex> lk(c->pin_mu);
-    if (ring(c) != GFC_OK) return 1;
+    if (!ring(c)) return 1;
     const size_t nb = (total + kSlot - 1) / kSlot;
     Copiers cp(nb);
     if (!cp.start(total, [=](size_t b, size_t off, size_t n) {
@@ -267,7 +278,7 @@ int ring_to_host(gfc_ctx *c, hipStream_t s, char *dst, const char *src, size_t t
 
 int ring_from_host(gfc_ctx *c, hipStream_t s, char *dst, const char *src, size_t total) {
     std::lock_guard<std::mutex> lk(c->pin_mu);
-    if (ring(c) != GFC_OK) return 1;
+    if (!ring(c)) return 1;
     const size_t nb = (total + kSlot - 1) / kSlot;
     Copiers cp(nb);
     cp.open.store(kSlots, std::memory_order_relaxed);  // every slot is free

@@ -1,0 +1,177 @@
+// The engine's host side without a GPU, for tests/test_host_engine.py: this
+// program defines the HIP calls that libgfc.so makes (its definitions come
+// before libamdhip64's), with device memory in host memory and kernels that do
+// nothing, so that error paths and launch decisions can be seen on the CPU.
+//
+// As in ROCm 7, an error stays the thread's last error until hipGetLastError
+// reads it, whatever succeeds in between.
+//
+// Usage: fake_hip_driver <scenario> [numbers]; see main.
+#include <hip/hip_runtime_api.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <string>
+#include <vector>
+
+#include "gfc.h"
+
+namespace {
+struct Fake {
+    std::mutex mu;
+    std::map<const void *, std::string> kernels;
+    std::vector<std::string> log;
+    size_t most_pinned = ~(size_t)0;  // larger hipHostMalloc requests fail
+    double sums = 1e3;                // what a reduction finds
+};
+Fake &fake() {
+    static Fake f;
+    return f;
+}
+thread_local hipError_t last = hipSuccess;
+thread_local dim3 cfg_grid, cfg_block;
+
+hipError_t err(hipError_t e) {
+    last = e;
+    return e;
+}
+void note(const std::string &s) {
+    std::lock_guard<std::mutex> lk(fake().mu);
+    fake().log.push_back(s);
+}
+hipError_t alloc(void **p, size_t n) {
+    *p = std::calloc(n ? n : 1, 1);
+    return *p ? hipSuccess : err(hipErrorOutOfMemory);
+}
+}  // namespace
+
+extern "C" {
+void **__hipRegisterFatBinary(const void *) {
+    static void *module;
+    return &module;
+}
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, void *,
+                           void *, void *, void *, int *) {
+    fake().kernels[f] = name;
+}
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t, hipStream_t) {
+    cfg_grid = g;
+    cfg_block = b;
+    return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *shared, hipStream_t *s) {
+    *g = cfg_grid;
+    *b = cfg_block;
+    *shared = 0;
+    *s = nullptr;
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t, hipStream_t) {
+    const std::string &name = fake().kernels[f];
+    note("launch " + name + " " + std::to_string(g.x) + " " + std::to_string(b.x));
+    if (name.find("k_reduce_final") != std::string::npos) {
+        double *out = *static_cast<double **>(args[2]);
+        for (int k = 0; k < 3; k++) out[k] = fake().sums;
+    }
+    return hipSuccess;
+}
+const char *hipGetErrorString(hipError_t e) {
+    return e == hipSuccess ? "no error" : e == hipErrorOutOfMemory ? "out of memory" : "error";
+}
+hipError_t hipGetLastError(void) {
+    const hipError_t e = last;
+    last = hipSuccess;
+    return e;
+}
+hipError_t hipGetDeviceCount(int *n) {
+    *n = 1;
+    return hipSuccess;
+}
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipMemGetInfo(size_t *f, size_t *t) {
+    *f = *t = (size_t)1 << 34;
+    return hipSuccess;
+}
+hipError_t hipGetSymbolAddress(void **p, const void *) { return alloc(p, 2u << 20); }
+hipError_t hipMalloc(void **p, size_t n) { return alloc(p, n); }
+hipError_t hipFree(void *p) {
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+    if (n > fake().most_pinned) return err(hipErrorOutOfMemory);
+    return alloc(p, n);
+}
+hipError_t hipHostFree(void *p) { return hipFree(p); }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {
+    note("copy " + std::to_string(n));
+    std::memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) {
+    std::memset(d, v, n);
+    return hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
+    *s = reinterpret_cast<hipStream_t>(std::malloc(1));
+    return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t s) { return hipFree(s); }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+    *e = reinterpret_cast<hipEvent_t>(std::malloc(1));
+    return hipSuccess;
+}
+hipError_t hipEventCreate(hipEvent_t *e) { return hipEventCreateWithFlags(e, 0); }
+hipError_t hipEventDestroy(hipEvent_t e) { return hipFree(e); }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
+    *ms = 1;
+    return hipSuccess;
+}
+}  // extern "C"
+
+namespace {
+// An FP64 configuration goes up and comes back; prints the return codes, whether
+// it came back as it was, and the message left behind.
+int round_trip(gfc_ctx *c, gfc_geom g) {
+    const size_t n = (size_t)gfc_geom_volume(&g) * 72;
+    std::vector<double> U(n), out(n);
+    for (size_t k = 0; k < n; k++) U[k] = (double)k;
+    gfc_job *j = nullptr;
+    int rc = gfc_job_create(c, &g, GFC_PREC_FP64, &j);
+    fake().log.clear();
+    if (rc == GFC_OK) rc = gfc_job_upload_config(j, U.data(), 8);
+    const int up = rc;
+    const int down = gfc_job_download_config(j, out.data());
+    std::printf("up %d down %d same %d message [%s]\n", up, down, (int)(out == U),
+                gfc_last_error());
+    gfc_job_destroy(j);
+    return 0;
+}
+}  // namespace
+
+int main(int argc, char **argv) {
+    const std::string what = argc > 1 ? argv[1] : "";
+    auto arg = [&](int k) { return argc > k ? std::atol(argv[k]) : 0; };
+    gfc_ctx *c = nullptr;
+    if (gfc_ctx_create(0, &c) != GFC_OK) return 1;
+    if (what == "no_ring") {
+        // no_ring ns nt: pinned requests above 1 MiB fail
+        fake().most_pinned = 1u << 20;
+        round_trip(c, {(int)arg(2), (int)arg(3)});
+    } else {
+        return 2;
+    }
+    for (const std::string &l : fake().log) std::printf("%s\n", l.c_str());
+    gfc_ctx_destroy(c);
+    return 0;
+}

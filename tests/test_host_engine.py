@@ -1,0 +1,42 @@
+"""Error paths and launch decisions of the engine's host side, on the CPU:
+libgfc.so runs against the HIP calls of tests/fake_hip_driver.cpp, whose device
+memory is host memory and whose kernels do nothing."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "gaugefix-coulomb_amd", "lib")
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+
+@pytest.fixture(scope="module")
+def driver(tmp_path_factory):
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None or not os.path.exists(os.path.join(ROCM, "include", "hip")):
+        pytest.skip("no host C++ compiler or no HIP headers")
+    exe = str(tmp_path_factory.mktemp("fake_hip") / "fake_hip_driver")
+    # -rdynamic: the driver's HIP calls are found before libamdhip64's
+    subprocess.run([cxx, "-std=c++17", "-O1", "-rdynamic", "-D__HIP_PLATFORM_AMD__",
+                    "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROCM, "include"),
+                    os.path.join(ROOT, "tests", "fake_hip_driver.cpp"), "-o", exe,
+                    "-L", LIB, "-lgfc", "-Wl,-rpath," + LIB, "-lpthread"], check=True)
+
+    def run(*args):
+        r = subprocess.run([exe, *map(str, args)], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, (r.returncode, r.stdout[-2000:], r.stderr[-2000:])
+        return r.stdout.splitlines()
+
+    return run
+
+
+def test_transfers_without_a_ring(driver):
+    """16^3 x 32 (75 MB) would go through the ring of pinned slots; when that
+    memory is not to be had, the plain copy takes its place and nothing of the
+    failed request is left behind, neither HIP's last error (the launch check
+    after the copy would report it) nor a message."""
+    first, *log = driver("no_ring", 16, 32)
+    assert first == "up 0 down 0 same 1 message []"
+    assert [l for l in log if l.startswith("copy")] == ["copy 75497472"] * 2
