@@ -24,6 +24,7 @@ struct Fake {
     std::mutex mu;
     std::map<const void *, std::string> kernels;
     std::vector<std::string> log;
+    std::map<const char *, size_t> pinned;
     size_t most_pinned = ~(size_t)0;  // larger hipHostMalloc requests fail
     double sums = 1e3;                // what a reduction finds
 };
@@ -105,9 +106,22 @@ hipError_t hipFree(void *p) {
 }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
     if (n > fake().most_pinned) return err(hipErrorOutOfMemory);
-    return alloc(p, n);
+    if (alloc(p, n) != hipSuccess) return hipErrorOutOfMemory;
+    fake().pinned[static_cast<char *>(*p)] = n;
+    return hipSuccess;
 }
-hipError_t hipHostFree(void *p) { return hipFree(p); }
+hipError_t hipHostFree(void *p) {
+    fake().pinned.erase(static_cast<char *>(p));
+    return hipFree(p);
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *ptr) {
+    const char *p = static_cast<const char *>(ptr);
+    *a = hipPointerAttribute_t{};
+    a->type = hipMemoryTypeUnregistered;
+    auto it = fake().pinned.upper_bound(p);
+    if (it != fake().pinned.begin() && p < (--it)->first + it->second) a->type = hipMemoryTypeHost;
+    return hipSuccess;
+}
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {
     note("copy " + std::to_string(n));
     std::memcpy(d, s, n);
@@ -140,21 +154,35 @@ hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
 }  // extern "C"
 
 namespace {
-// An FP64 configuration goes up and comes back; prints the return codes, whether
-// it came back as it was, and the message left behind.
-int round_trip(gfc_ctx *c, gfc_geom g) {
+// An FP64 configuration goes up and comes back, in pageable or pinned memory;
+// prints the return codes, whether it came back as it was, and the message left
+// behind.
+int round_trip(gfc_ctx *c, gfc_geom g, bool pinned) {
     const size_t n = (size_t)gfc_geom_volume(&g) * 72;
-    std::vector<double> U(n), out(n);
+    void *m[2] = {nullptr, nullptr};
+    for (void *&p : m) {
+        if (pinned)
+            (void)hipHostMalloc(&p, n * sizeof(double), 0);
+        else
+            p = std::calloc(n, sizeof(double));
+    }
+    double *U = static_cast<double *>(m[0]), *out = static_cast<double *>(m[1]);
     for (size_t k = 0; k < n; k++) U[k] = (double)k;
     gfc_job *j = nullptr;
     int rc = gfc_job_create(c, &g, GFC_PREC_FP64, &j);
     fake().log.clear();
-    if (rc == GFC_OK) rc = gfc_job_upload_config(j, U.data(), 8);
+    if (rc == GFC_OK) rc = gfc_job_upload_config(j, U, 8);
     const int up = rc;
-    const int down = gfc_job_download_config(j, out.data());
-    std::printf("up %d down %d same %d message [%s]\n", up, down, (int)(out == U),
-                gfc_last_error());
+    const int down = gfc_job_download_config(j, out);
+    std::printf("up %d down %d same %d message [%s]\n", up, down,
+                (int)(std::memcmp(U, out, n * sizeof(double)) == 0), gfc_last_error());
     gfc_job_destroy(j);
+    for (void *p : m) {
+        if (pinned)
+            (void)hipHostFree(p);
+        else
+            std::free(p);
+    }
     return 0;
 }
 }  // namespace
@@ -167,7 +195,10 @@ int main(int argc, char **argv) {
     if (what == "no_ring") {
         // no_ring ns nt: pinned requests above 1 MiB fail
         fake().most_pinned = 1u << 20;
-        round_trip(c, {(int)arg(2), (int)arg(3)});
+        round_trip(c, {(int)arg(2), (int)arg(3)}, false);
+    } else if (what == "round_trip") {
+        // round_trip ns nt pinned
+        round_trip(c, {(int)arg(2), (int)arg(3)}, arg(4) != 0);
     } else {
         return 2;
     }

@@ -40,3 +40,18 @@ def test_transfers_without_a_ring(driver):
     first, *log = driver("no_ring", 16, 32)
     assert first == "up 0 down 0 same 1 message []"
     assert [l for l in log if l.startswith("copy")] == ["copy 75497472"] * 2
+
+
+@pytest.mark.parametrize("pinned", [0, 1])
+@pytest.mark.parametrize("ns,nt", [(8, 16), (16, 32)])
+def test_route_of_host_arrays(driver, ns, nt, pinned):
+    """Small transfers and arrays in pinned memory are one plain copy; large
+    pageable ones (75 MB) go through the ring's 8 MiB slots."""
+    first, *log = driver("round_trip", ns, nt, pinned)
+    assert first == "up 0 down 0 same 1 message []"
+    n = ns ** 3 * nt * 576
+    copies = [int(l.split()[1]) for l in log if l.startswith("copy")]
+    if ns == 8 or pinned:
+        assert copies == [n, n]
+    else:
+        assert sum(copies) == 2 * n and max(copies) == 8 << 20
