@@ -678,16 +678,29 @@ StreamSet ctx_streams(gfc_ctx *c) {
     return ss;
 }
 
-// Lattices of at most this many parity sites per timeslice (ns <= 10) run their
-// FP64 sweeps between two host decisions in one launch (k_sweep_slices).  At
-// ns = 10 a workgroup fills a CU, so more than 256 timeslices take turns: us
-// per half-sweep at nt = 300 18.8 against 16.4 in groups of timeslices, at
-// nt = 1024 41 against 50.  At ns <= 8 it is the faster one at every nt.
+// Most parity sites of a timeslice for k_sweep_slices (ns <= 10).
 constexpr int kSliceSites = 512;
 
+// Whether the FP64 sweeps between two host decisions run in one launch, a
+// workgroup per timeslice (k_sweep_slices), rather than in launches over groups
+// of timeslices.  Two of its workgroups of 256 threads (ns <= 8) share a CU,
+// one of 512 (ns = 10) fills it; more timeslices than that take turns, and the
+// threads without a site of ns < 8 are then lost time.  us per half-sweep with
+// two hits, slices / launches:
+//   ns = 2   nt = 256 6.2 / 7.8, 384 10.2 / 7.8, 2048 35 / 7.9
+//   ns = 4   nt = 16 6.1 / 8.0, 512 4.8 / 8.3, 640 10.8 / 8.2, 2048 19 / 9.3
+//   ns = 6   nt = 256 4.6 / 8.1, 512 7.9 / 8.3 (eight hits 15.7 / 12.2),
+//            640 11.6 / 9.9, 2048 30 / 21
+//   ns = 8   nt = 16 4.7 / 6.9, 512 9.7 / 13, 2048 36 / 47
+//   ns = 10  nt = 64 8.1 / 7.8 (eight hits 15.8 / 11.7), 128 8.3 / 8.6, 256
+//            9.5 / 12.8, 300 18.8 / 16.4, 1024 38 / 47: launches have a
+//            timeslice's sites on two CUs until they are more than one
+//            workgroup per CU (kOneGroup).
 bool whole_slices(const gfc_job *j, const gfc_options &o, bool fp32) {
     const int ns = j->geom.ns, nt = j->geom.nt;
-    return !fp32 && o.slice_group == 0 && ns <= 10 && (ns <= 8 || nt <= 256 || nt >= 1024);
+    if (fp32 || o.slice_group != 0 || ns > 10) return false;
+    if (ns == 10) return nt >= 1024 || (nt <= 256 && j->Vh > kOneGroup);
+    return ns == 8 || nt <= (ns == 4 ? 512 : 256);
 }
 
 int sweep_slices(gfc_job *j, int from, int to, double omega, int hits, unsigned R) {

@@ -622,10 +622,10 @@ __global__ __launch_bounds__(kBlock) void k_sweep(const cplx<T> *__restrict__ u0
 // multiples of R, as in the timeslice-blocked sweeps; the same bits.
 //
 // Bound by one wave's chain of instructions: a half-sweep launch of 8^3 x 16
-// lasts 8.5 us alone (9.4 from one to the next) whatever its loads and code
-// size, a half-sweep here 4.7 us, at 8^3 x 2048 39 against 50 us; 10^3 x 20 8.0
-// against 10.1.  (Loading the next sweep's links before the local update:
-// 5.0 us, and with 512 threads the registers spill.)
+// lasts 6.9 us from one to the next whatever its loads and code size, a
+// half-sweep here 4.7 us; 8^3 x 2048 47 and 36 us, 10^3 x 256 12.8 and 9.5.
+// (Loading the next sweep's links before the local update: 5.0 us, and with 512
+// threads the registers spill.)
 template <int N>
 __global__ __launch_bounds__(N) void k_sweep_slices(const cplx<double> *__restrict__ u0,
                                                     cplx<double> *__restrict__ g, Extents x,

@@ -161,11 +161,11 @@ typedef struct {
                                Infinity Cache between half-sweeps (read with
                                cached loads); a lattice that fits in it whole
                                is swept as one, two or three groups, by its
-                               size, in FP64 with ns <= 10 in one launch
-                               between decisions; single timeslices when a wave
-                               of them does not fit; -1: whole-lattice
-                               sweeps.  With retire_slices, one timeslice per
-                               group.                                         */
+                               size, or in FP64 with ns <= 10, depending on
+                               nt, in one launch between decisions; single
+                               timeslices when a wave of them does not fit;
+                               -1: whole-lattice sweeps.  With retire_slices,
+                               one timeslice per group.                       */
     int slice_lanes;        /* streams over which the timeslice groups run
                                concurrently: 1-4, or 0 (default): up to three
                                for a lattice that fits the cache whole, two or

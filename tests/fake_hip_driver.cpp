@@ -79,6 +79,9 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t, h
         double *out = *static_cast<double **>(args[2]);
         for (int k = 0; k < 3; k++) out[k] = fake().sums;
     }
+    if (name.find("k_sweep_slices") != std::string::npos)
+        note("sweeps " + std::to_string(*static_cast<int *>(args[5])) + " " +
+             std::to_string(*static_cast<int *>(args[6])));
     return hipSuccess;
 }
 const char *hipGetErrorString(hipError_t e) {
@@ -199,6 +202,27 @@ int main(int argc, char **argv) {
     } else if (what == "round_trip") {
         // round_trip ns nt pinned
         round_trip(c, {(int)arg(2), (int)arg(3)}, arg(4) != 0);
+    } else if (what == "fix") {
+        // fix ns nt precision sweeps hits slice_group slice_lanes
+        gfc_geom g = {(int)arg(2), (int)arg(3)};
+        gfc_params p;
+        gfc_params_default(&p);
+        p.tolerance = 1e-300;
+        p.estimate_sweeps_to_gf_progress = 100000000;
+        p.max_sweeps_to_fix = (unsigned)arg(5);
+        p.hits = (unsigned)arg(6);
+        gfc_options o;
+        gfc_options_default(&o);
+        o.precision = (int)arg(4);
+        o.slice_group = (int)arg(7);
+        o.slice_lanes = (int)arg(8);
+        gfc_job *j = nullptr;
+        if (gfc_job_create(c, &g, o.precision, &j) != GFC_OK) return 1;
+        fake().log.clear();
+        gfc_report r;
+        const int rc = gfc_job_fix(j, &p, &o, &r);
+        std::printf("fix %d sweeps %d message [%s]\n", rc, r.sweeps, gfc_last_error());
+        gfc_job_destroy(j);
     } else {
         return 2;
     }

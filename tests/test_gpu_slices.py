@@ -53,3 +53,12 @@ def test_to_tolerance_with_dense_checks(ctx, proxy):
                    gfc.Params(tolerance=1e-14, estimate_sweeps_to_gf_progress=0, gfix_proxy=proxy,
                               sweeps_to_reunitarization=10))
     assert rc > 0
+
+
+@pytest.mark.parametrize("ns,nt", [(2, 256), (4, 300), (6, 258), (8, 300), (10, 132), (10, 256)])
+@pytest.mark.parametrize("hits", [2, 8])
+def test_both_sides_of_the_rule(ctx, ns, nt, hits):
+    """More timeslices than CUs and the edges of what runs in one launch."""
+    _both(ctx, gfc.Geometry(ns, nt),
+          gfc.Params(tolerance=1e-300, estimate_sweeps_to_gf_progress=100000000,
+                     max_sweeps_to_fix=23, sweeps_to_reunitarization=10, hits=hits))

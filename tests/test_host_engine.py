@@ -55,3 +55,22 @@ def test_route_of_host_arrays(driver, ns, nt, pinned):
         assert copies == [n, n]
     else:
         assert sum(copies) == 2 * n and max(copies) == 8 << 20
+
+
+def _fix(driver, ns, nt, prec=0, sweeps=20, hits=2, group=0, lanes=0):
+    first, *log = driver("fix", ns, nt, prec, sweeps, hits, group, lanes)
+    assert first.startswith(f"fix -1 sweeps {sweeps} ")
+    return log
+
+
+@pytest.mark.parametrize("ns,nt,slices", [
+    (2, 256, 1), (2, 258, 0), (2, 2000, 0), (4, 2, 1), (4, 512, 1), (4, 514, 0),
+    (6, 256, 1), (6, 258, 0), (8, 2, 1), (8, 2000, 1), (10, 64, 0), (10, 130, 0),
+    (10, 132, 1), (10, 256, 1), (10, 258, 0), (10, 1022, 0), (10, 1024, 1), (12, 16, 0)])
+def test_route_of_small_lattices(driver, ns, nt, slices):
+    """FP64 sweeps in one launch per host decision or in one per half-sweep, on
+    both sides of each line of the rule."""
+    log = _fix(driver, ns, nt)
+    assert len([l for l in log if "k_sweep_slices" in l]) == slices
+    launches = [l for l in log if "k_sweep" in l and "slices" not in l]
+    assert len(launches) == 0 if slices else len(launches) >= 20
