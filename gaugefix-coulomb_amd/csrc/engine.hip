@@ -708,10 +708,12 @@ int sweep_slices(gfc_job *j, int from, int to, double omega, int hits, unsigned 
     const gfc::Extents x = gfc::make_extents(ns, j->Vh);
     const dim3 grid((unsigned)j->geom.nt);
     hipStream_t s = j->ctx->stream;
-    // at most some 20 ms a launch
-    constexpr int kMost = 2000;
-    for (int a = from; a < to; a += kMost) {
-        const int b = std::min(to, a + kMost);
+    // at most about 20 ms a launch (one half-sweep at least): a turn of 256
+    // timeslices takes 3.5 us and 0.65 per hit at ns = 8, 6.1 and 1.2 at ns = 10
+    const double us = ((j->geom.nt + 255) / 256) * (6 + 1.2 * std::max(hits, 0));
+    const int most = std::max(1, (int)(20e3 / us));
+    for (int a = from; a < to; a += most) {
+        const int b = std::min(to, a + most);
         if (S <= 256)
             hipLaunchKernelGGL((gfc::k_sweep_slices<256>), grid, dim3(256), 0, s, j->u0, j->g, x,
                                omega, hits, a, b, to, R);

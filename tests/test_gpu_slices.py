@@ -3,7 +3,7 @@ one launch, a workgroup per timeslice with its G in LDS.  The result must equal
 whole-lattice sweeps bit for bit: timeslices smaller than a wave, ones that
 fill a workgroup exactly (ns = 8) or not (ns = 10), any reunitarization period
 and hits, odd sweep counts (either parity last), more sweeps than one launch
-takes (2000), and checks that fall on reunitarization points."""
+takes (some 2400), and checks that fall on reunitarization points."""
 import numpy as np
 import pytest
 

@@ -74,3 +74,19 @@ def test_route_of_small_lattices(driver, ns, nt, slices):
     assert len([l for l in log if "k_sweep_slices" in l]) == slices
     launches = [l for l in log if "k_sweep" in l and "slices" not in l]
     assert len(launches) == 0 if slices else len(launches) >= 20
+
+
+@pytest.mark.parametrize("nt,hits", [(16, 2), (4096, 2), (4096, 30), (16384, 2), (2, 100000)])
+def test_work_of_a_launch_is_bounded(driver, nt, hits):
+    """k_sweep_slices at ns = 8: the half-sweeps of a launch follow the
+    timeslices that take turns on a CU and the hits, so that a launch stays near
+    20 ms; together they are all of them, in order."""
+    n = 5000
+    log = _fix(driver, 8, nt, sweeps=n, hits=hits)
+    runs = [tuple(map(int, l.split()[1:])) for l in log if l.startswith("sweeps")]
+    assert runs[0][0] == 0 and runs[-1][1] == n
+    assert all(a[1] == b[0] for a, b in zip(runs, runs[1:]))
+    most = max(b - a for a, b in runs)
+    us = -(-nt // 256) * (3.5 + 0.65 * hits)
+    assert most == 1 or most * us < 20e3
+    assert most * us > 5e3  # and no shorter than that either
