@@ -683,7 +683,7 @@ constexpr int kSliceSites = 512;
 
 // Whether the FP64 sweeps between two host decisions run in one launch, a
 // workgroup per timeslice (k_sweep_slices), rather than in launches over groups
-// of timeslices.  Two of its workgroups of 256 threads (ns <= 8) share a CU,
+// of timeslices, which a caller may ask for by their size or streams.  Two of its workgroups of 256 threads (ns <= 8) share a CU,
 // one of 512 (ns = 10) fills it; more timeslices than that take turns, and the
 // threads without a site of ns < 8 are then lost time.  us per half-sweep with
 // two hits, slices / launches:
@@ -698,7 +698,8 @@ constexpr int kSliceSites = 512;
 //            workgroup per CU (kOneGroup).
 bool whole_slices(const gfc_job *j, const gfc_options &o, bool fp32) {
     const int ns = j->geom.ns, nt = j->geom.nt;
-    if (fp32 || o.slice_group != 0 || ns > 10) return false;
+    const bool lanes = o.slice_lanes >= 1 && o.slice_lanes <= gfc_ctx::kLanes;
+    if (fp32 || o.slice_group != 0 || lanes || ns > 10) return false;
     if (ns == 10) return nt >= 1024 || (nt <= 256 && j->Vh > kOneGroup);
     return ns == 8 || nt <= (ns == 4 ? 512 : 256);
 }

@@ -90,3 +90,14 @@ def test_work_of_a_launch_is_bounded(driver, nt, hits):
     us = -(-nt // 256) * (3.5 + 0.65 * hits)
     assert most == 1 or most * us < 20e3
     assert most * us > 5e3  # and no shorter than that either
+
+
+@pytest.mark.parametrize("group,lanes,launches", [(0, 1, 20), (0, 2, 40), (0, 4, 80), (4, 0, 80),
+                                                  (-1, 0, 20)])
+def test_groups_and_streams_that_are_asked_for(driver, group, lanes, launches):
+    """slice_group and slice_lanes are kept to where the default would be one
+    launch (8^3 x 16, 20 half-sweeps): nt / lanes timeslices per group."""
+    log = _fix(driver, 8, 16, group=group, lanes=lanes)
+    sweeps = [l.split() for l in log if "k_sweep" in l]
+    assert all("slices" not in l[1] for l in sweeps) and len(sweeps) == launches
+    assert all(int(l[2]) == (16 if group < 0 else 16 // (lanes or 4)) for l in sweeps)
