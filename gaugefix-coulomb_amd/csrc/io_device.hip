@@ -23,8 +23,10 @@
 #include <atomic>
 #include <cstdio>
 #include <cstring>
+#include <exception>
+#include <memory>
+#include <new>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -161,27 +163,29 @@ int make_ring(gfc_ctx *c) {
 // another way, so the failed request must not be reported by the next launch
 // check (HIP keeps an error until it is read) nor by gfc_last_error.
 bool ring(gfc_ctx *c) {
-    const std::string message = gfcx::last_error;
-    if (make_ring(c) == GFC_OK) return true;
-    (void)hipGetLastError();
-    gfcx::last_error = message;
-    return false;
+    std::string message;
+    message.swap(gfcx::last_error);
+    const bool have = make_ring(c) == GFC_OK;
+    if (!have) (void)hipGetLastError();
+    gfcx::last_error.swap(message);
+    return have;
 }
 
 // Host threads that take the pieces of a transfer in turn and copy each once
 // its block is open, i.e. below `open`.  done[b] counts the pieces of block b
 // that are copied.  They end when every piece is taken or `stop` is set, and
-// are joined by the destructor.
+// are joined by the destructor.  Nothing here throws: the callers are C entries.
 struct Copiers {
     std::atomic<size_t> open{0}, next{0};
     std::atomic<bool> stop{false};
-    std::vector<std::atomic<size_t>> done;
+    std::unique_ptr<std::atomic<size_t>[]> done;
     std::vector<std::thread> th;
 
-    explicit Copiers(size_t blocks) : done(blocks) {}
+    explicit Copiers(size_t blocks) : done(new (std::nothrow) std::atomic<size_t>[blocks]()) {}
     // copy(block, offset, n) for every piece; false if no thread could start.
     template <typename Copy>
     bool start(size_t total, Copy copy) {
+        if (!done) return false;
         const size_t pieces = (total + kPiece - 1) / kPiece;
         const int nth = (int)std::min<size_t>(
             kCopyThreads, std::max(1u, std::thread::hardware_concurrency()));
@@ -200,8 +204,8 @@ struct Copiers {
                         done[b].fetch_add(1, std::memory_order_release);
                     }
                 });
-        } catch (const std::system_error &) {
-            return !th.empty();  // fewer threads do the same work
+        } catch (const std::exception &) {  // no memory, or no thread
+            return !th.empty();             // fewer threads do the same work
         }
         return true;
     }
@@ -342,8 +346,9 @@ int gfcx::copy_from_host(gfc_ctx *c, hipStream_t s, void *dst, const void *src, 
 // Host array src -> host array dst, the server's own copy of an input (new
 // memory: most of its time is the first touch of its pages).
 void gfcx::copy_host(void *dst, const void *src, size_t total) {
-    Copiers cp((total + kSlot - 1) / kSlot);
-    cp.open.store(cp.done.size(), std::memory_order_relaxed);
+    const size_t blocks = (total + kSlot - 1) / kSlot;
+    Copiers cp(blocks);
+    cp.open.store(blocks, std::memory_order_relaxed);
     char *d = static_cast<char *>(dst);
     const char *f = static_cast<const char *>(src);
     if (total < kRingMin ||
@@ -351,7 +356,7 @@ void gfcx::copy_host(void *dst, const void *src, size_t total) {
         std::memcpy(d, f, total);
         return;
     }
-    for (size_t b = 0; b < cp.done.size(); b++) cp.wait(b, total);
+    for (size_t b = 0; b < blocks; b++) cp.wait(b, total);
 }
 
 extern "C" int gfc_job_load_config(gfc_job *j, const char *path, int in_precision,

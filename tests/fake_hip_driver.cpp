@@ -14,6 +14,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -33,15 +34,23 @@ Fake &fake() {
     return f;
 }
 thread_local hipError_t last = hipSuccess;
+thread_local bool no_memory = false;  // operator new fails on this thread
 thread_local dim3 cfg_grid, cfg_block;
 
 hipError_t err(hipError_t e) {
     last = e;
     return e;
 }
-void note(const std::string &s) {
+// Memory for the driver itself.
+struct Memory {
+    const bool was = no_memory;
+    Memory() { no_memory = false; }
+    ~Memory() { no_memory = was; }
+};
+void note(const char *what, size_t n) {
+    Memory m;
     std::lock_guard<std::mutex> lk(fake().mu);
-    fake().log.push_back(s);
+    fake().log.push_back(std::string(what) + " " + std::to_string(n));
 }
 hipError_t alloc(void **p, size_t n) {
     *p = std::calloc(n ? n : 1, 1);
@@ -73,15 +82,16 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *shared, hipStream
     return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t, hipStream_t) {
+    Memory m;
     const std::string &name = fake().kernels[f];
-    note("launch " + name + " " + std::to_string(g.x) + " " + std::to_string(b.x));
+    note(("launch " + name + " " + std::to_string(g.x)).c_str(), b.x);
     if (name.find("k_reduce_final") != std::string::npos) {
         double *out = *static_cast<double **>(args[2]);
         for (int k = 0; k < 3; k++) out[k] = fake().sums;
     }
     if (name.find("k_sweep_slices") != std::string::npos)
-        note("sweeps " + std::to_string(*static_cast<int *>(args[5])) + " " +
-             std::to_string(*static_cast<int *>(args[6])));
+        note(("sweeps " + std::to_string(*static_cast<int *>(args[5]))).c_str(),
+             *static_cast<int *>(args[6]));
     return hipSuccess;
 }
 const char *hipGetErrorString(hipError_t e) {
@@ -110,6 +120,7 @@ hipError_t hipFree(void *p) {
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
     if (n > fake().most_pinned) return err(hipErrorOutOfMemory);
     if (alloc(p, n) != hipSuccess) return hipErrorOutOfMemory;
+    Memory m;
     fake().pinned[static_cast<char *>(*p)] = n;
     return hipSuccess;
 }
@@ -126,7 +137,7 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *ptr) {
     return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {
-    note("copy " + std::to_string(n));
+    note("copy", n);
     std::memcpy(d, s, n);
     return hipSuccess;
 }
@@ -156,11 +167,19 @@ hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
 }
 }  // extern "C"
 
+void *operator new(size_t n) {
+    void *p = no_memory ? nullptr : std::malloc(n ? n : 1);
+    if (p == nullptr) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
+
 namespace {
 // An FP64 configuration goes up and comes back, in pageable or pinned memory;
 // prints the return codes, whether it came back as it was, and the message left
 // behind.
-int round_trip(gfc_ctx *c, gfc_geom g, bool pinned) {
+int round_trip(gfc_ctx *c, gfc_geom g, bool pinned, bool starved) {
     const size_t n = (size_t)gfc_geom_volume(&g) * 72;
     void *m[2] = {nullptr, nullptr};
     for (void *&p : m) {
@@ -174,9 +193,11 @@ int round_trip(gfc_ctx *c, gfc_geom g, bool pinned) {
     gfc_job *j = nullptr;
     int rc = gfc_job_create(c, &g, GFC_PREC_FP64, &j);
     fake().log.clear();
+    no_memory = starved;
     if (rc == GFC_OK) rc = gfc_job_upload_config(j, U, 8);
     const int up = rc;
     const int down = gfc_job_download_config(j, out);
+    no_memory = false;
     std::printf("up %d down %d same %d message [%s]\n", up, down,
                 (int)(std::memcmp(U, out, n * sizeof(double)) == 0), gfc_last_error());
     gfc_job_destroy(j);
@@ -198,10 +219,10 @@ int main(int argc, char **argv) {
     if (what == "no_ring") {
         // no_ring ns nt: pinned requests above 1 MiB fail
         fake().most_pinned = 1u << 20;
-        round_trip(c, {(int)arg(2), (int)arg(3)}, false);
+        round_trip(c, {(int)arg(2), (int)arg(3)}, false, false);
     } else if (what == "round_trip") {
-        // round_trip ns nt pinned
-        round_trip(c, {(int)arg(2), (int)arg(3)}, arg(4) != 0);
+        // round_trip ns nt pinned starved
+        round_trip(c, {(int)arg(2), (int)arg(3)}, arg(4) != 0, arg(5) != 0);
     } else if (what == "fix") {
         // fix ns nt precision sweeps hits slice_group slice_lanes
         gfc_geom g = {(int)arg(2), (int)arg(3)};

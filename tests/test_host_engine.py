@@ -57,6 +57,14 @@ def test_route_of_host_arrays(driver, ns, nt, pinned):
         assert sum(copies) == 2 * n and max(copies) == 8 << 20
 
 
+def test_transfers_without_host_memory(driver):
+    """No exception leaves a C entry: without memory for the copying threads the
+    transfer is one plain copy."""
+    first, *log = driver("round_trip", 16, 32, 0, 1)
+    assert first == "up 0 down 0 same 1 message []"
+    assert [l for l in log if l.startswith("copy")] == ["copy 75497472"] * 2
+
+
 def _fix(driver, ns, nt, prec=0, sweeps=20, hits=2, group=0, lanes=0):
     first, *log = driver("fix", ns, nt, prec, sweeps, hits, group, lanes)
     assert first.startswith(f"fix -1 sweeps {sweeps} ")
