@@ -797,35 +797,47 @@ int promote_g(gfc_job *j, SweepState &st) {
 }
 
 // The sums behind a per-sweep trace, one triple per half-sweep, kept on the
-// device until the fix ends: a host round trip after every sweep took 25 of the
-// 57 us of a traced sweep at 16^3 x 32.
+// device and read kMost at a time: a host round trip after every sweep took 25
+// of the 57 us of a traced sweep at 16^3 x 32.  A fix that fails part way leaves
+// the values it had.
 struct TraceSums {
+    static constexpr int kMost = 1024;
+    gfc_job *j;
+    int which;
+    double *trace;
     double *dev = nullptr;
-    int n = 0;
-    ~TraceSums() { hipFree(dev); }
-    int init(int len) {
-        HIP_TRY(hipMalloc(&dev, sizeof(double) * 3 * (size_t)len));
+    int n = 0;  // sums not yet in the trace, which ends before `trace`
+    TraceSums(gfc_job *j, int which, double *trace) : j(j), which(which), trace(trace) {}
+    ~TraceSums() {
+        (void)flush();
+        hipFree(dev);
+    }
+    int init() {
+        HIP_TRY(hipMalloc(&dev, sizeof(double) * 3 * kMost));
         return GFC_OK;
     }
-    // After half-sweep k (1, 2, ...).
-    int add(gfc_job *j, bool fp32, int k) {
+    // After each half-sweep.
+    int add(bool fp32) {
         RC_TRY(obs_partials(j, fp32));
-        RC_TRY(reduce_to(j->ctx, nblocks(2 * (int64_t)j->Vh), dev + 3 * (size_t)(k - 1)));
-        n = k;
+        RC_TRY(reduce_to(j->ctx, nblocks(2 * (int64_t)j->Vh), dev + 3 * n));
+        if (++n == kMost) HIP_TRY(flush());
         return GFC_OK;
     }
-    int finish(gfc_job *j, int which, double *trace) {
-        if (n == 0) return GFC_OK;
-        std::vector<double> s(3 * (size_t)n);
-        HIP_TRY(hipMemcpyAsync(s.data(), dev, sizeof(double) * s.size(), hipMemcpyDeviceToHost,
-                               j->ctx->stream));
-        HIP_TRY(hipStreamSynchronize(j->ctx->stream));
-        for (int k = 0; k < n; k++) {
+    hipError_t flush() {
+        if (n == 0) return hipSuccess;
+        double s[3 * kMost];
+        const int m = n;
+        n = 0;
+        hipError_t e = hipMemcpyAsync(s, dev, sizeof(double) * 3 * m, hipMemcpyDeviceToHost,
+                                      j->ctx->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(j->ctx->stream);
+        if (e != hipSuccess) return e;
+        for (int k = 0; k < m; k++) {
             double ob[3];
-            obs_means(j, &s[3 * (size_t)k], ob);
-            trace[k] = ob[which];
+            obs_means(j, s + 3 * k, ob);
+            *trace++ = ob[which];
         }
-        return GFC_OK;
+        return e;
     }
 };
 
@@ -1009,10 +1021,8 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
         RC_TRY(sl.init(j));
     }
 
-    TraceSums sums;
-    if (trace && trace_len > 0)
-        RC_TRY(sums.init((int)std::min<unsigned>((unsigned)trace_len,
-                                                 std::max(1u, p->max_sweeps_to_fix))));
+    TraceSums sums(j, which, trace);
+    if (trace && trace_len > 0) RC_TRY(sums.init());
 
     RC_TRY(begin_fix(j, j->ctx->stream, st.fp32));
     RC_TRY(obs_factored(j, st.fp32, ob));
@@ -1067,7 +1077,7 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
             if (in32) r.sweeps_fp32++;
         }
         timer.after();
-        if (trace && sweep <= trace_len) RC_TRY(sums.add(j, st.fp32, sweep));
+        if (trace && sweep <= trace_len) RC_TRY(sums.add(st.fp32));
         if (((st.fp32 && !ho.at_floor) || sl.on) && sweep != due &&
             sweep % o.mixed_probe_every == 0) {
             double g = 0;
@@ -1118,7 +1128,7 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
     // the FP32 phase (tolerance reached there or max sweeps).
     RC_TRY(end_frame(j, j->ctx->stream, st.fp32, sweep, !done));
     RC_TRY(materialize(j, !done));
-    if (trace) RC_TRY(sums.finish(j, which, trace));
+    HIP_TRY(sums.flush());
     HIP_TRY(hipStreamSynchronize(j->ctx->stream));
     r.seconds_sweeps = timer.seconds();
     r.sweeps = sweep;

@@ -28,6 +28,7 @@ struct Fake {
     std::map<const char *, size_t> pinned;
     size_t most_pinned = ~(size_t)0;  // larger hipHostMalloc requests fail
     double sums = 1e3;                // what a reduction finds
+    long sweeps_left = -1;            // sweep launches before one fails (< 0: none)
 };
 Fake &fake() {
     static Fake f;
@@ -84,6 +85,9 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *shared, hipStream
 hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t, hipStream_t) {
     Memory m;
     const std::string &name = fake().kernels[f];
+    if (name.find("k_sweep") != std::string::npos && fake().sweeps_left >= 0 &&
+        fake().sweeps_left-- == 0)
+        return err(hipErrorLaunchFailure);
     note(("launch " + name + " " + std::to_string(g.x)).c_str(), b.x);
     if (name.find("k_reduce_final") != std::string::npos) {
         double *out = *static_cast<double **>(args[2]);
@@ -243,6 +247,28 @@ int main(int argc, char **argv) {
         gfc_report r;
         const int rc = gfc_job_fix(j, &p, &o, &r);
         std::printf("fix %d sweeps %d message [%s]\n", rc, r.sweeps, gfc_last_error());
+        gfc_job_destroy(j);
+    } else if (what == "trace") {
+        // trace ns nt sweeps trace_len done: the launch of half-sweep done + 1
+        // fails; 8 numbers behind the trace are looked at too
+        gfc_geom g = {(int)arg(2), (int)arg(3)};
+        gfc_params p;
+        gfc_params_default(&p);
+        p.tolerance = 1e-300;
+        p.estimate_sweeps_to_gf_progress = 100000000;
+        p.max_sweeps_to_fix = (unsigned)arg(4);
+        gfc_job *j = nullptr;
+        if (gfc_job_create(c, &g, GFC_PREC_FP64, &j) != GFC_OK) return 1;
+        fake().log.clear();
+        const int len = (int)arg(5);
+        std::vector<double> tr(len + 8, -1.0);
+        gfc_report r;
+        fake().sweeps_left = arg(6);
+        const int rc = gfc_job_fix_trace(j, &p, nullptr, &r, tr.data(), len);
+        fake().sweeps_left = -1;
+        int set = 0;
+        while (set < (int)tr.size() && tr[set] > 0) set++;
+        std::printf("trace %d set %d of %d\n", rc, set, len);
         gfc_job_destroy(j);
     } else {
         return 2;

@@ -109,3 +109,15 @@ def test_groups_and_streams_that_are_asked_for(driver, group, lanes, launches):
     sweeps = [l.split() for l in log if "k_sweep" in l]
     assert all("slices" not in l[1] for l in sweeps) and len(sweeps) == launches
     assert all(int(l[2]) == (16 if group < 0 else 16 // (lanes or 4)) for l in sweeps)
+
+
+@pytest.mark.parametrize("sweeps,length,done", [
+    (20, 20, -1), (20, 7, -1), (20, 40, -1), (20, 0, -1), (3000, 2500, -1), (2048, 2048, -1),
+    (20, 20, 5), (20, 3, 5), (3000, 2500, 1024), (3000, 2500, 1030)])
+def test_trace_of_a_fix_that_ends_anywhere(driver, sweeps, length, done):
+    """Every value of the trace up to its length or the last half-sweep is set,
+    and none behind it; a fix whose launch after half-sweep `done` fails leaves
+    those it had."""
+    rc, done = (-3, done) if done >= 0 else (-1, sweeps)
+    assert driver("trace", 4, 2, sweeps, length, done if rc == -3 else -1)[0] == \
+        f"trace {rc} set {min(length, done)} of {length}"
