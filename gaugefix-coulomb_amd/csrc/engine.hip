@@ -985,6 +985,20 @@ struct SliceTracker {
     }
 };
 
+// A fix that fails leaves G = 1: during it G is in another frame than the
+// job's U, which is only written at its end.
+struct GaugeGuard {
+    gfc_job *j;
+    bool done = false;
+    ~GaugeGuard() {
+        if (done) return;
+        std::string message;
+        message.swap(gfcx::last_error);
+        (void)set_identity(j);
+        gfcx::last_error.swap(message);
+    }
+};
+
 int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report *rep,
             double *trace, int trace_len) {
     if (j == nullptr || p == nullptr) return fail(GFC_EINVAL, "gfc_job_fix: NULL argument");
@@ -1009,15 +1023,14 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
     st.fp32 = o.precision == GFC_PREC_MIXED;
     double ob[3];
 
+    GaugeGuard guard{j};
     SweepTimer timer;
     timer.on = o.time_sweeps != 0;
     timer.s = j->ctx->stream;
     SliceTracker sl;
     if (o.retire_slices) {
-        if (j->geom.ns % 8) {
-            RC_TRY(set_identity(j));
+        if (j->geom.ns % 8)
             return fail(GFC_EINVAL, "gfc_job_fix: retire_slices needs ns a multiple of 8");
-        }
         RC_TRY(sl.init(j));
     }
 
@@ -1127,6 +1140,7 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
     // the max-sweeps and stall exits return before it.  The loop may be left in
     // the FP32 phase (tolerance reached there or max sweeps).
     RC_TRY(end_frame(j, j->ctx->stream, st.fp32, sweep, !done));
+    guard.done = true;
     RC_TRY(materialize(j, !done));
     HIP_TRY(sums.flush());
     HIP_TRY(hipStreamSynchronize(j->ctx->stream));

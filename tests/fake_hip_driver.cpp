@@ -228,7 +228,8 @@ int main(int argc, char **argv) {
         // round_trip ns nt pinned starved
         round_trip(c, {(int)arg(2), (int)arg(3)}, arg(4) != 0, arg(5) != 0);
     } else if (what == "fix") {
-        // fix ns nt precision sweeps hits slice_group slice_lanes
+        // fix ns nt precision sweeps hits slice_group slice_lanes retire done:
+        // the launch of half-sweep done + 1 fails if done is given
         gfc_geom g = {(int)arg(2), (int)arg(3)};
         gfc_params p;
         gfc_params_default(&p);
@@ -241,11 +242,14 @@ int main(int argc, char **argv) {
         o.precision = (int)arg(4);
         o.slice_group = (int)arg(7);
         o.slice_lanes = (int)arg(8);
+        o.retire_slices = (int)arg(9);
         gfc_job *j = nullptr;
         if (gfc_job_create(c, &g, o.precision, &j) != GFC_OK) return 1;
         fake().log.clear();
-        gfc_report r;
+        gfc_report r{};
+        fake().sweeps_left = argc > 10 ? arg(10) : -1;
         const int rc = gfc_job_fix(j, &p, &o, &r);
+        fake().sweeps_left = -1;
         std::printf("fix %d sweeps %d message [%s]\n", rc, r.sweeps, gfc_last_error());
         gfc_job_destroy(j);
     } else if (what == "trace") {

@@ -121,3 +121,15 @@ def test_trace_of_a_fix_that_ends_anywhere(driver, sweeps, length, done):
     rc, done = (-3, done) if done >= 0 else (-1, sweeps)
     assert driver("trace", 4, 2, sweeps, length, done if rc == -3 else -1)[0] == \
         f"trace {rc} set {min(length, done)} of {length}"
+
+
+@pytest.mark.parametrize("ns,prec,retire,rc,why", [
+    (16, 0, 0, -3, "hipGetLastError(): error"), (16, 1, 0, -3, "hipGetLastError(): error"),
+    (16, 0, 1, -3, "hipGetLastError(): error"),
+    (6, 0, 1, -6, "gfc_job_fix: retire_slices needs ns a multiple of 8")])
+def test_failed_fix_leaves_the_identity(driver, ns, prec, retire, rc, why):
+    """Whether a launch fails half way or the call is refused, the last thing
+    written is G = 1, and the message is that of the failure."""
+    first, *log = driver("fix", ns, 4, prec, 20, 2, 0, 0, retire, 7)
+    assert first == f"fix {rc} sweeps 0 message [{why}]"
+    assert "k_g_identity" in [l for l in log if l.startswith("launch")][-1]
