@@ -423,6 +423,9 @@ int obs_partials(gfc_job *j, bool fp32) {
     if (fp32)
         hipLaunchKernelGGL((gfc::k_obs_factored<float>), dim3(b), dim3(kBlock), 0, c->stream,
                            j->u0, j->gf, j->geom.ns, j->Vh, c->part);
+    else if (j->own)
+        hipLaunchKernelGGL((gfc::k_obs_factored<double, true>), dim3(b), dim3(kBlock), 0,
+                           c->stream, j->u0, j->g, j->geom.ns, j->Vh, c->part);
     else
         hipLaunchKernelGGL((gfc::k_obs_factored<double>), dim3(b), dim3(kBlock), 0, c->stream,
                            j->u0, j->g, j->geom.ns, j->Vh, c->part);
@@ -446,11 +449,16 @@ int obs_factored(gfc_job *j, bool fp32, double out[3]) {
     return GFC_OK;
 }
 
-int obs_aos(gfc_job *j, double out[3]) {
+// Residues of cfg; *off, if given, is set to 1 when a link is not near SU(3).
+int obs_aos(gfc_job *j, double out[3], int *off = nullptr) {
     gfc_ctx *c = j->ctx;
     const unsigned b = gfc::aos_blocks(j->V);
-    hipLaunchKernelGGL(gfc::k_obs_aos, dim3(b), dim3(kBlock), 0, c->stream, j->cfg, j->geom.ns,
-                       j->V, gfc::aos_groups(j->V), c->part);
+    if (off)
+        hipLaunchKernelGGL(gfc::k_obs_aos<true>, dim3(b), dim3(kBlock), 0, c->stream, j->cfg,
+                           j->geom.ns, j->V, gfc::aos_groups(j->V), c->part, off);
+    else
+        hipLaunchKernelGGL(gfc::k_obs_aos<>, dim3(b), dim3(kBlock), 0, c->stream, j->cfg,
+                           j->geom.ns, j->V, gfc::aos_groups(j->V), c->part, off);
     LAUNCH_CHECK();
     double s[3];
     RC_TRY(finish_reduction(c, b, s));
@@ -470,24 +478,32 @@ int begin_frame(gfc_job *j, hipStream_t s) {
     return GFC_OK;
 }
 
-// State at the start of a fix: G = 1 and u0, for FP64 sweeps in the axial
-// frame, for the FP32 phase of a mixed fix in the configuration's own.
-int begin_fix(gfc_job *j, hipStream_t s, bool mixed) {
-    if (!mixed) return begin_frame(j, s);
+// State at the start of a fix: G = 1 and u0, for FP64 sweeps in the axial frame
+// unless j->own, for the FP32 phase of a mixed fix in the configuration's own;
+// *off, if given, is set to 1 when a link of a mixed fix is not near SU(3).
+int begin_fix(gfc_job *j, hipStream_t s, bool mixed, int *off) {
+    if (!mixed && !j->own) return begin_frame(j, s);
     const unsigned b = nblocks(2 * (int64_t)j->Vh);
-    hipLaunchKernelGGL(gfc::k_build_u0, dim3(b), dim3(kBlock), 0, s, j->cfg, j->u0, j->u0f,
-                       j->geom.ns, j->Vh);
+    hipLaunchKernelGGL(gfc::k_build_u0, dim3(b), dim3(kBlock), 0, s, j->cfg, j->u0,
+                       mixed ? j->u0f : nullptr, j->geom.ns, j->Vh, off);
     LAUNCH_CHECK();
-    hipLaunchKernelGGL(gfc::k_g_identity<float>, dim3(b), dim3(kBlock), 0, s, j->gf, j->Vh);
+    if (mixed)
+        hipLaunchKernelGGL(gfc::k_g_identity<float>, dim3(b), dim3(kBlock), 0, s, j->gf, j->Vh);
+    else
+        hipLaunchKernelGGL(gfc::k_g_identity<double>, dim3(b), dim3(kBlock), 0, s, j->g, j->Vh);
     LAUNCH_CHECK();
     return GFC_OK;
 }
 
-// FP32 -> FP64 hand-off: u0 and G go into the axial frame.
+// FP32 -> FP64 hand-off: u0 and G go into the axial frame, unless j->own.
 int promote_g(gfc_job *j, hipStream_t s) {
-    RC_TRY(begin_frame(j, s));
-    hipLaunchKernelGGL(gfc::k_g_promote<true>, dim3(nblocks(2 * (int64_t)j->Vh)), dim3(kBlock), 0,
-                       s, j->gf, j->g, j->Vh);
+    const dim3 b(nblocks(2 * (int64_t)j->Vh));
+    if (j->own) {
+        hipLaunchKernelGGL(gfc::k_g_promote<false>, b, dim3(kBlock), 0, s, j->gf, j->g, j->Vh);
+    } else {
+        RC_TRY(begin_frame(j, s));
+        hipLaunchKernelGGL(gfc::k_g_promote<true>, b, dim3(kBlock), 0, s, j->gf, j->g, j->Vh);
+    }
     LAUNCH_CHECK();
     return GFC_OK;
 }
@@ -496,8 +512,9 @@ int promote_g(gfc_job *j, hipStream_t s) {
 // its last reunitarization if `project`; if it ended in the FP32 phase, promoted
 // (and so projected) in the configuration's own frame, which that phase keeps
 // (mixed fixes stopped in it, through the axial frame and without: 16^3 x 32
-// after 100 half-sweeps 0.996 and 0.837 ms, 56^3 x 56 after 60 27.1 and 23.7).  Without a sweep G is the identity (also for a configuration whose
-// residue is no number).
+// after 100 half-sweeps 0.996 and 0.837 ms, 56^3 x 56 after 60 27.1 and 23.7).
+// Without a sweep G is the identity (also for a configuration whose residue is
+// no number).
 int end_frame(gfc_job *j, hipStream_t s, bool fp32, int sweeps, bool project) {
     if (sweeps == 0) return set_identity(j, s);
     if (fp32) {
@@ -506,6 +523,7 @@ int end_frame(gfc_job *j, hipStream_t s, bool fp32, int sweeps, bool project) {
         LAUNCH_CHECK();
         return GFC_OK;
     }
+    if (j->own) return project ? reunit_g(j, s, false, 0, 2) : GFC_OK;
     const int ns = j->geom.ns, ncol = ns * ns * j->geom.nt;
     hipLaunchKernelGGL(gfc::k_frame_end, dim3((ncol + 63) / 64), dim3(64), 0, s, j->cfg, j->g, ns,
                        j->Vh, ncol, project);
@@ -589,31 +607,44 @@ int lane_count(const gfc_job *j, const gfc_options &o, bool fp32) {
     return gfc_ctx::kLanes;
 }
 
+template <typename T, bool POUT, bool STREAM, bool PIN>
+void launch_sweep_frame(const cplx<T> *u0, cplx<T> *g, hipStream_t s, const gfc::Extents &x, int p,
+                        T omega, int hits, int h0, int count, bool own) {
+    const dim3 b(nblocks(count));
+    if constexpr (sizeof(T) == sizeof(double))
+        if (own) {
+            hipLaunchKernelGGL((gfc::k_sweep<T, POUT, STREAM, PIN, true>), b, dim3(kBlock), 0, s,
+                               u0, g, p, omega, hits, h0, count, x);
+            return;
+        }
+    hipLaunchKernelGGL((gfc::k_sweep<T, POUT, STREAM, PIN>), b, dim3(kBlock), 0, s, u0, g, p,
+                       omega, hits, h0, count, x);
+}
+
 template <typename T, bool POUT, bool STREAM>
 void launch_sweep_pin(const cplx<T> *u0, cplx<T> *g, hipStream_t s, const gfc::Extents &x, int p,
-                      T omega, int hits, int h0, int count, bool pin) {
-    const unsigned b = nblocks(count);
+                      T omega, int hits, int h0, int count, bool pin, bool own) {
     if (pin)
-        hipLaunchKernelGGL((gfc::k_sweep<T, POUT, STREAM, true>), dim3(b), dim3(kBlock), 0, s,
-                           u0, g, p, omega, hits, h0, count, x);
+        launch_sweep_frame<T, POUT, STREAM, true>(u0, g, s, x, p, omega, hits, h0, count, own);
     else
-        hipLaunchKernelGGL((gfc::k_sweep<T, POUT, STREAM, false>), dim3(b), dim3(kBlock), 0, s,
-                           u0, g, p, omega, hits, h0, count, x);
+        launch_sweep_frame<T, POUT, STREAM, false>(u0, g, s, x, p, omega, hits, h0, count, own);
 }
 
 // A half-sweep launch: pout projects the swept parity's new G on output, pin
-// its G on input (see sweep_site), stream selects non-temporal loads.
+// its G on input (see sweep_site), stream selects non-temporal loads, own the
+// configuration's own frame in FP64.
 template <typename T>
 int launch_sweep(const cplx<T> *u0, cplx<T> *g, hipStream_t s, const gfc::Extents &x, int p,
-                 T omega, int hits, int h0, int count, bool pout, bool stream, bool pin = false) {
+                 T omega, int hits, int h0, int count, bool own, bool pout, bool stream,
+                 bool pin = false) {
     if (pout && stream)
-        launch_sweep_pin<T, true, true>(u0, g, s, x, p, omega, hits, h0, count, pin);
+        launch_sweep_pin<T, true, true>(u0, g, s, x, p, omega, hits, h0, count, pin, own);
     else if (pout)
-        launch_sweep_pin<T, true, false>(u0, g, s, x, p, omega, hits, h0, count, pin);
+        launch_sweep_pin<T, true, false>(u0, g, s, x, p, omega, hits, h0, count, pin, own);
     else if (stream)
-        launch_sweep_pin<T, false, true>(u0, g, s, x, p, omega, hits, h0, count, pin);
+        launch_sweep_pin<T, false, true>(u0, g, s, x, p, omega, hits, h0, count, pin, own);
     else
-        launch_sweep_pin<T, false, false>(u0, g, s, x, p, omega, hits, h0, count, pin);
+        launch_sweep_pin<T, false, false>(u0, g, s, x, p, omega, hits, h0, count, pin, own);
     LAUNCH_CHECK();
     return GFC_OK;
 }
@@ -624,8 +655,9 @@ int half_sweep(gfc_job *j, SweepState &st, int parity, double omega, int hits) {
     const gfc::Extents x = gfc::make_extents(j->geom.ns, Vh);
     const bool stream = stream_loads(j, st.fp32, 0, 1);
     if (st.fp32)
-        return launch_sweep(j->u0f, j->gf, s, x, parity, (float)omega, hits, 0, Vh, false, stream);
-    return launch_sweep(j->u0, j->g, s, x, parity, omega, hits, 0, Vh, false, stream);
+        return launch_sweep(j->u0f, j->gf, s, x, parity, (float)omega, hits, 0, Vh, false, false,
+                            stream);
+    return launch_sweep(j->u0, j->g, s, x, parity, omega, hits, 0, Vh, j->own, false, stream);
 }
 
 // Projects G on parities [p0, p0 + np) of the live array.
@@ -699,7 +731,7 @@ constexpr int kSliceSites = 512;
 bool whole_slices(const gfc_job *j, const gfc_options &o, bool fp32) {
     const int ns = j->geom.ns, nt = j->geom.nt;
     const bool lanes = o.slice_lanes >= 1 && o.slice_lanes <= gfc_ctx::kLanes;
-    if (fp32 || o.slice_group != 0 || lanes || ns > 10) return false;
+    if (fp32 || j->own || o.slice_group != 0 || lanes || ns > 10) return false;
     if (ns == 10) return nt >= 1024 || (nt <= 256 && j->Vh > kOneGroup);
     return ns == 8 || nt <= (ns == 4 ? 512 : 256);
 }
@@ -769,10 +801,10 @@ int sweep_blocked(gfc_job *j, const StreamSet &ss, bool fp32, int from, int to, 
                     const int count = (t0 + group <= nt ? group : nt - t0) * S;
                     if (fp32)
                         RC_TRY(launch_sweep(j->u0f, j->gf, s, x, k & 1, (float)omega, hits,
-                                            h0, count, pout, stream, pin));
+                                            h0, count, false, pout, stream, pin));
                     else
                         RC_TRY(launch_sweep(j->u0, j->g, s, x, k & 1, omega, hits, h0,
-                                            count, pout, stream, pin));
+                                            count, j->own, pout, stream, pin));
                 }
             }
         }
@@ -919,6 +951,14 @@ struct SliceTracker {
         hipStream_t s = j->ctx->stream;
         slice_sweeps += (double)n_active / nt;
         if (n_active == 0) return GFC_OK;
+        if (j->own && !fp32) {  // not in the batched kernel
+            const gfc::Extents x = gfc::make_extents(j->geom.ns, j->Vh);
+            for (int t = 0; t < nt; t++)
+                if (active[t])
+                    RC_TRY(launch_sweep(j->u0, j->g, s, x, p, omega, hits, t * S, S, true, false,
+                                        stream_loads(j, false, 0, 1)));
+            return GFC_OK;
+        }
         if (dirty || desc_fp32 != fp32) {
             gfc::BatchJob b{};
             b.u0 = fp32 ? (const void *)j->u0f : (const void *)j->u0;
@@ -1037,8 +1077,19 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
     TraceSums sums(j, which, trace);
     if (trace && trace_len > 0) RC_TRY(sums.init());
 
-    RC_TRY(begin_fix(j, j->ctx->stream, st.fp32));
-    RC_TRY(obs_factored(j, st.fp32, ob));
+    int *off = j->ctx->off_su3();
+    *off = 0;
+    j->own = false;
+    if (st.fp32) {
+        RC_TRY(begin_fix(j, j->ctx->stream, true, off));
+        RC_TRY(obs_factored(j, true, ob));
+        j->own = *off != 0;
+    } else {
+        RC_TRY(obs_aos(j, ob, off));
+        j->own = *off != 0;
+        RC_TRY(begin_fix(j, j->ctx->stream, false, nullptr));
+        if (j->own) RC_TRY(obs_factored(j, false, ob));
+    }
     r.residue_evals++;
     double res = ob[which];
     r.residue_initial = res;
@@ -1329,8 +1380,8 @@ extern "C" int gfc_config_observables_noalloc(gfc_ctx *ctx, const gfc_geom *g,
     const cplx<double> *cfg = reinterpret_cast<const cplx<double> *>(U_dev);
     // the same kernels and block decomposition as gfc_job_observables and
     // gfc_job_plaquette, with the partials and sums in the scratch
-    hipLaunchKernelGGL(gfc::k_obs_aos, dim3(b), dim3(kBlock), 0, s, cfg, g->ns, V,
-                       gfc::aos_groups(V), ptr);
+    hipLaunchKernelGGL(gfc::k_obs_aos<>, dim3(b), dim3(kBlock), 0, s, cfg, g->ns, V,
+                       gfc::aos_groups(V), ptr, nullptr);
     LAUNCH_CHECK();
     hipLaunchKernelGGL(gfc::k_reduce_final, dim3(1), dim3(kBlock), 0, s, ptr, (int)b,
                        ptr + kNoallocOut);

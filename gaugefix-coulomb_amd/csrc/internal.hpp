@@ -52,6 +52,8 @@ struct gfc_ctx {
     double *part = nullptr;  // per-block partial sums
     size_t part_cap = 0;     // in blocks
     double *res_host = nullptr;  // pinned, 8 doubles
+    // ... the last one as the flag of links that are not near SU(3)
+    int *off_su3() { return reinterpret_cast<int *>(res_host + 7); }
     int *flag_dev = nullptr;
     // extra streams (default priority) over which independent timeslice
     // groups are spread, and the events that fork them from and join them
@@ -83,6 +85,9 @@ struct gfc_job {
     gfc::cplx<float> *u0f = nullptr;     // SoA spatial links, FP32 (MIXED)
     gfc::cplx<float> *gf = nullptr;      // SoA G, FP32 (MIXED)
     gfc::cplx<double> *saved = nullptr;  // gfc_job_save_config copy of cfg
+    // the FP64 u0 and G of the fix under way are in the configuration's own
+    // frame, not in the axial one
+    bool own = false;
 };
 
 namespace gfcx {
@@ -91,7 +96,7 @@ namespace gfcx {
 // stream, or on j->ctx->stream without one.
 int set_identity(gfc_job *j);
 int set_identity(gfc_job *j, hipStream_t s);
-int begin_fix(gfc_job *j, hipStream_t s, bool mixed);
+int begin_fix(gfc_job *j, hipStream_t s, bool mixed, int *off);
 int end_frame(gfc_job *j, hipStream_t s, bool fp32, int sweeps, bool project);
 int materialize(gfc_job *j, bool project);
 int materialize(gfc_job *j, hipStream_t s, bool project);

@@ -567,11 +567,12 @@ __device__ __forceinline__ void sweep_axial(const cplx<double> *__restrict__ u0,
     store_su3<true>(out, gp, h);
 }
 
-template <typename T, bool POUT = false, bool STREAM = true, bool PIN = false>
+// OWN: FP64 too in the configuration's own frame.
+template <typename T, bool POUT = false, bool STREAM = true, bool PIN = false, bool OWN = false>
 __device__ __forceinline__ void sweep_site(const cplx<T> *__restrict__ u0,
                                            cplx<T> *__restrict__ g, const Extents &x, int p,
                                            T omega, int hits, int first, int lane) {
-    if constexpr (sizeof(T) == sizeof(double))
+    if constexpr (sizeof(T) == sizeof(double) && !OWN)
         sweep_axial<POUT, STREAM, PIN>(u0, g, x, p, omega, hits, first, lane);
     else
         sweep_own<T, POUT, STREAM, PIN>(u0, g, x.ns, x.Vh, p, omega, hits, first + lane);
@@ -603,7 +604,7 @@ __device__ __forceinline__ unsigned xcd_order(unsigned i, unsigned n) {
 // first 64 bytes, and the number of workgroups is computed rather than read from
 // behind them (FP32, us per half-sweep: 8^3 x 16 7.5 -> 7.2, 16^3 x 32 7.65 ->
 // 7.35).
-template <typename T, bool POUT = false, bool STREAM = true, bool PIN = false>
+template <typename T, bool POUT = false, bool STREAM = true, bool PIN = false, bool OWN = false>
 __global__ __launch_bounds__(kBlock) void k_sweep(const cplx<T> *__restrict__ u0,
                                                   cplx<T> *__restrict__ g, int p, T omega,
                                                   int hits, int h0, int count, Extents x) {
@@ -611,7 +612,7 @@ __global__ __launch_bounds__(kBlock) void k_sweep(const cplx<T> *__restrict__ u0
     const unsigned b = STREAM ? blockIdx.x : xcd_order(blockIdx.x, nb);
     const int lane = (int)threadIdx.x;
     if ((int)(b * kBlock) + lane >= count) return;
-    sweep_site<T, POUT, STREAM, PIN>(u0, g, x, p, omega, hits, h0 + (int)(b * kBlock), lane);
+    sweep_site<T, POUT, STREAM, PIN, OWN>(u0, g, x, p, omega, hits, h0 + (int)(b * kBlock), lane);
 }
 
 // Half-sweeps [from, to) of a small lattice in FP64, one workgroup per
@@ -898,12 +899,34 @@ __global__ __launch_bounds__(kBlock) void k_axial_u0(const cplx<double> *__restr
     }
 }
 
-// cfg (AoS FP64) spatial links -> u0 fields in FP64 and FP32 in the
-// configuration's own frame, for the FP32 phase of a mixed fix.
+// Whether a matrix is one of SU(3) to within 1e-6, some ten times what storing
+// it in FP32 makes of it.  The axial frame multiplies links up a column and
+// keeps the nearest SU(3) matrices; links further off are swept in the
+// configuration's own frame, where each stands for itself, as its first two
+// rows.  (No number is not near.)
+__device__ __forceinline__ bool near_su3(const mat3<double> &u) {
+    mat3<double> c = u;
+    m_fill_row2(c);
+    cplx<double> s = c_make<double>(0, 0);
+    double d = fmax(fabs(row_norm(u.e) - 1), fabs(row_norm(u.e + 3) - 1));
+    bool ok = true;
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+        c_mac_cb(s, u.e[b], u.e[3 + b]);
+        const cplx<double> r = c_make<double>(u.e[6 + b].re - c.e[6 + b].re,
+                                              u.e[6 + b].im - c.e[6 + b].im);
+        ok = ok && fabs(r.re) < 1e-6 && fabs(r.im) < 1e-6;
+    }
+    return ok && d < 1e-6 && fabs(s.re) < 1e-6 && fabs(s.im) < 1e-6;
+}
+
+// cfg (AoS FP64) spatial links -> u0 fields in FP64 and, unless u0f is null,
+// FP32 in the configuration's own frame; *off, if given, is set to 1 when a
+// link is not near SU(3).
 __global__ __launch_bounds__(kBlock) void k_build_u0(const cplx<double> *__restrict__ cfg,
                                                      cplx<double> *__restrict__ u0,
                                                      cplx<float> *__restrict__ u0f, int ns,
-                                                     int Vh) {
+                                                     int Vh, int *off) {
     const int idx = blockIdx.x * kBlock + threadIdx.x;
     if (idx >= 2 * Vh) return;
     const int p = idx >= Vh, h = idx - p * Vh;
@@ -914,9 +937,10 @@ __global__ __launch_bounds__(kBlock) void k_build_u0(const cplx<double> *__restr
         const cplx<double> *src = cfg + (lex * 4 + 1 + i) * 9;
         mat3<double> m;
 #pragma unroll
-        for (int k = 0; k < kPlanes; k++) m.e[k] = src[k];
+        for (int k = 0; k < 9; k++) m.e[k] = src[k];
+        if (off && !near_su3(m)) *off = 1;
         store_u0(m, u0_field(u0, Vh, p, i), h);
-        store_u0(m, u0_field(u0f, Vh, p, i), h);
+        if (u0f) store_u0(m, u0_field(u0f, Vh, p, i), h);
     }
 }
 
@@ -1146,7 +1170,7 @@ __device__ __forceinline__ void block_reduce3(Obs o, double *__restrict__ part, 
 }
 
 // Observables of the factored state at site index idx in [0, 2 Vh) (parity
-// idx >= Vh); u0 in FP64 (in the axial frame with an FP64 G, in the
+// idx >= Vh); u0 in FP64 (in the axial frame with an FP64 G unless OWN, in the
 // configuration's own with an FP32 one), arithmetic in FP64.  They come
 // from the site's w = G(n) W(n), formed as the sweep forms it:
 // w = sum_i [U_i(n) + U_i(n-i)^dagger], so w - w^dagger is the divergence
@@ -1155,7 +1179,7 @@ __device__ __forceinline__ void block_reduce3(Obs o, double *__restrict__ part, 
 // Re Tr w / 2 summed over all sites is the sum over links of Re Tr U that F
 // measures (calculateF, src/gauge_fixing.c).  Seven products (five in the axial
 // frame) instead of the twelve of forming every link.
-template <typename TG>
+template <typename TG, bool OWN = false>
 __device__ __forceinline__ Obs obs_site(const cplx<double> *__restrict__ u0,
                                         const cplx<TG> *__restrict__ g, int ns, int Vh,
                                         int idx) {
@@ -1167,7 +1191,7 @@ __device__ __forceinline__ Obs obs_site(const cplx<double> *__restrict__ u0,
         const cplx<TG> *gq = g_field(g, Vh, 1 - p);
         mat3<double> W;
         m_zero(W);
-        constexpr bool axial = sizeof(TG) == sizeof(double);
+        constexpr bool axial = sizeof(TG) == sizeof(double) && !OWN;
         if constexpr (axial) {
             mat3<double> gf, gb;
             load_su3_d(gf, gq, nb.fwd[0]);
@@ -1213,14 +1237,14 @@ __host__ __device__ inline unsigned parity_order(unsigned b, unsigned n) {
 // site order.  The workgroups run in XCD-contiguous order (xcd_order), so that
 // the neighbour G and backward u0 links a site reads were mostly brought into
 // its XCD's L2 by the sites next to it.
-template <typename TG>
+template <typename TG, bool OWN = false>
 __global__ __launch_bounds__(kBlock, 3) void k_obs_factored(const cplx<double> *__restrict__ u0,
                                                             const cplx<TG> *__restrict__ g,
                                                             int ns, int Vh,
                                                             double *__restrict__ part) {
     const unsigned b = parity_order(xcd_order(blockIdx.x, gridDim.x), gridDim.x);
     const int idx = (int)(b * kBlock + threadIdx.x);
-    block_reduce3(obs_site<TG>(u0, g, ns, Vh, idx), part, b);
+    block_reduce3(obs_site<TG, OWN>(u0, g, ns, Vh, idx), part, b);
 }
 
 // The sums of each timeslice t (one workgroup), out[3 t + j]: partials
@@ -1301,10 +1325,12 @@ __device__ __forceinline__ int aos_neighbour(int lex, int mu, bool fwd, int ns, 
 }
 
 // Observables of an AoS FP64 configuration.  Thread i (1 to 3) of a site adds
-// its direction's U_i(n) - U_i(n-i); thread 0 takes the sum.
+// its direction's U_i(n) - U_i(n-i); thread 0 takes the sum.  With CHECK, *off
+// is set to 1 when a spatial link is not near SU(3).
+template <bool CHECK = false>
 __global__ __launch_bounds__(kBlock) void k_obs_aos(const cplx<double> *__restrict__ cfg, int ns,
                                                     int64_t V, int groups,
-                                                    double *__restrict__ part) {
+                                                    double *__restrict__ part, int *off) {
     __shared__ double2 tile[kAosSites * 27];
     __shared__ int nbr[kAosSites * 3];
     const double2 *src = reinterpret_cast<const double2 *>(cfg);
@@ -1321,7 +1347,10 @@ __global__ __launch_bounds__(kBlock) void k_obs_aos(const cplx<double> *__restri
         if (on) nbr[site * 3 + i - 1] = aos_neighbour(lex0 + site, i, false, ns, 1 << 30);
         stage_tile<27>(tile, src, count * 27,
                        [&](int k) { return (int64_t)lex0 * 36 + 9 + k + k / 27 * 9; });
-        if (on) lds_mat(u, mine);
+        if (on) {
+            lds_mat(u, mine);
+            if (CHECK && !near_su3(u)) *off = 1;
+        }
         __syncthreads();
         stage_tile<27>(tile, src, count * 27,
                        [&](int k) { return (int64_t)nbr[k / 9] * 36 + 9 + k % 27; });

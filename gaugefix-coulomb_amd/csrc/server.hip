@@ -273,7 +273,8 @@ int admit_one(gfc_server *s, Lane &L, Req &r, bool &admitted) {
                        job->cfg, job->V * 4, L.d_flags + slot);
     LAUNCH_CHECK();
     r.fp32 = r.o.precision == GFC_PREC_MIXED;
-    RC_TRY(gfcx::begin_fix(job, L.st, r.fp32));
+    job->own = false;
+    RC_TRY(gfcx::begin_fix(job, L.st, r.fp32, nullptr));
     r.state = INIT;
     r.t_admit = s->clock();
     fill_desc(L, r);

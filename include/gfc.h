@@ -242,7 +242,13 @@ int gfc_job_plaquette(gfc_job *job, double *spatial, double *temporal);
  * overrelaxation sweeps with the reference's check schedule, stall test,
  * max-sweeps test and reunitarization every sweeps_to_reunitarization
  * sweeps; U and G are left gauge-fixed on the device.  Returns the sweep
- * count, GFC_ENOTCONVERGED or GFC_EPARAMS (or a device error). */
+ * count, GFC_ENOTCONVERGED or GFC_EPARAMS (or a device error; G is then 1).
+ * The links are meant to be SU(3): gfc_job_reunitarize first.  FP64 sweeps
+ * multiply them up the Z columns and keep the nearest SU(3) matrices, also of
+ * links rounded to FP32.  When a spatial link is further than 1e-6 from SU(3)
+ * (the norms and overlap of its first two rows, its third row) each link is
+ * taken for itself, by its first two rows alone (an FP64 link by row 0 and two
+ * elements of row 1, the rest from unitarity), and the sweeps are slower. */
 int gfc_job_fix(gfc_job *job, const gfc_params *p, const gfc_options *o, gfc_report *rep);
 /* gfc_job_fix that also stores the proxy measured after each half-sweep k
  * (before that sweep's reunitarization) in trace[k-1], for k <= trace_len.
@@ -280,10 +286,8 @@ int gfc_job_write_config(gfc_job *job, const char *path, int out_precision, int 
 /* The drop-in entry point: gaugefixOverrelaxation(U, G, params) on host
  * arrays (include/gauge_fixing.h:67-69).  U (4*V*18 doubles) and G (V*18
  * doubles) are updated in place with the same return codes.  o and rep may
- * be NULL.  U must hold SU(3) links, as the reference's main leaves them
- * (reunitarizeField before the call, gauge_fix_coulomb.c:126): the engine
- * keeps each link as its first two rows (an FP64 link as row 0 and two
- * elements of row 1) and rebuilds the rest from unitarity. */
+ * be NULL.  U must hold SU(3) links (see gfc_job_fix), as the reference's main
+ * leaves them (reunitarizeField before the call, gauge_fix_coulomb.c:126). */
 int gfc_fix_coulomb_or(gfc_ctx *ctx, const gfc_geom *g, const gfc_params *p,
                        const gfc_options *o, double *U, double *G, gfc_report *rep);
 /* reunitarizeField (src/fields.c:144-187) on a host array of n matrices. */
