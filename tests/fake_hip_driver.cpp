@@ -229,7 +229,8 @@ int main(int argc, char **argv) {
         round_trip(c, {(int)arg(2), (int)arg(3)}, arg(4) != 0, arg(5) != 0);
     } else if (what == "fix") {
         // fix ns nt precision sweeps hits slice_group slice_lanes retire done:
-        // the launch of half-sweep done + 1 fails if done is given
+        // the launch of half-sweep done + 1 fails if done is given; without
+        // sweeps, the tolerance is one that the input meets
         gfc_geom g = {(int)arg(2), (int)arg(3)};
         gfc_params p;
         gfc_params_default(&p);
@@ -237,6 +238,7 @@ int main(int argc, char **argv) {
         p.estimate_sweeps_to_gf_progress = 100000000;
         p.max_sweeps_to_fix = (unsigned)arg(5);
         p.hits = (unsigned)arg(6);
+        if (arg(5) == 0) p.tolerance = 1e9;
         gfc_options o;
         gfc_options_default(&o);
         o.precision = (int)arg(4);

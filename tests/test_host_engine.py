@@ -133,3 +133,13 @@ def test_failed_fix_leaves_the_identity(driver, ns, prec, retire, rc, why):
     first, *log = driver("fix", ns, 4, prec, 20, 2, 0, 0, retire, 7)
     assert first == f"fix {rc} sweeps 0 message [{why}]"
     assert "k_g_identity" in [l for l in log if l.startswith("launch")][-1]
+
+
+def test_fixed_configuration_costs_no_frame(driver):
+    """An FP64 fix whose input meets the tolerance looks at it, writes G = 1 and
+    U, and builds nothing for sweeps."""
+    first, *log = driver("fix", 16, 4, 0, 0, 2, 0, 0)
+    assert first == "fix 0 sweeps 0 message []"
+    names = [l.split()[1] for l in log if l.startswith("launch")]
+    kernels = ("k_obs_aos", "k_reduce_final", "k_g_identity", "k_materialize")
+    assert len(names) == 4 and all(k in n for k, n in zip(kernels, names))
