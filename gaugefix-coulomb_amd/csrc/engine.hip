@@ -231,12 +231,11 @@ int64_t gfc_job_footprint(const gfc_geom *g, int precision) {
     const int64_t V = gfc_geom_volume(g);
     // G keeps two rows (6 complex numbers) per SU(3) matrix, in fields of
     // whole 32-site tiles per parity; the u0 fields are allocated at the same
-    // size per direction (FP64 u0 uses five numbers of them; the allocation
-    // also stages FP32 input)
+    // size per direction
     const int64_t fs = gfc::field_size(V / 2);
-    int64_t b = V * 4 * 144       // cfg
-                + 6 * fs * 16     // u0
-                + 2 * fs * 16;    // g
+    int64_t b = V * 4 * 144                                // cfg
+                + gfc::u0_alloc_size(V / 2, g->ns) * 16    // u0
+                + 2 * fs * 16;                             // g
     if (precision == GFC_PREC_MIXED) b += 6 * fs * 8 + 2 * fs * 8;
     return b;
 }
@@ -305,7 +304,8 @@ extern "C" int gfc_job_create(gfc_ctx *ctx, const gfc_geom *g, int precision, gf
     j->precision = precision;
     hipError_t e = hipMalloc(&j->cfg, (size_t)V * 4 * 9 * sizeof(cplx<double>));
     const size_t fs = (size_t)gfc::field_size(j->Vh);  // per parity and direction
-    if (e == hipSuccess) e = hipMalloc(&j->u0, 6 * fs * sizeof(cplx<double>));
+    if (e == hipSuccess)
+        e = hipMalloc(&j->u0, (size_t)gfc::u0_alloc_size(j->Vh, g->ns) * sizeof(cplx<double>));
     if (e == hipSuccess) e = hipMalloc(&j->g, 2 * fs * sizeof(cplx<double>));
     if (e == hipSuccess && precision == GFC_PREC_MIXED) {
         e = hipMalloc(&j->u0f, 6 * fs * sizeof(cplx<float>));
@@ -524,9 +524,8 @@ int end_frame(gfc_job *j, hipStream_t s, bool fp32, int sweeps, bool project) {
         return GFC_OK;
     }
     if (j->own) return project ? reunit_g(j, s, false, 0, 2) : GFC_OK;
-    const int ns = j->geom.ns, ncol = ns * ns * j->geom.nt;
-    hipLaunchKernelGGL(gfc::k_frame_end, dim3((ncol + 63) / 64), dim3(64), 0, s, j->cfg, j->g, ns,
-                       j->Vh, ncol, project);
+    hipLaunchKernelGGL(gfc::k_frame_end, dim3(nblocks(2 * (int64_t)j->Vh)), dim3(kBlock), 0, s,
+                       j->u0, j->g, j->geom.ns, j->Vh, project);
     LAUNCH_CHECK();
     return GFC_OK;
 }

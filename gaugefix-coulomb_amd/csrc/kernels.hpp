@@ -156,9 +156,9 @@ __device__ __forceinline__ cplx<T> *u0_field(cplx<T> *u0, int Vh, int p, int i) 
     return u0 + (p * 3 + i) * u0_field_size<T>(Vh);
 }
 // In the axial frame: field of the links u0_i on parity p, i = 1 (Y), 2 (X);
-// and of the Z links of the plane z = ns - 1 on parity p, by their index in
-// the plane, t ns^2/2 + y ns/2 + x/2 (Vh / ns sites).  Together at most 30 of
-// the allocation's 36 planes of Vh numbers.
+// of the Z links of the plane z = ns - 1 on parity p, by their index in the
+// plane, t ns^2/2 + y ns/2 + x/2 (Vh / ns sites); and of h^dagger on parity p,
+// kept for the way out of the frame.
 template <typename C>
 __device__ __forceinline__ C *axial_field(C *u0, int Vh, int p, int i) {
     return u0 + (p * 2 + i - 1) * u0_field_size<double>(Vh);
@@ -166,6 +166,20 @@ __device__ __forceinline__ C *axial_field(C *u0, int Vh, int p, int i) {
 template <typename C>
 __device__ __forceinline__ C *axial_wrap(C *u0, int Vh, int ns, int p) {
     return u0 + 4 * u0_field_size<double>(Vh) + p * u0_field_size<double>(Vh / ns);
+}
+template <typename C>
+__device__ __forceinline__ C *axial_h(C *u0, int Vh, int ns, int p) {
+    return axial_wrap(u0, Vh, ns, 2) + p * field_size(Vh);
+}
+// Numbers of the u0 allocation: the six fields of links in the configuration's
+// frame at six planes each (which also stage FP32 input), or those of the axial
+// frame, 32 to 37 planes of Vh numbers (more than 36 for ns = 2 and lattices
+// of a few tiles).
+__host__ __device__ constexpr int64_t u0_alloc_size(int64_t Vh, int ns) {
+    const int64_t own = 6 * field_size(Vh);
+    const int64_t axial = 4 * u0_field_size<double>(Vh) + 2 * u0_field_size<double>(Vh / ns) +
+                          2 * field_size(Vh);
+    return own > axial ? own : axial;
 }
 template <typename T>
 __device__ __forceinline__ const cplx<T> *g_field(const cplx<T> *g, int Vh, int p) {
@@ -847,31 +861,32 @@ __global__ __launch_bounds__(64) void k_frame_begin(const cplx<double> *__restri
 }
 
 // End of a fix: G = G' h, projected onto SU(3) if `project` (the last
-// reunitarization of G).
-__global__ __launch_bounds__(64) void k_frame_end(const cplx<double> *__restrict__ cfg,
-                                                  cplx<double> *__restrict__ g, int ns, int Vh,
-                                                  int ncol, bool project) {
-    const int c = blockIdx.x * 64 + threadIdx.x;
-    if (c >= ncol) return;
-    const Column q = column_of(c, ns);
-    walk_column(cfg, ns, q.lex0, [&](int z, const mat3<double> &d) {
-        cplx<double> *field = g_field(g, Vh, (q.x + q.y + z + q.t) & 1);
-        const int h = (int)((q.lex0 + (int64_t)z * ns * ns) >> 1);
-        mat3<double> gp, zero, out, lo;
-        m_zero(zero);
-        load_su3<false>(gp, static_cast<const cplx<double> *>(field), h);
-        m_mul2<2>(gp, zero, m_dagger(d), out, lo);
+// reunitarization of G).  One thread per site; bound by its three matrices.
+__global__ __launch_bounds__(kBlock) void k_frame_end(const cplx<double> *__restrict__ u0,
+                                                      cplx<double> *__restrict__ g, int ns,
+                                                      int Vh, bool project) {
+    const int idx = blockIdx.x * kBlock + threadIdx.x;
+    if (idx >= 2 * Vh) return;
+    const int p = idx >= Vh, h = idx - p * Vh;
+    cplx<double> *field = g_field(g, Vh, p);
+    mat3<double> gp, d, zero, out, lo;
+    m_zero(zero);
+    load_su3<false>(gp, static_cast<const cplx<double> *>(field), h);
+    load_rows01<false>(d, axial_h(u0, Vh, ns, p), h);
+    m_close_row2(d);
+    m_mul2<2>(gp, zero, m_dagger(d), out, lo);
 #pragma unroll
-        for (int k = 0; k < kPlanes; k++)
-            out.e[k] = c_make<double>(out.e[k].re + lo.e[k].re, out.e[k].im + lo.e[k].im);
-        if (project) m_project_su3(out);
-        store_su3<false>(out, field, h);
-    });
+    for (int k = 0; k < kPlanes; k++)
+        out.e[k] = c_make<double>(out.e[k].re + lo.e[k].re, out.e[k].im + lo.e[k].im);
+    if (project) m_project_su3(out);
+    store_su3<false>(out, field, h);
 }
 
 // The Y and X links of cfg (AoS FP64) in the axial frame, u0_i(n) =
-// h(n) u_i(n) h(n+i)^dagger with h = G'^dagger (k_frame_begin).  One thread per
-// site.
+// h(n) u_i(n) h(n+i)^dagger with h = G'^dagger (k_frame_begin), and h^dagger for
+// k_frame_end, which walked the columns a second time before (a fix of one
+// half-sweep at 8^3 x 16 / 16^3 x 32 / 48^3 x 96: 114 -> 83, 226 -> 163, 7840 ->
+// 7400 us).  One thread per site.
 __global__ __launch_bounds__(kBlock) void k_axial_u0(const cplx<double> *__restrict__ cfg,
                                                      const cplx<double> *__restrict__ g,
                                                      cplx<double> *__restrict__ u0, int ns,
@@ -884,6 +899,7 @@ __global__ __launch_bounds__(kBlock) void k_axial_u0(const cplx<double> *__restr
     const int64_t lex = (int64_t)2 * s.row + s.x;
     mat3<double> gn;
     load_su3<false>(gn, g_field(g, Vh, p), h);
+    store_su3<true>(gn, axial_h(u0, Vh, ns, p), h);
 #pragma unroll
     for (int i = 1; i < 3; i++) {
         const cplx<double> *src = cfg + (lex * 4 + 1 + i) * 9;

@@ -371,6 +371,19 @@ __device__ __forceinline__ void m_mul2(const mat3<double> &a, const mat3<double>
         }
 }
 
+// Row 2 = conj(r0 x r1), each element rounded once.
+__device__ __forceinline__ void m_close_row2(mat3<double> &o) {
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+        const cplx<double> x0 = o.e[(b + 1) % 3], x1 = o.e[3 + (b + 2) % 3];
+        const cplx<double> y0 = o.e[(b + 2) % 3], y1 = o.e[3 + (b + 1) % 3];
+        sum2 re = {0, 0}, im = {0, 0};
+        s2_cmac(re, im, x0, x1);
+        s2_cmac(re, im, c_make<double>(-y0.re, -y0.im), y1);
+        o.e[6 + b] = c_make<double>(re.hi + re.lo, -(im.hi + im.lo));
+    }
+}
+
 // The SU(3) matrix nearest hi + lo, whose rows 0 and 1 are orthonormal to
 // within some roundings, rounded once: first-order corrections of the rows'
 // norms and overlap from compensated sums, row 2 = conj(r0 x r1).  Matrices
@@ -410,15 +423,7 @@ __device__ __forceinline__ void m_polish_su3(const mat3<double> &hi, const mat3<
         o.e[b] = c_make<double>(r0[b].re + k0.re, r0[b].im + k0.im);
         o.e[3 + b] = c_make<double>(r1[b].re + k1.re, r1[b].im + k1.im);
     }
-#pragma unroll
-    for (int b = 0; b < 3; b++) {
-        const cplx<double> x0 = o.e[(b + 1) % 3], x1 = o.e[3 + (b + 2) % 3];
-        const cplx<double> y0 = o.e[(b + 2) % 3], y1 = o.e[3 + (b + 1) % 3];
-        sum2 re = {0, 0}, im = {0, 0};
-        s2_cmac(re, im, x0, x1);
-        s2_cmac(re, im, c_make<double>(-y0.re, -y0.im), y1);
-        o.e[6 + b] = c_make<double>(re.hi + re.lo, -(im.hi + im.lo));
-    }
+    m_close_row2(o);
     m = o;
 }
 

@@ -143,3 +143,11 @@ def test_fixed_configuration_costs_no_frame(driver):
     names = [l.split()[1] for l in log if l.startswith("launch")]
     kernels = ("k_obs_aos", "k_reduce_final", "k_g_identity", "k_materialize")
     assert len(names) == 4 and all(k in n for k, n in zip(kernels, names))
+
+
+def test_the_columns_are_walked_once(driver):
+    """A fix walks the columns on its way into the axial frame (a thread per
+    column) and leaves it site by site."""
+    log = [l.split() for l in _fix(driver, 16, 4) if l.startswith("launch")]
+    assert [l[2:] for l in log if "k_frame_begin" in l[1]] == [["16", "64"]]
+    assert [l[2:] for l in log if "k_frame_end" in l[1]] == [["64", "256"]]
