@@ -1238,7 +1238,7 @@ extern "C" int gfc_job_plaquette(gfc_job *j, double *spatial, double *temporal) 
     HIP_TRY(hipSetDevice(j->ctx->device));
     gfc_ctx *c = j->ctx;
     const unsigned b = gfc::aos_blocks(j->V);
-    hipLaunchKernelGGL(gfc::k_plaquette_aos, dim3(b), dim3(kBlock), 0, c->stream, j->cfg,
+    hipLaunchKernelGGL(gfc::k_plaquette_aos<>, dim3(b), dim3(kBlock), 0, c->stream, j->cfg,
                        j->geom.ns, j->geom.nt, j->V, gfc::aos_groups(j->V), c->part);
     LAUNCH_CHECK();
     double s[3];
@@ -1381,15 +1381,26 @@ extern "C" int gfc_config_observables_noalloc(gfc_ctx *ctx, const gfc_geom *g,
     hipStream_t s = ctx->stream;
     const cplx<double> *cfg = reinterpret_cast<const cplx<double> *>(U_dev);
     // the same kernels and block decomposition as gfc_job_observables and
-    // gfc_job_plaquette, with the partials and sums in the scratch
-    hipLaunchKernelGGL(gfc::k_obs_aos<>, dim3(b), dim3(kBlock), 0, s, cfg, g->ns, V,
-                       gfc::aos_groups(V), ptr, nullptr);
+    // gfc_job_plaquette, with the partials and sums in the scratch; a caller's
+    // array may lie at any double's address, and only one at a multiple of 16
+    // bytes can be moved straight to LDS
+    const bool aligned = reinterpret_cast<uintptr_t>(U_dev) % 16 == 0;
+    if (aligned)
+        hipLaunchKernelGGL(gfc::k_obs_aos<>, dim3(b), dim3(kBlock), 0, s, cfg, g->ns, V,
+                           gfc::aos_groups(V), ptr, nullptr);
+    else
+        hipLaunchKernelGGL((gfc::k_obs_aos<false, false>), dim3(b), dim3(kBlock), 0, s, cfg, g->ns,
+                           V, gfc::aos_groups(V), ptr, nullptr);
     LAUNCH_CHECK();
     hipLaunchKernelGGL(gfc::k_reduce_final, dim3(1), dim3(kBlock), 0, s, ptr, (int)b,
                        ptr + kNoallocOut);
     LAUNCH_CHECK();
-    hipLaunchKernelGGL(gfc::k_plaquette_aos, dim3(b), dim3(kBlock), 0, s, cfg, g->ns, g->nt, V,
-                       gfc::aos_groups(V), ptr);
+    if (aligned)
+        hipLaunchKernelGGL(gfc::k_plaquette_aos<>, dim3(b), dim3(kBlock), 0, s, cfg, g->ns, g->nt,
+                           V, gfc::aos_groups(V), ptr);
+    else
+        hipLaunchKernelGGL(gfc::k_plaquette_aos<false>, dim3(b), dim3(kBlock), 0, s, cfg, g->ns,
+                           g->nt, V, gfc::aos_groups(V), ptr);
     LAUNCH_CHECK();
     hipLaunchKernelGGL(gfc::k_reduce_final, dim3(1), dim3(kBlock), 0, s, ptr, (int)b,
                        ptr + kNoallocOut + 3);

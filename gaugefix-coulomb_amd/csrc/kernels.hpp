@@ -964,8 +964,10 @@ __global__ __launch_bounds__(kBlock) void k_build_u0(const cplx<double> *__restr
 // straight to LDS, 64 pieces by a wave's load, all of them in flight together
 // (through registers, a piece at a time, they arrived one after the other:
 // 4.6 instead of 3.3 ms for the plaquettes of 48^3 x 96).  Pieces from n on get
-// src[at(0)].  Complete on return; the tile must have been read before.
-template <int P, typename At>
+// src[at(0)].  Complete on return; the tile must have been read before.  With
+// ALIGNED = false src need only lie at a double's alignment, and its pieces go
+// through registers.
+template <int P, bool ALIGNED = true, typename At>
 __device__ __forceinline__ void stage_tile(double2 *tile, const double2 *src, int n, At at) {
     typedef __attribute__((address_space(3))) void *lds_ptr;
     typedef const __attribute__((address_space(1))) void *global_ptr;
@@ -974,9 +976,14 @@ __device__ __forceinline__ void stage_tile(double2 *tile, const double2 *src, in
 #pragma unroll
     for (int j = 0; j < (P + 3) / 4; j++) {
         const int c = wave + 4 * j, k = c * 64 + ((int)threadIdx.x & 63);
-        if (c < P)
-            __builtin_amdgcn_global_load_lds((global_ptr)(src + at(k < n ? k : 0)),
-                                             (lds_ptr)(tile + c * 64), 16, 0, 0);
+        if (c >= P) continue;
+        const double2 *from = src + at(k < n ? k : 0);
+        if constexpr (ALIGNED) {
+            __builtin_amdgcn_global_load_lds((global_ptr)from, (lds_ptr)(tile + c * 64), 16, 0, 0);
+        } else {
+            const double *d = reinterpret_cast<const double *>(from);
+            tile[k] = double2{d[0], d[1]};
+        }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -1343,7 +1350,7 @@ __device__ __forceinline__ int aos_neighbour(int lex, int mu, bool fwd, int ns, 
 // Observables of an AoS FP64 configuration.  Thread i (1 to 3) of a site adds
 // its direction's U_i(n) - U_i(n-i); thread 0 takes the sum.  With CHECK, *off
 // is set to 1 when a spatial link is not near SU(3).
-template <bool CHECK = false>
+template <bool CHECK = false, bool ALIGNED = true>
 __global__ __launch_bounds__(kBlock) void k_obs_aos(const cplx<double> *__restrict__ cfg, int ns,
                                                     int64_t V, int groups,
                                                     double *__restrict__ part, int *off) {
@@ -1361,15 +1368,15 @@ __global__ __launch_bounds__(kBlock) void k_obs_aos(const cplx<double> *__restri
         const double2 *mine = tile + site * 27 + (i - 1) * 9;
         mat3<double> u, v;
         if (on) nbr[site * 3 + i - 1] = aos_neighbour(lex0 + site, i, false, ns, 1 << 30);
-        stage_tile<27>(tile, src, count * 27,
-                       [&](int k) { return (int64_t)lex0 * 36 + 9 + k + k / 27 * 9; });
+        stage_tile<27, ALIGNED>(tile, src, count * 27,
+                                [&](int k) { return (int64_t)lex0 * 36 + 9 + k + k / 27 * 9; });
         if (on) {
             lds_mat(u, mine);
             if (CHECK && !near_su3(u)) *off = 1;
         }
         __syncthreads();
-        stage_tile<27>(tile, src, count * 27,
-                       [&](int k) { return (int64_t)nbr[k / 9] * 36 + 9 + k % 27; });
+        stage_tile<27, ALIGNED>(tile, src, count * 27,
+                                [&](int k) { return (int64_t)nbr[k / 9] * 36 + 9 + k % 27; });
         // D = sum_i (E_i - E_i^dagger), E_i = U_i(n) - U_i(n-i): the imaginary
         // parts of its diagonal, D01, D02, D12, and Re Tr U
         double d[10];
@@ -1435,6 +1442,7 @@ __device__ __forceinline__ double plaquette_trace(const mat3<double> &a) {
 // (XY, XZ, YZ) into slot 0 and temporal planes (TZ, TY, TX) into slot 1.
 // Thread r of a site meets each other direction d = r ^ X once, X = 1, 2, 3;
 // both threads of a plane find its trace, and each counts half.
+template <bool ALIGNED = true>
 __global__ __launch_bounds__(kBlock) void k_plaquette_aos(const cplx<double> *__restrict__ cfg,
                                                           int ns, int nt, int64_t V, int groups,
                                                           double *__restrict__ part) {
@@ -1449,15 +1457,16 @@ __global__ __launch_bounds__(kBlock) void k_plaquette_aos(const cplx<double> *__
         const int lex0 = aos_group(b, gridDim.x, q, groups), count = min(kAosSites, n - lex0);
         if (count <= 0) break;
         if (site < count) nbr[threadIdx.x] = aos_neighbour(lex0 + site, r, true, ns, nt);
-        stage_tile<36>(tile, src, count * 36, [&](int k) { return (int64_t)lex0 * 36 + k; });
+        stage_tile<36, ALIGNED>(tile, src, count * 36,
+                                [&](int k) { return (int64_t)lex0 * 36 + k; });
         mat3<double> own;  // U_r(n)
         m_zero(own);
         if (site < count) lds_mat(own, tile + threadIdx.x * 9);
 #pragma unroll
         for (int X = 1; X < 4; X++) {
             __syncthreads();  // the tile has been read
-            stage_tile<36>(tile, src, count * 36,
-                           [&](int k) { return (int64_t)nbr[(k / 9) ^ X] * 36 + k % 36; });
+            stage_tile<36, ALIGNED>(tile, src, count * 36,
+                                    [&](int k) { return (int64_t)nbr[(k / 9) ^ X] * 36 + k % 36; });
             mat3<double> u, v, a;
 #pragma unroll
             for (int k = 0; k < 9; k++)

@@ -254,6 +254,16 @@ int main(int argc, char **argv) {
         fake().sweeps_left = -1;
         std::printf("fix %d sweeps %d message [%s]\n", rc, r.sweeps, gfc_last_error());
         gfc_job_destroy(j);
+    } else if (what == "noalloc") {
+        // noalloc offset: a configuration that many bytes behind a multiple of 16
+        gfc_geom g = {4, 4};
+        void *m = std::aligned_alloc(16, 4 * 4 * 4 * 4 * 576 + 16);
+        double o[5];
+        const int rc = gfc_config_observables_noalloc(
+            c, &g, reinterpret_cast<double *>(static_cast<char *>(m) + arg(2)), o, o + 1, o + 2,
+            o + 3, o + 4);
+        std::printf("noalloc %d\n", rc);
+        std::free(m);
     } else if (what == "trace") {
         // trace ns nt sweeps trace_len done: the launch of half-sweep done + 1
         // fails; 8 numbers behind the trace are looked at too

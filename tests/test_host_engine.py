@@ -151,3 +151,14 @@ def test_the_columns_are_walked_once(driver):
     log = [l.split() for l in _fix(driver, 16, 4) if l.startswith("launch")]
     assert [l[2:] for l in log if "k_frame_begin" in l[1]] == [["16", "64"]]
     assert [l[2:] for l in log if "k_frame_end" in l[1]] == [["64", "256"]]
+
+
+@pytest.mark.parametrize("offset", [0, 8])
+def test_loads_by_the_alignment_of_a_callers_array(driver, offset):
+    """16-byte loads straight to LDS only from addresses that allow them."""
+    first, *log = driver("noalloc", offset)
+    assert first == "noalloc 0"
+    names = [l.split()[1] for l in log if "_aos" in l]
+    # template arguments CHECK, ALIGNED of the residues, ALIGNED of the plaquettes
+    lo = "ILb0ELb%dEE" % (offset == 0), "ILb%dEE" % (offset == 0)
+    assert len(names) == 2 and all(t in n for t, n in zip(lo, names))

@@ -51,3 +51,16 @@ def test_noalloc_rejects_lattices_beyond_the_scratch(ctx):
         assert e.value.code == gfc.EINVAL
     finally:
         _hip.hipFree(p)
+
+
+def test_noalloc_at_a_doubles_address(ctx):
+    """An array that begins 8 bytes behind a multiple of 16 gives the same bits."""
+    for ns, nt in ((2, 2), (6, 4), (16, 66)):
+        geom = gfc.Geometry(ns, nt)
+        U = gfc.generate_smooth(geom, 5, 0.3)
+        d = _to_device(np.concatenate([[0.0], U.view(np.float64).ravel()]))
+        try:
+            got = gfc.config_observables_noalloc(ctx, geom, d + 8)
+        finally:
+            _hip.hipFree(C.c_void_p(d))
+        assert got == gfc.config_observables(ctx, geom, U)
