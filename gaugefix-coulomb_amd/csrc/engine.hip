@@ -1107,8 +1107,7 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
     // timeslice per group so that retired slices are left out (small lattices:
     // in whole-lattice launches over the active slices)
     const bool may_block = trace == nullptr;
-    const bool per_slice = o.slice_group > 0 || j->Vh >= kSplitMinSites ||
-                           j->geom.nt * slice_bytes(j, st.fp32) > kCacheBytes;
+    const bool per_slice = o.slice_group > 0 || j->Vh >= kSplitMinSites;
     while (res > p->tolerance) {
         int group = may_block ? group_size(j, o, st.fp32) : 0;
         if (sl.on && group > 0) group = per_slice ? 1 : 0;

@@ -1622,18 +1622,6 @@ __global__ __launch_bounds__(kBlock) void k_reduce_batch(const BatchJob *__restr
     reduce_parts(part + 3 * (int64_t)J.part_off, nb, out + 3 * blockIdx.x);
 }
 
-// item = (job index, block index within [0, 2 Vh), _, _): project G
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_reunit_batch(const BatchJob *__restrict__ jobs,
-                                                         const int4 *__restrict__ items) {
-    const int4 it = items[blockIdx.x];
-    const BatchJob J = jobs[it.x];
-    const int idx = it.y * kBlock + (int)threadIdx.x;
-    if (idx >= 2 * J.x.Vh) return;
-    const int p = idx >= J.x.Vh;
-    reunit_site<T>(static_cast<cplx<T> *>(J.g), J.x.Vh, p, idx - p * J.x.Vh);
-}
-
 // ---------------------------------------------------------------------------
 // Device-side synthetic configuration: the same construction as the host
 // generator (host_gen.c: splitmix64 draws, Box-Muller normals, Gram-Schmidt
