@@ -43,7 +43,10 @@ def _reference(U, ns, nt):
     return (e2, theta, F / (9 * V)), plaq
 
 
-@pytest.mark.parametrize("ns,nt", [(2, 2), (2, 6), (4, 2), (6, 2), (10, 4), (16, 64), (16, 66)])
+@pytest.mark.parametrize("ns,nt", [(2, 2), (2, 6), (4, 2), (6, 2), (10, 4), (16, 64), (16, 66),
+                                   # above 2^18 sites: a last group of 48 sites; two
+                                   # of the last workgroup's four groups empty
+                                   (18, 46), (26, 16)])
 def test_against_numpy(ctx, ns, nt):
     geom = gfc.Geometry(ns, nt)
     rng = np.random.default_rng(ns * 1000 + nt)

@@ -64,11 +64,11 @@ def test_blocked_stop_at_max_sweeps(ctx):
 @pytest.mark.parametrize("nt", [16, 6])
 @pytest.mark.parametrize("precision", [gfc.PREC_FP64, gfc.PREC_MIXED])
 def test_cached_and_streamed_loads_agree(ctx, precision, nt):
-    # 48^3 x nt: one timeslice holds 40.5 MiB of u0 and G in FP64 (20.25 MiB
-    # in FP32), so whole-lattice sweeps and groups of 3 timeslices on four
-    # streams use non-temporal loads, groups of 1 and the default grouping
-    # cached ones (with nt = 6 the FP64 waves end with a ragged one of 2
-    # groups, and in FP32 the whole lattice, 122 MiB, is swept from the cache)
+    # 48^3 x nt: the sweeps of a timeslice touch 27 MiB in FP64 (20.25 MiB in
+    # FP32), so whole-lattice sweeps and groups of 3 timeslices on four streams
+    # use non-temporal loads, groups of 1 and the default grouping cached ones;
+    # with nt = 6 the whole lattice (162 and 122 MiB) is swept from the cache,
+    # in three groups
     geom = gfc.Geometry(48, nt)
     p = gfc.Params(tolerance=1e-300, estimate_sweeps_to_gf_progress=100000000,
                    max_sweeps_to_fix=64, sweeps_to_reunitarization=10)
@@ -109,3 +109,31 @@ def test_blocked_tiles_shared_across_timeslices(ctx, precision, ns, nt):
             assert rep.residue_final == rep0.residue_final
             assert np.array_equal(G, G0)
             assert np.array_equal(U, U0)
+
+
+@pytest.mark.parametrize("ns,nt", [(18, 36), (24, 10)])
+@pytest.mark.parametrize("precision", [gfc.PREC_FP64, gfc.PREC_MIXED])
+def test_two_groups(ctx, precision, ns, nt):
+    """Lattices in the cache of more than 2^16 and fewer than 2^17 parity sites
+    are swept as two groups by default: the same bits as whole-lattice sweeps."""
+    geom = gfc.Geometry(ns, nt)
+    assert 1 << 16 < geom.volume // 2 < 1 << 17
+    _same_bits(ctx, geom, precision, dict(slice_group=0))
+
+
+def test_streamed_single_timeslices(ctx):
+    """FP64 timeslices whose waves leave the cache (64^3: 64 MiB, four streams),
+    as the default has it from ns = 74 on."""
+    _same_bits(ctx, gfc.Geometry(64, 6), gfc.PREC_FP64, dict(slice_group=1, slice_lanes=4))
+
+
+def _same_bits(ctx, geom, precision, options):
+    p = gfc.Params(tolerance=1e-300, estimate_sweeps_to_gf_progress=100000000,
+                   max_sweeps_to_fix=23, sweeps_to_reunitarization=10)
+    with gfc.Job(ctx, geom, precision) as job:
+        job.generate_smooth(9, 0.35)
+        job.reunitarize()
+        job.save_config()
+        G = [_run(job, p, gfc.Options(precision=precision, **o))[2]
+             for o in (dict(slice_group=-1), options)]
+        assert np.array_equal(G[0], G[1])

@@ -1,7 +1,6 @@
 """Full fixes on lattice shapes that take each branch of the default sweep
-grouping (whole lattice from the cache; cache-sized groups of several
-timeslices with cached loads; single timeslices with streaming loads), with
-spatial extents that are not multiples of 8.
+grouping (whole lattice from the cache; cache-sized groups of one or several
+timeslices with cached loads), with spatial extents that are not multiples of 8.
 
 For each shape, under the reference schedule:
 * the default grouping gives G bit for bit equal to whole-lattice sweeps
@@ -17,9 +16,10 @@ import gfc
 
 pytestmark = [pytest.mark.gpu, pytest.mark.slow]
 
-# (ns, nt): 12^3 x 24 and 20^3 x 40 fit in the cache whole; 40^3 x 80 runs
-# cached groups of 2 timeslices (23.4 MiB each in FP64); 56^3 x 112 runs single
-# timeslices (64.3 MiB in FP64, streamed; 32.2 MiB in FP32, cached)
+# (ns, nt): 12^3 x 24 (one group) and 20^3 x 40 (three) fit in the cache whole;
+# 40^3 x 80 runs cached groups of 4 timeslices on 3 streams (15.6 MiB each in
+# FP64; in FP32, 11.7 MiB, 4 on 4); 56^3 x 112 cached groups of 2 timeslices on
+# 2 streams (42.9 MiB each in FP64), in FP32 single ones (32.2 MiB) on 4
 SHAPES = [(12, 24), (20, 40), (40, 80), (56, 112)]
 
 
