@@ -759,8 +759,7 @@ int sweep_slices(gfc_job *j, int from, int to, double omega, int hits, unsigned 
 
 // Half-sweeps [from, to) (parity = sweep number & 1), timeslice group by
 // timeslice group, with the reunitarization of G after every sweep number
-// s + 1 < to that is a multiple of R folded into the two sweeps around it:
-// sweep s projects its own parity's G on output, sweep s + 1 the other
+// s + 1 < to for which it is due folded into the two sweeps around it: sweep s projects its own parity's G on output, sweep s + 1 the other
 // parity's on input.  Every site update reads only sites of its own
 // timeslice, so each group runs through the sweeps on its own and the result
 // equals that of whole-lattice sweeps bit for bit.
@@ -785,14 +784,15 @@ int sweep_blocked(gfc_job *j, const StreamSet &ss, bool fp32, int from, int to, 
     }
     // `lanes` groups at a time, one per stream, launched in step so that the
     // streams stay busy together
+    const bool frame = !fp32 && !j->own;
     auto launch_all = [&]() -> int {
         for (int w0 = 0; w0 < ng; w0 += lanes) {
             const int w1 = std::min(ng, w0 + lanes);
             for (int k = from; k < to; k++) {
                 // a reunitarization after sweep number k + 1 < to: sweep k projects
                 // its own parity on output, sweep k + 1 the other parity on input
-                const bool pout = k + 1 < to && (unsigned)(k + 1) % R == 0;
-                const bool pin = k > from && (unsigned)k % R == 0;
+                const bool pout = k + 1 < to && gfc::reunit_due((unsigned)(k + 1), R, frame);
+                const bool pin = k > from && gfc::reunit_due((unsigned)k, R, frame);
                 for (int wi = w0; wi < w1; wi++) {
                     hipStream_t s = ss.lane[wi - w0];
                     const int t0 = groups[wi] * group;
@@ -1185,7 +1185,7 @@ int run_fix(gfc_job *j, const gfc_params *p, const gfc_options *o_in, gfc_report
             done = true;
             break;
         }
-        if (!((unsigned)sweep % p->sweeps_to_reunitarization))
+        if (gfc::reunit_due((unsigned)sweep, p->sweeps_to_reunitarization, !st.fp32 && !j->own))
             RC_TRY(reunit_g(j, st.fp32, 0, 2));
     }
     // converged: the final reunitarization of G and U (src/gauge_fixing.c:822-823);

@@ -125,8 +125,8 @@ StreamSet ctx_streams(gfc_ctx *c);
 int group_size(const gfc_job *j, const gfc_options &o, bool fp32);
 int lane_count(const gfc_job *j, const gfc_options &o, bool fp32);
 // Half-sweeps [from, to) timeslice group by timeslice group on the streams of
-// ss, with the reunitarization of G after every sweep s + 1 < to that is a
-// multiple of R folded in; bit-identical to whole-lattice sweeps.
+// ss, with the reunitarization of G after every sweep s + 1 < to for which it is
+// due folded in; bit-identical to whole-lattice sweeps.
 int sweep_blocked(gfc_job *j, const StreamSet &ss, bool fp32, int from, int to, int group,
                   int max_lanes, double omega, int hits, unsigned R,
                   const std::vector<char> *active = nullptr);

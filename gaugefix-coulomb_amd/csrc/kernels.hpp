@@ -612,6 +612,22 @@ __device__ __forceinline__ unsigned xcd_order(unsigned i, unsigned n) {
     return base + x * q + (x < r ? x : r) + j / kXcd;
 }
 
+// Whether G is reunitarized after half-sweep s (1, 2, ...): every R, and in the
+// axial frame every kFrameReunit at least.  In exact arithmetic these more
+// projections do nothing; here G drifts off SU(3) by its rounding, and with it a
+// timeslice turns as a whole, a direction no gauge condition holds.  In the
+// frame that drift is another one, by parameters 0.7 to 1.5 times that in the
+// configuration's own: relative error of G against 80-bit arithmetic after 240
+// half-sweeps at 14^3 x 12 with one / two hits (omega 1.7, R = 250), own frame
+// 7.8e-15 / 7.9e-15, axial 8.6e-15 / 10.5e-15, axial with this 4.3e-15 / 2.5e-15
+// (every 25: 2.6e-15 / 2.0e-15, but served lattices, which are projected one
+// launch each, take 20% longer at 8^3 x 16).
+constexpr unsigned kFrameReunit = 50;
+
+__host__ __device__ inline bool reunit_due(unsigned s, unsigned R, bool frame) {
+    return s % R == 0 || (frame && R > kFrameReunit && s % kFrameReunit == 0);
+}
+
 // One red/black half-sweep on parity p over parity indices [h0, h0 + count), in
 // as many workgroups as count takes.  A small lattice's launch is a chain that
 // begins with its arguments, so those that every sweep needs first lie in their
@@ -633,8 +649,8 @@ __global__ __launch_bounds__(kBlock) void k_sweep(const cplx<T> *__restrict__ u0
 // timeslice and one thread per site of each parity (S = ns^3 / 2 <= N sites):
 // timeslices do not interact, so a workgroup runs through all the sweeps by
 // itself, its G in LDS, with a workgroup barrier where the other path has a
-// launch boundary.  Reunitarizations after the sweeps s + 1 < end that are
-// multiples of R, as in the timeslice-blocked sweeps; the same bits.
+// launch boundary.  Reunitarizations after the sweeps s + 1 < end for which
+// they are due, as in the timeslice-blocked sweeps; the same bits.
 //
 // Bound by one wave's chain of instructions: a half-sweep launch of 8^3 x 16
 // lasts 6.9 us from one to the next whatever its loads and code size, a
@@ -696,7 +712,7 @@ __global__ __launch_bounds__(N) void k_sweep_slices(const cplx<double> *__restri
             store_su3<false>(out, sh[p], lane);
         }
         __syncthreads();
-        if (k + 1 < end && (unsigned)(k + 1) % R == 0) {
+        if (k + 1 < end && reunit_due((unsigned)(k + 1), R, true)) {
             if (on) {
 #pragma unroll
                 for (int q = 0; q < 2; q++) {

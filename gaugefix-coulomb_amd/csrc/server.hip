@@ -22,8 +22,7 @@
 //      per lattice: stall, convergence, next check, max sweeps,
 //      reunitarization; finished lattices are materialised and retired;
 //   4. a chunk of half-sweeps: each lattice runs up to its next event (next
-//      multiple of sweeps_to_reunitarization, next check, next probe, hand-off,
-//      max), and every half-sweep step is ONE launch per precision that packs
+//      reunitarization, next check, next probe, hand-off, max), and every half-sweep step is ONE launch per precision that packs
 //      the 256-site chunks of the lane's lattices (k_sweep_batch).  The chunk's
 //      launch sequence is captured in a HIP graph and replayed while the plan
 //      repeats.  The large lane instead runs its oldest lattice up to its
@@ -418,6 +417,8 @@ int plan_and_run(gfc_server *s, Lane &L) {
         Req &r = *a;
         const int R = (int)r.p.sweeps_to_reunitarization;
         int stop = next_multiple(r.sweep, R);
+        if (!r.fp32 && R > (int)gfc::kFrameReunit)
+            stop = std::min(stop, next_multiple(r.sweep, (int)gfc::kFrameReunit));
         if (r.due > r.sweep) stop = std::min(stop, r.due);
         if ((int64_t)r.p.max_sweeps_to_fix > r.sweep)
             stop = (int)std::min<int64_t>(stop, (int64_t)r.p.max_sweeps_to_fix);
@@ -618,8 +619,8 @@ int poll_lane(gfc_server *s, int li) {
         }
         if (r.state != RUN || r.sweep == 0) continue;
         const int s_ = r.sweep;
-        const int R = (int)r.p.sweeps_to_reunitarization;
-        const bool at_stop = s_ % R == 0 || s_ == r.due ||
+        const unsigned R = r.p.sweeps_to_reunitarization;
+        const bool at_stop = gfc::reunit_due((unsigned)s_, R, !r.fp32) || s_ == r.due ||
                              (int64_t)s_ >= (int64_t)r.p.max_sweeps_to_fix ||
                              (r.fp32 && ((!r.ho.at_floor && s_ % r.o.mixed_probe_every == 0) ||
                                          s_ >= r.ho.switch_at));
@@ -648,7 +649,7 @@ int poll_lane(gfc_server *s, int li) {
             RC_TRY(finish(L, r, GFC_ENOTCONVERGED));
             continue;
         }
-        if (!((unsigned)s_ % r.p.sweeps_to_reunitarization))
+        if (gfc::reunit_due((unsigned)s_, R, !r.fp32))
             RC_TRY(gfcx::reunit_g(r.job, L.st, r.fp32, 0, 2));
     }
     // retire finished requests (their results are materialised in HBM)

@@ -241,7 +241,7 @@ int gfc_job_plaquette(gfc_job *job, double *spatial, double *temporal);
  * include/gauge_fixing.h:67-69) on the resident job: G <- 1, red/black
  * overrelaxation sweeps with the reference's check schedule, stall test,
  * max-sweeps test and reunitarization every sweeps_to_reunitarization
- * sweeps; U and G are left gauge-fixed on the device.  Returns the sweep
+ * sweeps (in FP64 every 50 at least, against the drift of rounding); U and G are left gauge-fixed on the device.  Returns the sweep
  * count, GFC_ENOTCONVERGED or GFC_EPARAMS (or a device error; G is then 1).
  * The links are meant to be SU(3): gfc_job_reunitarize first.  FP64 sweeps
  * multiply them up the Z columns and keep the nearest SU(3) matrices, also of

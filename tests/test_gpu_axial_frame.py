@@ -88,3 +88,30 @@ def test_mixed_stopped_in_fp32(ctx, ns, nt):
         assert np.abs(Ut[..., mu, :, :] - Gt @ V0[..., mu, :, :]
                       @ dag(np.roll(Gt, -1, axis=mu))).max() < 1e-13
     assert np.abs(G - out[gfc.PREC_FP64][0]).max() < 1000 * 6e-8
+
+
+@pytest.mark.parametrize("route", [dict(), dict(slice_group=-1), dict(trace_len=240)])
+@pytest.mark.parametrize("ns,nt", [(8, 6), (14, 4)])
+def test_drift_off_su3_is_bounded(ctx, ns, nt, route):
+    """With rare reunitarizations (R = 1000) the frame still projects G every 50
+    half-sweeps, in which a site is updated 25 times at most.  An update biases a
+    row's norm by a unit roundoff at most, its square by 2 * 1.1e-16: 5.5e-15 in
+    all, and row 2, the product of two, by twice that.  (Not projected, row 1 is
+    off by 9e-15 and row 2 by 14e-15 after 240, with one hit and omega 1.7.)  All
+    routes keep the same bits."""
+    geom = gfc.Geometry(ns, nt)
+    p = gfc.Params(tolerance=1e-300, estimate_sweeps_to_gf_progress=100000000,
+                   max_sweeps_to_fix=240, sweeps_to_reunitarization=1000, omega_OR=1.7, hits=1)
+    out = []
+    for r in (dict(), route):
+        trace_len = r.get("trace_len", 0)
+        o = gfc.Options(**{k: v for k, v in r.items() if k != "trace_len"})
+        with gfc.Job(ctx, geom) as job:
+            job.generate_smooth(7, 0.3)
+            job.reunitarize()
+            assert job.fix(p, o, trace_len=trace_len)[0] == gfc.ENOTCONVERGED
+            out.append(job.download_gauge())
+    assert np.array_equal(out[0], out[1])
+    norms = (np.abs(out[0].astype(np.clongdouble)) ** 2).sum(-1).mean(0) - 1
+    print(norms)
+    assert np.all(np.abs(norms) < [5.5e-15, 5.5e-15, 1.1e-14])
