@@ -32,14 +32,16 @@
 // read a Z link.  G = G' h is formed at the end of a fix (k_frame_end).  The
 // sweeps are bound by the rate of their bytes and next by instructions: 768 ->
 // 608 B and 2414 -> about 2080 VALU instructions per update took the 48^3 x 96
-// FP64 fix from 0.652 to 0.547 s, of which entering and leaving the frame are
-// 3.6 ms; 32^3 x 64 from 131 to 110 ms, 8^3 x 16 from 9.4 to 7.9 ms.  (With the
-// update as it stands, 1895 instructions and 639 B of L2 misses per update, the
-// fix takes 0.513 s.)
-// The FP32 phase of a mixed fix keeps the configuration's own frame: the
-// rounding of its sweeps is carried to the result in the directions that do
-// not change the gauge condition, up to 1e-3 on the odd timeslice, and another
-// frame would give another one.
+// FP64 fix from 0.652 to 0.547 s; 32^3 x 64 from 131 to 110 ms, 8^3 x 16 from
+// 9.4 to 7.9 ms.  (With the update as it stands, 1895 instructions and 639 B of
+// L2 misses per update, the fix takes 0.513 s, of which entering and leaving the
+// frame are 3.1 ms.)
+// Two kinds of sweeps keep the configuration's own frame.  The FP32 phase of a
+// mixed fix: the rounding of its sweeps is carried to the result in the
+// directions that do not change the gauge condition, 1e-6 to 1e-5 of G as a
+// rule but 1e-3 on the odd timeslice (1.3e-4 of G), and another frame would give
+// another one.  And links that are not near SU(3) (near_su3), which the products
+// up a column would spread.
 #pragma once
 
 #include "su3.hpp"
@@ -438,9 +440,9 @@ __device__ __forceinline__ void axial_z(mat3<double> &W, const cplx<double> *__r
 }
 
 // ---------------------------------------------------------------------------
-// The site update of parity index h = first + lane on parity p: reads the u0 links (FP64: 4
-// in the axial frame, and a Z link next to the wrap; FP32: 6), 6 neighbour G
-// and G(n); writes G(n).  Shared by the single-lattice and the
+// The site update of parity index h = first + lane on parity p: reads the u0
+// links (in the axial frame 4, and a Z link next to the wrap; else 6), 6
+// neighbour G and G(n); writes G(n).  Shared by the single-lattice and the
 // batched (serving) kernels, so a site computes the same bits in both.
 // POUT projects the new G(n) onto SU(3) (in FP64, project_g) before storing
 // it: the same bits as a reunitarization of this parity's G right after the
@@ -452,8 +454,8 @@ __device__ __forceinline__ void axial_z(mat3<double> &W, const cplx<double> *__r
 // without it they are cached, for sweeps whose data stays in the Infinity
 // Cache from one half-sweep to the next.
 //
-// FP32, in the configuration's own frame: the four matrices of a direction are
-// loaded together, one memory round trip per direction rather than the
+// In the configuration's own frame: the four matrices of a direction are loaded
+// together, one memory round trip per direction rather than the
 // compiler's two.
 template <typename T, bool POUT, bool STREAM, bool PIN>
 __device__ __forceinline__ void sweep_own(const cplx<T> *__restrict__ u0,

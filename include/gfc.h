@@ -165,7 +165,9 @@ typedef struct {
                                nt, in one launch between decisions; single
                                timeslices when a wave of them does not fit;
                                -1: whole-lattice sweeps.  With retire_slices,
-                               one timeslice per group.                       */
+                               one timeslice per group on lattices of at least
+                               2^17 parity sites or where groups are asked
+                               for, else the active timeslices together.      */
     int slice_lanes;        /* streams over which the timeslice groups run
                                concurrently: 1-4, or 0 (default): up to three
                                for a lattice that fits the cache whole, two or
