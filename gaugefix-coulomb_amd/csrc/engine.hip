@@ -950,14 +950,6 @@ struct SliceTracker {
         hipStream_t s = j->ctx->stream;
         slice_sweeps += (double)n_active / nt;
         if (n_active == 0) return GFC_OK;
-        if (j->own && !fp32) {  // not in the batched kernel
-            const gfc::Extents x = gfc::make_extents(j->geom.ns, j->Vh);
-            for (int t = 0; t < nt; t++)
-                if (active[t])
-                    RC_TRY(launch_sweep(j->u0, j->g, s, x, p, omega, hits, t * S, S, true, false,
-                                        stream_loads(j, false, 0, 1)));
-            return GFC_OK;
-        }
         if (dirty || desc_fp32 != fp32) {
             gfc::BatchJob b{};
             b.u0 = fp32 ? (const void *)j->u0f : (const void *)j->u0;
@@ -990,6 +982,12 @@ struct SliceTracker {
         else if (fp32)
             hipLaunchKernelGGL((gfc::k_sweep_batch<float, false>), dim3(n), dim3(kBlock), 0, s,
                                d_job, d_items[p], n);
+        else if (j->own && stream)
+            hipLaunchKernelGGL((gfc::k_sweep_batch<double, true, true>), dim3(n), dim3(kBlock), 0,
+                               s, d_job, d_items[p], n);
+        else if (j->own)
+            hipLaunchKernelGGL((gfc::k_sweep_batch<double, false, true>), dim3(n), dim3(kBlock), 0,
+                               s, d_job, d_items[p], n);
         else if (stream)
             hipLaunchKernelGGL((gfc::k_sweep_batch<double, true>), dim3(n), dim3(kBlock), 0, s,
                                d_job, d_items[p], n);

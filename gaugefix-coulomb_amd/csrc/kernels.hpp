@@ -1598,9 +1598,9 @@ struct BatchJob {
 };
 
 // One workgroup per item = (job index, first parity index, parity, unused).
-// (Looping a workgroup over several items measured 17% slower.)  STREAM as in
-// sweep_site.
-template <typename T, bool STREAM = true>
+// (Looping a workgroup over several items measured 17% slower.)  STREAM and OWN
+// as in sweep_site.
+template <typename T, bool STREAM = true, bool OWN = false>
 __global__ __launch_bounds__(kBlock) void k_sweep_batch(const BatchJob *__restrict__ jobs,
                                                         const int4 *__restrict__ items,
                                                         int nitems) {
@@ -1610,9 +1610,9 @@ __global__ __launch_bounds__(kBlock) void k_sweep_batch(const BatchJob *__restri
     const BatchJob J = jobs[it.x];
     const int lane = (int)threadIdx.x;
     if (it.y + lane < J.x.Vh)
-        sweep_site<T, false, STREAM>(static_cast<const cplx<T> *>(J.u0),
-                                     static_cast<cplx<T> *>(J.g), J.x, it.z, (T)J.omega, J.hits,
-                                     it.y, lane);
+        sweep_site<T, false, STREAM, false, OWN>(static_cast<const cplx<T> *>(J.u0),
+                                                 static_cast<cplx<T> *>(J.g), J.x, it.z,
+                                                 (T)J.omega, J.hits, it.y, lane);
 }
 
 // item = (job index, block index within the lattice's [0, 2 Vh) range, fp32 G?, _)
